@@ -44,9 +44,10 @@ HIP_FLAGS = [
     "-I" + CSRC_DIR,
 ]
 
-# Per-file additions. The flash kernel never produces NaN from finite inputs (masked logits are
+# Per-file additions. The flash kernels never produce NaN from finite inputs (masked logits are
 # -inf, fully masked rows are handled explicitly), so NaN-preserving max operations are not needed.
-FILE_FLAGS = {"flash_fwd.hip": ["-fno-honor-nans"]}
+FILE_FLAGS = {name: ["-fno-honor-nans"] for name in
+              ("flash_fwd.hip", "flash_reg.hip", "flash_pair.hip", "flash_wide.hip")}
 
 HOST_FLAGS = [
     "-std=c++20",

@@ -1,0 +1,432 @@
+// Shared pieces of the flash prefill kernels (flash_reg.hip, flash_pair.hip, flash_wide.hip) and of
+// their dispatch (flash_fwd.hip): MFMA wrappers, the workgroup order, the LDS-DMA pipeline's
+// helpers, the online-softmax row state, the tile geometries and the launchers' declarations.
+//
+// Formulation (every kernel): S^T = K Q^T with v_mfma_f32_32x32x16_{f16,bf16} (A = K rows from LDS,
+// B = Q^T in registers for the whole tile). In the S^T accumulator every lane holds 16 keys of ONE
+// query row, so the row max/sum need a single exchange between the two 32-lane halves and the
+// online-softmax state (m, l) is one register per lane. The P^T accumulator, converted to
+// fp16/bf16, is directly the B operand of O^T = V^T P^T (the key order inside an MFMA k-step
+// matches the accumulator layout), so P never leaves registers. The O rescale is lazy (only when
+// the running max grows by more than kRescaleSlack, decided per wave).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+#include <utility>
+
+#include "sca_device.hpp"
+
+namespace sca_hip {
+
+constexpr int kRowsPerWave = 32;
+constexpr int kRowGroups = 4;
+constexpr int kBlockM = kRowGroups * kRowsPerWave;  // 128 query rows per workgroup
+constexpr int kKPad = 8;        // K rows padded by 16 B
+constexpr int kVPad = 4;        // V^T rows padded by 8 B
+constexpr float kRescaleSlack = 8.0f;  // log2 units the running max may lag behind
+
+// Geometry per head_dim. Every wave owns 32 query rows and 32 keys of each KV tile:
+// KSPLIT waves share a row group and split the tile's keys between them (their softmax states
+// are merged once at the end), so a SIMD holds KSPLIT waves whose MFMA and VALU phases overlap.
+template <int D>
+struct FlashGeom {
+    static constexpr int KSPLIT = D <= 128 ? 2 : 1;
+    static constexpr int WAVES = kRowGroups * KSPLIT;
+    static constexpr int THREADS = WAVES * kWave;
+    static constexpr int BN = 32 * KSPLIT;               // keys per tile
+    static constexpr int STAGES = 3;                     // LDS ring depth
+    static constexpr int KS = D / 16;                    // QK k-steps
+    static constexpr int DT = D / 32;                    // 32-row tiles of O^T
+    static constexpr int KSTR = D + kKPad;               // K row stride (elements)
+    static constexpr int VSTR = BN + kVPad;              // V^T row stride (elements)
+    static constexpr int K_CHUNKS = BN * D / 8;          // 16 B chunks per K tile
+    static constexpr int K_PER_THREAD = (K_CHUNKS + THREADS - 1) / THREADS;
+    static constexpr int V_UNITS = (BN / 4) * (D / 8);   // 4 keys x 8 dims per unit
+    static constexpr int V_PER_THREAD = (V_UNITS + THREADS - 1) / THREADS;
+    static constexpr int K_STAGE = BN * KSTR;
+    static constexpr int V_STAGE = D * VSTR;
+    static constexpr int STAGE_BYTES = STAGES * (K_STAGE + V_STAGE) * 2;
+    static constexpr int MERGE_FLOATS = DT * 16 + 2;     // per lane: O^T + m + l
+    static constexpr int MERGE_BYTES = KSPLIT > 1 ? kRowGroups * kWave * MERGE_FLOATS * 4 : 0;
+    static constexpr int LDS_BYTES = STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES;
+};
+
+// ---- Two-group causal pair kernel ---------------------------------------------------------------
+// Small causal grids: each workgroup owns the complementary 64-row tiles A = T-1-t (long) and
+// B = t (short) and runs them concurrently in two groups of four waves (one wave of each group
+// per SIMD), each group with its own K/V ring. Group 0 takes A's key tiles [0, x); group 1
+// takes all of B, finishes B (a two-way merge and the stores), then takes A's key tiles
+// [x, n_A). The two groups' A states are merged once at the end, so the short tile's setup,
+// merge and stores run beside the long tile's key loop instead of after it. x balances the
+// two groups' barrier intervals.
+// Within a group: 2 row groups of 32 rows x 2 waves of 32 keys per 64-key tile; the pipeline
+// step j computes QK of tile j+1 under the softmax of tile j, then PV of tile j.
+template <int D>
+struct PairGeom {
+    static constexpr int GW = 4;                      // waves per group
+    static constexpr int THREADS = 2 * GW * kWave;
+    static constexpr int BM = 64;                     // rows per row tile
+    static constexpr int BN = 64;                     // keys per key tile
+    static constexpr int KS = D / 16;
+    static constexpr int DT = D / 32;
+    static constexpr int CPR = D / 8;
+    static constexpr int ROW_BYTES = D * 2;
+    static constexpr int TILE_BYTES = BN * D * 2;
+    static constexpr int IPW = BN * CPR / (kWave * GW);  // DMA instructions per wave per tile
+    static constexpr int RING_BYTES = 4 * TILE_BYTES;    // K slots 0, 1, then V slots 0, 1
+    // Final merge: per row group, three partial states (16-byte quads) and their (m, l).
+    static constexpr int MERGE_QUADS = 2 * 3 * 4 * DT * kWave;
+    static constexpr int MERGE_BYTES = MERGE_QUADS * 16 + 2 * 3 * kWave * 8;
+    static constexpr int LDS_BYTES = 2 * RING_BYTES > MERGE_BYTES ? 2 * RING_BYTES : MERGE_BYTES;
+    static_assert(IPW >= 1 && BN * CPR == IPW * kWave * GW, "tile must split evenly into DMAs");
+    static_assert(2 * 4 * DT * kWave * 16 + 2 * kWave * 8 <= RING_BYTES,
+                  "the B merge fits group 1's ring");
+    static_assert(TILE_BYTES < 65536, "slot offsets are DS immediates");
+};
+
+template <int D>
+struct WideGeom {
+    static constexpr int WAVES = 4;
+    static constexpr int THREADS = WAVES * kWave;
+    static constexpr int RT = 2;                      // 32-row subtiles per wave
+    static constexpr int BM = 128;                    // rows per workgroup
+    static constexpr int BN = 64;                     // keys per tile
+    static constexpr int KS = D / 16;                 // QK k-steps
+    static constexpr int DT = D / 32;                 // O^T tiles of 32 dims
+    static constexpr int CPR = D / 8;                 // 16-byte chunks per row
+    static constexpr int ROW_BYTES = 2 * D;
+    static constexpr int TILE_BYTES = BN * ROW_BYTES;
+    static constexpr int IPW = BN * CPR / (kWave * WAVES);  // DMA instructions per wave per tile
+    static constexpr int SLOTS = 4;
+    static constexpr int V_BASE = SLOTS * TILE_BYTES;
+    static constexpr int RING_BYTES = 2 * SLOTS * TILE_BYTES;
+    // Merge: the two kq = 1 waves' O (RT*DT*16 floats per lane) and (m, l) per subtile.
+    static constexpr int MERGE_FLOATS = RT * DT * 16 + 2 * RT;
+    static constexpr int MERGE_BYTES = 2 * kWave * MERGE_FLOATS * 4;
+    static constexpr int LDS_BYTES = RING_BYTES > MERGE_BYTES ? RING_BYTES : MERGE_BYTES;
+    static_assert(IPW >= 1 && BN * CPR == IPW * kWave * WAVES, "tile must split evenly");
+    // V reads of the two upper slots go through a second address (slot offsets are DS immediates
+    // below 64 KB).
+    static constexpr bool V_SPLIT = (SLOTS - 1) * TILE_BYTES + 25 * ROW_BYTES > 65536;
+    static_assert((SLOTS - 1) * TILE_BYTES + ROW_BYTES <= 65536 && TILE_BYTES + 25 * ROW_BYTES <= 65536,
+                  "slot offsets are DS immediates");
+};
+
+// Packed variable-length launch: cumulative token offsets and the work list (2 int32 per row
+// tile: sequence, tile), device-resident.
+struct VarlenArgs {
+    const int32_t* cu_q;
+    const int32_t* cu_kv;
+    const int32_t* tiles;
+};
+
+// Launchers, instantiated in the file of their kernel. Every one validates its grid and returns 0
+// or a status.
+template <typename E, int D, bool kCausal>
+int LaunchFlashReg(const sca_flash_params& p, hipStream_t s);   // flash_reg.hip
+template <typename E, int D>
+int LaunchFlashPair(const sca_flash_params& p, hipStream_t s);  // flash_pair.hip (causal)
+template <typename E, int D, bool kCausal>
+int LaunchFlashWide(const sca_flash_params& p, hipStream_t s);  // flash_wide.hip
+template <typename E, int D, bool kCausal>
+int LaunchFlashVarlen(const sca_flash_varlen_params& v, hipStream_t s);  // flash_wide.hip
+
+namespace {
+
+template <typename E>
+struct Mfma;
+
+template <>
+struct Mfma<F16> {
+    typedef _Float16 pair_t __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ floatx16 mma(const half8& a, const half8& b, floatx16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+    }
+    // Two floats -> packed pair (round to nearest even), as the raw 32-bit word.
+    static __device__ __forceinline__ uint32_t pack(float a, float b) {
+        typedef float f2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){a, b}, pair_t));
+    }
+    // acc + a.x + a.y in fp32 (v_dot2 with (1, 1)).
+    static __device__ __forceinline__ float sum2(uint32_t w, float acc) {
+        const pair_t ones = {static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)};
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(pair_t, w), ones, acc, false);
+    }
+};
+
+template <>
+struct Mfma<BF16> {
+    typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ floatx16 mma(const bf16x8& a, const bf16x8& b, floatx16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ uint32_t pack(float a, float b) {
+        typedef float f2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){a, b}, pair_t));
+    }
+    static __device__ __forceinline__ float sum2(uint32_t w, float acc) {
+        const pair_t ones = {static_cast<__bf16>(1.0f), static_cast<__bf16>(1.0f)};
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pair_t, w), ones, acc, false);
+    }
+};
+
+// Workgroup -> (row tile index, batch*head). The dispatcher deals workgroups to the eight XCDs
+// round robin (workgroup w on XCD w % 8), and each XCD has its own L2. When the (batch, KV head)
+// groups divide by eight, XCD x takes groups x, x + 8, ...: the query heads that read one KV head
+// run on one XCD and share its L2 (C3, 4 x 8 groups of 4 heads: +5%). Otherwise w runs row tile
+// w / bh_count of head w % bh_count. Either way row tile t starts before t + 1 (so longest-first
+// orders survive), and the mapping is a bijection on [0, tiles * bh_count).
+__device__ __forceinline__ void XcdOrder(const sca_flash_params& p, int64_t bh_count,
+                                         int64_t* tile_linear, int64_t* bh) {
+    const int64_t w = blockIdx.x;
+    const int64_t groups = p.batch * p.num_kv_heads;
+    if (groups % 8 != 0) {
+        *tile_linear = w / bh_count;
+        *bh = w % bh_count;
+        return;
+    }
+    const int64_t gsz = p.num_heads / p.num_kv_heads;
+    const int64_t per_tile = bh_count / 8;  // workgroups of one row tile on one XCD
+    const int64_t pos = w / 8;
+    const int64_t rem = pos % per_tile;
+    *tile_linear = pos / per_tile;
+    *bh = ((rem / gsz) * 8 + w % 8) * gsz + rem % gsz;
+}
+
+// Scheduling-group masks of __builtin_amdgcn_sched_group_barrier.
+constexpr int kSchedValu = 0x002;
+constexpr int kSchedMfma = 0x008;
+constexpr int kSchedDsRead = 0x100;
+
+
+// ============================================================================================
+// The DMA pipeline of the head_dim 64 / 128 kernels (pair and wide).
+//
+// K and V tiles go straight from global memory to LDS with buffer loads to LDS (16 bytes per
+// lane, no VGPR staging, no transposition) through a buffer resource bounded at the sequence's
+// last row, so rows past seq_kv read as zero. Loads are issued ahead of their use and retired
+// with explicit vmcnt waits plus one barrier per tile. LDS rows are unpadded; 16-byte chunks are
+// XOR-swizzled per row (SwzK / SwzV) so that both the K reads and the V transpose reads are
+// bank-conflict free. The PV A operand (V^T fragments) comes from ds_read_b64_tr_b16: within each
+// 16-lane group, lane j receives element j % 4 of the 8 bytes read by lane 4*i + j/4 (i = 0..3),
+// i.e. one head-dim column over 4 consecutive keys.
+// ============================================================================================
+
+// 16-byte-chunk swizzles for 64 LDS banks (a 256-byte bank window of 16 chunks). A row of D
+// elements is D/8 chunks, so row r starts at chunk (D/8 * r) mod 16 of the window, and XOR with a
+// value below the power of two that divides D/8 stays inside the row:
+//   K: the 32 rows a wave reads in one ds_read_b128 land on 16 distinct 4-bank groups;
+//   V: the 8 keys x 4 chunks of one transpose read land on 16 distinct groups.
+// D/8 = 0 mod 16 (128, 256): every row starts at the same chunk, the swizzle does all the work;
+// 8 mod 16 (64, 192): odd rows start half a window on; 4 or 12 mod 16 (32, 96, 160): four rows
+// already cover the window, so V needs none.
+template <int D>
+__device__ __forceinline__ int SwzK(int row) {
+    constexpr int kStart = (D / 8) % 16;
+    static_assert(kStart % 4 == 0, "head_dim is a multiple of 32");
+    return kStart == 0 ? (row & 15) : kStart == 8 ? ((row >> 1) & 7) : ((row >> 2) & 3);
+}
+template <int D>
+__device__ __forceinline__ int SwzV(int row) {
+    constexpr int kStart = (D / 8) % 16;
+    return kStart == 0 ? ((row & 3) << 2) : kStart == 8 ? (((row >> 1) & 1) << 2) : 0;
+}
+
+// Fragment addresses: the swizzle permutes chunks only inside aligned groups, so the addresses of
+// k-step ks and ks + KPeriod (and of O tile dt and dt + VPeriod) differ by a constant, which goes
+// into the read's immediate offset.
+template <int D>
+constexpr int KPeriod() {
+    constexpr int kStart = (D / 8) % 16;
+    return kStart == 0 ? (D / 16 < 8 ? D / 16 : 8) : kStart == 8 ? 4 : 2;
+}
+template <int D>
+constexpr int VPeriod() {
+    constexpr int kStart = (D / 8) % 16;
+    return kStart == 0 ? (D / 32 < 4 ? D / 32 : 4) : kStart == 8 ? 2 : 1;
+}
+
+// (lower-half value, upper-half value) of v for lanes l and l ^ 32, on every lane, from one
+// v_permlane32_swap: it exchanges the upper 32 lanes of its first operand with the lower 32 lanes
+// of its second, so with both operands holding v the first ends as (v_lo, v_lo) and the second as
+// (v_hi, v_hi). Issued from inline asm with both registers as in/out operands (the builtin's
+// second result is not reliably kept apart from the first), after the two wait states a VALU
+// write needs before the permlane reads it.
+__device__ __forceinline__ void HalfPair(float v, float* lo, float* hi) {
+    uint32_t a = __builtin_bit_cast(uint32_t, v);
+    uint32_t b = a;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    *lo = __builtin_bit_cast(float, a);
+    *hi = __builtin_bit_cast(float, b);
+}
+__device__ __forceinline__ float HalfMax(float v) {
+    float lo, hi;
+    HalfPair(v, &lo, &hi);
+    return fmaxf(lo, hi);
+}
+__device__ __forceinline__ float HalfSum(float v) {
+    float lo, hi;
+    HalfPair(v, &lo, &hi);
+    return lo + hi;
+}
+
+// ---- Online softmax of one 32-key x 32-row S^T tile (lane: 16 keys of one row; lanes l and
+// l ^ 32 hold the other 16 keys of the same row) -----------------------------------------------
+// Per-lane row state: the running max used for the exponentials (m, log2 units), the raw-score
+// threshold above which it must move (thr = (m + kRescaleSlack) / scale2), the exponent bias
+// (-m, or 0 while no key of the row was visible) and this lane's share of the denominator.
+struct RowState {
+    float m;
+    float thr;
+    float neg_mu;
+    float l;
+};
+
+__device__ __forceinline__ void ResetRow(RowState& r) {
+    r.m = neg_inf();
+    r.thr = neg_inf();
+    r.neg_mu = 0.0f;
+    r.l = 0.0f;
+}
+
+__device__ __forceinline__ float Max16(const floatx16& s) {
+    const float a = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+    const float b = fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7]));
+    const float c = fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11]));
+    const float d = fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]));
+    return fmaxf(fmaxf(a, b), fmaxf(c, d));
+}
+
+// Transposed 8-byte LDS read at byte address addr + OFF. Issued from inline asm so that the
+// compiler's conservative LDS-DMA tracking adds no wait for DMAs still in flight; the caller
+// retires the reads with WaitLdsTied before the registers are used.
+template <int OFF>
+__device__ __forceinline__ uint2 TrReadAsm(uint32_t addr) {
+    uint2 r;
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF));
+    return r;
+}
+
+// lgkmcnt(0), tied to the registers it guards so that no use of them is scheduled above it,
+// and to the P operands (a, b) so that it is not hoisted above the exponentials either.
+template <typename V, int N>
+__device__ __forceinline__ void WaitLdsTied(V (&regs)[N], V& a, V& b) {
+    if constexpr (N == 8) {
+        asm volatile("s_waitcnt lgkmcnt(0)"
+                     : "+v"(regs[0]), "+v"(regs[1]), "+v"(regs[2]), "+v"(regs[3]), "+v"(regs[4]),
+                       "+v"(regs[5]), "+v"(regs[6]), "+v"(regs[7]), "+v"(a), "+v"(b));
+    } else if constexpr (N == 4) {
+        asm volatile("s_waitcnt lgkmcnt(0)"
+                     : "+v"(regs[0]), "+v"(regs[1]), "+v"(regs[2]), "+v"(regs[3]), "+v"(a),
+                       "+v"(b));
+    } else {
+        static_assert(N == 8 || N == 4, "tied wait covers 4 or 8 registers");
+    }
+}
+
+__device__ __forceinline__ uint32_t LdsAddr(const void* p) {
+    return static_cast<uint32_t>(
+        reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) uint8_t*)(p)));
+}
+
+// V^T fragments of one key tile for the PV MFMAs: for O tile dt, k-step ps, the transposed
+// reads at rows 16*ps and 16*ps + 8 of the lane's V position (v_addr[dt], LDS byte address of
+// the slot-0 copy); SLOT_OFF selects the slot.
+template <int SLOT_OFF, int ROW_BYTES, int DT, typename vec8>
+__device__ __forceinline__ void ReadVFrags(const uint32_t (&v_addr)[DT], vec8 (&va)[2 * DT]) {
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        const uint2 l0 = TrReadAsm<SLOT_OFF>(v_addr[dt]);
+        const uint2 h0 = TrReadAsm<SLOT_OFF + 8 * ROW_BYTES>(v_addr[dt]);
+        const uint2 l1 = TrReadAsm<SLOT_OFF + 16 * ROW_BYTES>(v_addr[dt]);
+        const uint2 h1 = TrReadAsm<SLOT_OFF + 24 * ROW_BYTES>(v_addr[dt]);
+        va[2 * dt] = __builtin_bit_cast(vec8, make_uint4(l0.x, l0.y, h0.x, h0.y));
+        va[2 * dt + 1] = __builtin_bit_cast(vec8, make_uint4(l1.x, l1.y, h1.x, h1.y));
+    }
+}
+
+constexpr int kSchedValuTrans = 0x402;  // VALU and transcendental
+
+// 16-byte DMA of lane data from a raw buffer (base, num_records) at voffset + soffset into LDS
+// at lds + 16 * lane. Bytes at or beyond num_records read as zero. (The buffer resource is
+// built here rather than in the kernel body: a buffer-resource local in a kernel body makes the
+// host pass drop the kernel's launch stub.)
+__device__ __forceinline__ void DmaToLds(const uint8_t* base, int num_records, uint8_t* lds,
+                                         uint32_t voffset, uint32_t soffset) {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(base), 0, num_records, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(lds), 16,
+                                             voffset, soffset, 0, 0);
+}
+
+// MFMAs issued from inline asm: S^T accumulators in VGPRs, O^T accumulators in AGPRs.
+template <typename E>
+struct MfmaAsm;
+
+template <>
+struct MfmaAsm<F16> {
+    // S^T: A (K fragment) in VGPRs, B (Q fragment) in AGPRs, accumulator in VGPRs.
+    template <typename V>
+    static __device__ __forceinline__ void first_v(floatx16& c, const V& a, const V& b) {
+        asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "a"(b));
+    }
+    template <typename V>
+    static __device__ __forceinline__ void acc_v(floatx16& c, const V& a, const V& b) {
+        asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(b));
+    }
+    template <typename V>
+    static __device__ __forceinline__ void acc_a(floatx16& c, const V& a, const V& b) {
+        asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    }
+};
+
+template <>
+struct MfmaAsm<BF16> {
+    // S^T: A (K fragment) in VGPRs, B (Q fragment) in AGPRs, accumulator in VGPRs.
+    template <typename V>
+    static __device__ __forceinline__ void first_v(floatx16& c, const V& a, const V& b) {
+        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "a"(b));
+    }
+    template <typename V>
+    static __device__ __forceinline__ void acc_v(floatx16& c, const V& a, const V& b) {
+        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(b));
+    }
+    template <typename V>
+    static __device__ __forceinline__ void acc_a(floatx16& c, const V& a, const V& b) {
+        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    }
+};
+
+template <int OFF, typename V>
+__device__ __forceinline__ void ReadB128Asm(V& dst, uint32_t addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "i"(OFF));
+}
+
+// lgkmcnt(N) tied to the register it guards (the asm uses below it cannot move above it).
+template <int N, typename V>
+__device__ __forceinline__ void WaitLgkmTied(V& reg) {
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(reg) : "i"(N));
+}
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): for asm immediates.
+template <int N, typename F>
+__device__ __forceinline__ void StaticFor(F&& f) {
+    [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+        (f(std::integral_constant<int, I>{}), ...);
+    }(std::make_integer_sequence<int, N>{});
+}
+
+__device__ __forceinline__ void Fence() { __builtin_amdgcn_sched_barrier(0); }
+
+// Gives a value the AGPR register class (an empty asm with an AGPR in/out operand), so that the
+// loop-carried accumulators and Q fragments stay in AGPRs instead of being copied in and out.
+template <typename V>
+__device__ __forceinline__ void PinAgpr(V& x) {
+    asm volatile("" : "+a"(x));
+}
+
+
+}  // namespace
+}  // namespace sca_hip

@@ -312,3 +312,14 @@ def test_xcd_group_order(hip, B, Hq, Hkv, S, D, dtype):
     eight; every (row tile, head) must still be computed exactly once."""
     for j, causal in enumerate([False, True]):
         _case(dtype, causal, B, Hq, Hkv, S, S, D, 88000 + 97 * Hq + S + j)
+
+
+@pytest.mark.parametrize("D", [32, 96, 160])
+@pytest.mark.parametrize("causal", [False, True])
+def test_wide_kernel_other_head_dims(hip, D, causal):
+    """Row tiles of 128 and key tiles of 64 at their edges, every slot of the four-deep ring as the
+    last one, the steady four-step loop (from 8 key tiles), a moved diagonal, GQA and LSE."""
+    for sq, skv in [(1, 1), (63, 64), (128, 65), (129, 192), (64, 255), (200, 320), (65, 449),
+                    (100, 577), (300, 640), (33, 1000)]:
+        _case("bf16", causal, 1, 4, 2, sq, skv, D, 91000 + sq + skv + D, want_lse=True)
+    _case("f16", causal, 2, 8, 4, 260, 900, D, 92000 + D, want_lse=True)
