@@ -114,6 +114,28 @@ struct WideGeom {
                   "slot offsets are DS immediates");
 };
 
+template <int D>
+struct DsplitGeom {
+    static constexpr int WAVES = 4;
+    static constexpr int THREADS = WAVES * kWave;
+    static constexpr int BM = 128;                    // rows per workgroup
+    static constexpr int BN = 32;                     // keys per tile
+    static constexpr int KS = D / 16;                 // QK k-steps
+    static constexpr int DT = D / 64;                 // O^T tiles of 32 dims per wave (half of D)
+    static constexpr int CPR = D / 8;                 // 16-byte chunks per row
+    static constexpr int ROW_BYTES = 2 * D;
+    static constexpr int TILE_BYTES = BN * ROW_BYTES;
+    static constexpr int IPW = BN * CPR / (kWave * WAVES);  // DMA instructions per wave per tile
+    static constexpr int SLOTS = 4;
+    static constexpr int V_BASE = SLOTS * TILE_BYTES;
+    static constexpr int P_BASE = 2 * V_BASE;            // 2 parities x 4 waves x 2 KB
+    static constexpr int ALPHA_BASE = P_BASE + 16384;    // 2 parities x 4 waves x 32 floats
+    static constexpr int FLAG_BASE = ALPHA_BASE + 1024;  // 2 parities x 4 ints
+    static constexpr int LDS_BYTES = FLAG_BASE + 32;
+    static_assert(D % 64 == 0 && BN * CPR == IPW * kWave * WAVES, "tile must split evenly");
+    static_assert((SLOTS - 1) * TILE_BYTES + 25 * ROW_BYTES <= 65536, "slot offsets are DS immediates");
+};
+
 // Packed variable-length launch: cumulative token offsets and the work list (2 int32 per row
 // tile: sequence, tile), device-resident.
 struct VarlenArgs {
@@ -130,6 +152,8 @@ template <typename E, int D>
 int LaunchFlashPair(const sca_flash_params& p, hipStream_t s);  // flash_pair.hip (causal)
 template <typename E, int D, bool kCausal>
 int LaunchFlashWide(const sca_flash_params& p, hipStream_t s);  // flash_wide.hip
+template <typename E, int D, bool kCausal>
+int LaunchFlashDsplit(const sca_flash_params& p, hipStream_t s);  // flash_dsplit.hip
 template <typename E, int D, bool kCausal>
 int LaunchFlashVarlen(const sca_flash_varlen_params& v, hipStream_t s);  // flash_wide.hip
 
@@ -404,6 +428,16 @@ __device__ __forceinline__ void ReadB128Asm(V& dst, uint32_t addr) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "i"(OFF));
 }
 
+template <int OFF>
+__device__ __forceinline__ void ReadB64Asm(uint2& dst, uint32_t addr) {
+    asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "i"(OFF));
+}
+
+template <int OFF, typename V>
+__device__ __forceinline__ void WriteB128Asm(uint32_t addr, const V& src) {
+    asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(addr), "v"(src), "i"(OFF) : "memory");
+}
+
 // lgkmcnt(N) tied to the register it guards (the asm uses below it cannot move above it).
 template <int N, typename V>
 __device__ __forceinline__ void WaitLgkmTied(V& reg) {
@@ -427,6 +461,17 @@ __device__ __forceinline__ void PinAgpr(V& x) {
     asm volatile("" : "+a"(x));
 }
 
+// 32 wait states ahead of VALU access to the O accumulators (AGPRs), tied to them: the compiler
+// does not track the inline-asm MFMAs that last wrote O.
+template <int DT>
+__device__ __forceinline__ void SettleO(floatx16 (&o)[2][DT]) {
+    asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) PinAgpr(o[r][dt]);
+    }
+}
 
 }  // namespace
 }  // namespace sca_hip

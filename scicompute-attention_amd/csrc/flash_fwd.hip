@@ -12,7 +12,9 @@
 //     128, packed variable-length batches in one launch): 4 waves of 64 query rows, K/V tiles
 //     DMA'd into LDS;
 //   * flash_pair.hip (head_dim 64 and 128, causal grids too small to balance 128-row tiles);
-//   * flash_reg.hip (head_dim 192 and 256): K/V staged through registers.
+//   * flash_dsplit.hip (head_dim 192 and 256): the same with the dims of O split over two waves;
+//   * flash_reg.hip (any head_dim whose K/V extent passes the 32-bit buffer offsets of the DMA
+//     kernels, or with negative K/V row strides): K/V staged through registers.
 
 #include <hip/hip_runtime.h>
 
@@ -56,8 +58,8 @@ int LaunchForDim(const sca_flash_params& p, hipStream_t s) {
             if (kCausal && UsePairs(p)) return LaunchFlashPair<E, 128>(p, s);
             return LaunchFlashWide<E, 128, kCausal>(p, s);
         case 160: return LaunchFlashWide<E, 160, kCausal>(p, s);
-        case 192: return LaunchFlashReg<E, 192, kCausal>(p, s);
-        case 256: return LaunchFlashReg<E, 256, kCausal>(p, s);
+        case 192: return LaunchFlashDsplit<E, 192, kCausal>(p, s);
+        case 256: return LaunchFlashDsplit<E, 256, kCausal>(p, s);
         default: break;
     }
     return SetError(SCA_E_UNSUPPORTED_HEAD_DIM,
@@ -84,8 +86,8 @@ int LdsBytesFor(int64_t head_dim) {
         case 96: return WideGeom<96>::LDS_BYTES;
         case 128: return std::max(WideGeom<128>::LDS_BYTES, PairGeom<128>::LDS_BYTES);
         case 160: return WideGeom<160>::LDS_BYTES;
-        case 192: return FlashGeom<192>::LDS_BYTES;
-        case 256: return FlashGeom<256>::LDS_BYTES;
+        case 192: return DsplitGeom<192>::LDS_BYTES;
+        case 256: return DsplitGeom<256>::LDS_BYTES;
         default: return -1;
     }
 }
@@ -109,12 +111,12 @@ int sca_hip_flash_tile(int32_t head_dim, int32_t* block_m, int32_t* block_n, int
                         "flash: no tile for head_dim=" + std::to_string(head_dim));
     }
     // The wide kernel's tile (at head_dim 64 and 128: every non-causal and every large causal
-    // grid); head_dim 192 and 256 the register-staged one's.
+    // grid); head_dim 192 and 256 the split-dims kernel's.
     int32_t bn = sca_hip::WideGeom<128>::BN, nw = sca_hip::WideGeom<128>::WAVES,
             ns = sca_hip::WideGeom<128>::SLOTS;
     if (head_dim > 160) {
-        using G = sca_hip::FlashGeom<256>;
-        bn = G::BN, nw = G::WAVES, ns = G::STAGES;
+        using G = sca_hip::DsplitGeom<256>;
+        bn = G::BN, nw = G::WAVES, ns = G::SLOTS;
     }
     if (block_m != nullptr) *block_m = sca_hip::kBlockM;
     if (block_n != nullptr) *block_n = bn;

@@ -32,18 +32,6 @@
 namespace sca_hip {
 namespace {
 
-// 32 wait states ahead of VALU access to the O accumulators (AGPRs), tied to them: the compiler
-// does not track the inline-asm MFMAs that last wrote O.
-template <int DT>
-__device__ __forceinline__ void SettleO(floatx16 (&o)[2][DT]) {
-    asm volatile("s_nop 15\n\ts_nop 15");
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) PinAgpr(o[r][dt]);
-    }
-}
-
 template <typename E, int D, bool kCausal, bool kVarlen>
 __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel(
     const sca_flash_params p, int num_q_tiles, const VarlenArgs vl) {

@@ -325,3 +325,25 @@ def test_wide_kernel_other_head_dims(hip, D, causal):
             skv = max(sq, skv)
         _case("bf16", causal, 1, 4, 2, sq, skv, D, 91000 + sq + skv + D, want_lse=True)
     _case("f16", causal, 2, 8, 4, 260, 900, D, 92000 + D, want_lse=True)
+
+
+@pytest.mark.parametrize("D", [192, 256])
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_dims_kernel(hip, D, causal):
+    """Key tiles of 32 at their edges and every slot of the four-deep rings as the last one, the
+    steady four-step loop (from 6 plain tiles), a moved diagonal, GQA, LSE, and row maxima that keep
+    growing along the keys (the rescale that one wave decides and both apply)."""
+    for sq, skv in [(1, 1), (32, 33), (65, 64), (128, 95), (100, 129), (129, 160), (64, 193),
+                    (200, 255), (33, 320), (300, 353), (40, 1000)]:
+        if causal:
+            skv = max(sq, skv)
+        _case("bf16", causal, 1, 4, 2, sq, skv, D, 93000 + sq + skv + D, want_lse=True)
+    _case("f16", causal, 2, 8, 4, 260, 900, D, 94000 + D, want_lse=True)
+    sq, skv = 130, 500
+    q = np.abs(uniform((1, 2, sq, D), 95000 + D)) + 0.1
+    k = uniform((1, 2, skv, D), 95001 + D) * 0.1 + np.linspace(0.0, 12.0, skv)[None, None, :, None]
+    v = uniform((1, 2, skv, D), 95002 + D)
+    (qb, qd), (kb, kd), (vb, vd) = (quantize(x.astype(np.float32), "bf16") for x in (q, k, v))
+    out, _ = run_flash(qb, kb, vb, "bf16", causal, B=1, Hq=2, Hkv=2, Sq=sq, Skv=skv, D=D)
+    ref, _ = orc.reference_attention(qd, kd, vd, causal)
+    check_attention(out.reshape(-1, D), ref, "bf16", f"growing maxima D={D}")
