@@ -102,9 +102,9 @@ struct WideGeom {
     static constexpr int SLOTS = 4;
     static constexpr int V_BASE = SLOTS * TILE_BYTES;
     static constexpr int RING_BYTES = 2 * SLOTS * TILE_BYTES;
-    // Merge: the two kq = 1 waves' O (RT*DT*16 floats per lane) and (m, l) per subtile.
-    static constexpr int MERGE_FLOATS = RT * DT * 16 + 2 * RT;
-    static constexpr int MERGE_BYTES = 2 * kWave * MERGE_FLOATS * 4;
+    // Merge: every wave hands one subtile's O (DT*16 floats per lane) and (m, l) to its partner.
+    static constexpr int MERGE_FLOATS = DT * 16 + 2;
+    static constexpr int MERGE_BYTES = WAVES * kWave * MERGE_FLOATS * 4;
     static constexpr int LDS_BYTES = RING_BYTES > MERGE_BYTES ? RING_BYTES : MERGE_BYTES;
     static_assert(IPW >= 1 && BN * CPR == IPW * kWave * WAVES, "tile must split evenly");
     // V reads of the two upper slots go through a second address (slot offsets are DS immediates
@@ -202,21 +202,30 @@ struct Mfma<BF16> {
 // run on one XCD and share its L2 (C3, 4 x 8 groups of 4 heads: +5%). Otherwise w runs row tile
 // w / bh_count of head w % bh_count. Either way row tile t starts before t + 1 (so longest-first
 // orders survive), and the mapping is a bijection on [0, tiles * bh_count).
-__device__ __forceinline__ void XcdOrder(const sca_flash_params& p, int64_t bh_count,
-                                         int64_t* tile_linear, int64_t* bh) {
-    const int64_t w = blockIdx.x;
-    const int64_t groups = p.batch * p.num_kv_heads;
+// In 32 bits (the launchers bound the grid, and with it every factor, below 2^31): a 64-bit division
+// takes about 130 instructions on this chip, and eight of them cost each workgroup 0.4 us.
+__device__ __forceinline__ void XcdOrder(const sca_flash_params& p, int* tile_linear, int* b, int* h,
+                                         int* h_kv) {
+    const uint32_t w = blockIdx.x;
+    const uint32_t heads = static_cast<uint32_t>(p.num_heads);
+    const uint32_t kv_heads = static_cast<uint32_t>(p.num_kv_heads);
+    const uint32_t groups = static_cast<uint32_t>(p.batch) * kv_heads;
+    const uint32_t gsz = heads / kv_heads;
+    const uint32_t bh_count = groups * gsz;
+    uint32_t bh;
     if (groups % 8 != 0) {
-        *tile_linear = w / bh_count;
-        *bh = w % bh_count;
-        return;
+        *tile_linear = static_cast<int>(w / bh_count);
+        bh = w % bh_count;
+    } else {
+        const uint32_t per_tile = bh_count / 8;  // workgroups of one row tile on one XCD
+        const uint32_t pos = w / 8;
+        const uint32_t rem = pos % per_tile;
+        *tile_linear = static_cast<int>(pos / per_tile);
+        bh = ((rem / gsz) * 8 + w % 8) * gsz + rem % gsz;
     }
-    const int64_t gsz = p.num_heads / p.num_kv_heads;
-    const int64_t per_tile = bh_count / 8;  // workgroups of one row tile on one XCD
-    const int64_t pos = w / 8;
-    const int64_t rem = pos % per_tile;
-    *tile_linear = pos / per_tile;
-    *bh = ((rem / gsz) * 8 + w % 8) * gsz + rem % gsz;
+    *b = static_cast<int>(bh / heads);
+    *h = static_cast<int>(bh % heads);
+    *h_kv = *h / static_cast<int>(gsz);
 }
 
 // Scheduling-group masks of __builtin_amdgcn_sched_group_barrier.
@@ -294,6 +303,24 @@ __device__ __forceinline__ float HalfSum(float v) {
     float lo, hi;
     HalfPair(v, &lo, &hi);
     return lo + hi;
+}
+
+// Stores one 32-dim O^T tile of a row (16 values per lane, two lanes per row: lane half hh holds dims
+// 8g + 4hh + 0..3 of each group g) scaled by inv, as 16-byte chunks: the two halves of a row swap
+// words so that hh = 0 holds all of groups 0 and 2 and hh = 1 all of 1 and 3. `dst` is the row's first
+// dim of the tile (8-byte aligned); every lane of the wave takes part in the swap.
+template <typename M>
+__device__ __forceinline__ void StoreTile(uint16_t* dst, int hh, bool row_ok, const float (&v)[16]) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(8)));
+#pragma unroll
+    for (int g = 0; g < 4; g += 2) {
+        uint32_t a0 = M::pack(v[4 * g], v[4 * g + 1]), a1 = M::pack(v[4 * g + 2], v[4 * g + 3]);
+        uint32_t b0 = M::pack(v[4 * g + 4], v[4 * g + 5]), b1 = M::pack(v[4 * g + 6], v[4 * g + 7]);
+        // (a, b) -> lower half: a of both halves; upper half: b of both (see HalfPair for the waits).
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1"
+                     : "+v"(a0), "+v"(a1), "+v"(b0), "+v"(b1));
+        if (row_ok) *reinterpret_cast<u32x4*>(dst + 8 * (g + hh)) = u32x4{a0, a1, b0, b1};
+    }
 }
 
 // ---- Online softmax of one 32-key x 32-row S^T tile (lane: 16 keys of one row; lanes l and

@@ -54,13 +54,10 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
     const int rg = wave & 1;   // rows 64*rg .. +64 of the row tile
     const int dh = wave >> 1;  // QK: rows 32*dh of those; PV: dims D/2*dh .. +D/2
 
-    const int64_t bh_count = p.batch * p.num_heads;
-    int64_t tile_linear, bh;
-    XcdOrder(p, bh_count, &tile_linear, &bh);
-    const int64_t b = bh / p.num_heads;
-    const int64_t h = bh % p.num_heads;
-    const int64_t h_kv = h / (p.num_heads / p.num_kv_heads);
-    const int qt = static_cast<int>(kCausal ? (num_q_tiles - 1 - tile_linear) : tile_linear);
+    int tile_linear, b_, h_, h_kv_;
+    XcdOrder(p, &tile_linear, &b_, &h_, &h_kv_);
+    const int64_t b = b_, h = h_, h_kv = h_kv_;
+    const int qt = kCausal ? (num_q_tiles - 1 - tile_linear) : tile_linear;
     const int seq_q = static_cast<int>(p.seq_q);
     const int seq_kv = static_cast<int>(p.seq_kv);
     const int diag = static_cast<int>(p.diagonal);
@@ -80,19 +77,6 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
         if (plain < n_plain) n_plain = plain;
     }
     if (n_plain > n_tiles) n_plain = n_tiles;
-
-    // ---- Q fragments of the owned subtile (B operand of S^T = K Q^T) ----
-    vec8 qf[G::KS];
-    {
-        const uint16_t* q_row = static_cast<const uint16_t*>(p.q) + b * p.q_sb + h * p.q_sh +
-                                static_cast<int64_t>(my_q) * p.q_ss + 8 * hh;
-#pragma unroll
-        for (int ks = 0; ks < G::KS; ++ks) {
-            uint4 raw = make_uint4(0, 0, 0, 0);
-            if (my_q < seq_q) raw = *reinterpret_cast<const uint4*>(q_row + 16 * ks);
-            qf[ks] = __builtin_bit_cast(vec8, raw);
-        }
-    }
 
     // ---- DMA (buffer resources bounded at the last row any row of this tile attends) ----
     const uint8_t* k_bytes = reinterpret_cast<const uint8_t*>(
@@ -161,8 +145,6 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
             PinAgpr(o[r][dt]);
         }
     }
-#pragma unroll
-    for (int ks = 0; ks < G::KS; ++ks) PinAgpr(qf[ks]);
     RowState rs;
     float l2 = 0.0f;  // second half of the denominator (two addition chains)
     ResetRow(rs);
@@ -281,8 +263,22 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
 #pragma unroll
         for (int i = 0; i < G::IPW; ++i) dma_k(i, t, t);
     }
+    // Q fragments of the owned subtile (B operand of S^T = K Q^T). Rows past seq_q repeat the last
+    // one (their results are not stored); pinned only after the other tiles' DMAs are issued, so that
+    // nothing waits for them but the first QK.
+    vec8 qf[G::KS];
+    {
+        const uint16_t* q_row = static_cast<const uint16_t*>(p.q) + b * p.q_sb + h * p.q_sh +
+                                static_cast<int64_t>(min(my_q, seq_q - 1)) * p.q_ss + 8 * hh;
+#pragma unroll
+        for (int ks = 0; ks < G::KS; ++ks) {
+            qf[ks] = __builtin_bit_cast(vec8, *reinterpret_cast<const uint4*>(q_row + 16 * ks));
+        }
+    }
     issue(2, 0);
     issue(3, 1);
+#pragma unroll
+    for (int ks = 0; ks < G::KS; ++ks) PinAgpr(qf[ks]);
     if (tid < 8) s_flag[tid] = 0;  // tile 0 is never rescaled for
     WaitVm<4 * G::IPW>();          // K(0), K(1)
     __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -442,18 +438,14 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
         const int sub = dh ^ r;
         const float inv = s_alpha[(rg * 2 + sub) * 32 + lr];
         const int row = row0 + 32 * sub;
-        if (row >= seq_q) continue;
         uint16_t* out_row = static_cast<uint16_t*>(p.out) + b * p.o_sb + h * p.o_sh +
                             static_cast<int64_t>(row) * p.o_ss + dh * (D / 2);
 #pragma unroll
         for (int dt = 0; dt < G::DT; ++dt) {
+            float a[16];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d0 = 32 * dt + 8 * g + 4 * hh;
-                const uint32_t lo = M::pack(o[r][dt][4 * g] * inv, o[r][dt][4 * g + 1] * inv);
-                const uint32_t hi = M::pack(o[r][dt][4 * g + 2] * inv, o[r][dt][4 * g + 3] * inv);
-                *reinterpret_cast<uint2*>(out_row + d0) = make_uint2(lo, hi);
-            }
+            for (int i = 0; i < 16; ++i) a[i] = o[r][dt][i] * inv;
+            StoreTile<M>(out_row + 32 * dt, hh, row < seq_q, a);
         }
     }
 }

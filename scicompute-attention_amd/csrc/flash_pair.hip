@@ -42,12 +42,9 @@ __global__ __launch_bounds__(PairGeom<D>::THREADS, 1) void flash_fwd_pair_kernel
         ++syncs;
     };
 
-    const int64_t bh_count = p.batch * p.num_heads;
-    int64_t tile_linear, bh;
-    XcdOrder(p, bh_count, &tile_linear, &bh);
-    const int64_t b = bh / p.num_heads;
-    const int64_t h = bh % p.num_heads;
-    const int64_t h_kv = h / (p.num_heads / p.num_kv_heads);
+    int tile_linear, b_, h_, h_kv_;
+    XcdOrder(p, &tile_linear, &b_, &h_, &h_kv_);
+    const int64_t b = b_, h = h_, h_kv = h_kv_;
     const int seq_q = static_cast<int>(p.seq_q);
     const int seq_kv = static_cast<int>(p.seq_kv);
     const int diag = static_cast<int>(p.diagonal);
@@ -136,14 +133,13 @@ __global__ __launch_bounds__(PairGeom<D>::THREADS, 1) void flash_fwd_pair_kernel
 
     vec8 qf[G::KS];
     auto load_q = [&](int qt) {
-        const int row = qt * BM + rg * 32 + lr;
+        // Rows past seq_q repeat the last one (their results are not stored).
+        const int row = min(qt * BM + rg * 32 + lr, seq_q - 1);
         const uint16_t* q_row = static_cast<const uint16_t*>(p.q) + b * p.q_sb + h * p.q_sh +
                                 static_cast<int64_t>(row) * p.q_ss + 8 * hh;
 #pragma unroll
         for (int ks = 0; ks < G::KS; ++ks) {
-            uint4 raw = make_uint4(0, 0, 0, 0);
-            if (row < seq_q) raw = *reinterpret_cast<const uint4*>(q_row + 16 * ks);
-            qf[ks] = __builtin_bit_cast(vec8, raw);
+            qf[ks] = __builtin_bit_cast(vec8, *reinterpret_cast<const uint4*>(q_row + 16 * ks));
         }
     };
 
@@ -256,10 +252,11 @@ __global__ __launch_bounds__(PairGeom<D>::THREADS, 1) void flash_fwd_pair_kernel
         uint32_t ph_cur[4];
         float sh_cur;
         if (kb >= n_plain) mask(kb, lim, s_cur);
-        {
-            const float lm = prep(s_cur, ph_cur, sh_cur);
-            fix(lm, s_cur, ph_cur, sh_cur);
-        }
+        // The first maxima; O and l are zero, so nothing is rescaled.
+        rs.m = HalfMax(Max16(s_cur)) * scale2;
+        rs.thr = (rs.m + kRescaleSlack) * inv_scale2;
+        rs.neg_mu = (rs.m == neg_inf()) ? 0.0f : -rs.m;
+        prep(s_cur, ph_cur, sh_cur);
         WaitVm<0>();
         gsync();  // K(kb) read by every wave before step kb refills its slot
         // Step j (S = j & 1): K(j+2) into K slot S and V(j+1) into V slot S^1 (both read in
@@ -419,15 +416,9 @@ __global__ __launch_bounds__(PairGeom<D>::THREADS, 1) void flash_fwd_pair_kernel
                         acc[4 * q4 + 2] = o[dt][4 * q4 + 2] * w0 + v.z * w1;
                         acc[4 * q4 + 3] = o[dt][4 * q4 + 3] * w0 + v.w * w1;
                     }
-                    if (row_ok) {
 #pragma unroll
-                        for (int q4 = 0; q4 < 4; ++q4) {
-                            const int d0 = 32 * dt + 8 * q4 + 4 * hh;
-                            const uint32_t lo = M::pack(acc[4 * q4] * inv, acc[4 * q4 + 1] * inv);
-                            const uint32_t hi = M::pack(acc[4 * q4 + 2] * inv, acc[4 * q4 + 3] * inv);
-                            *reinterpret_cast<uint2*>(out_row + d0) = make_uint2(lo, hi);
-                        }
-                    }
+                    for (int i = 0; i < 16; ++i) acc[i] *= inv;
+                    StoreTile<M>(out_row + 32 * dt, hh, row_ok, acc);
                 }
                 if (row_ok && p.lse != nullptr && hh == 0) {
                     p.lse[(b * p.num_heads + h) * p.seq_q + row] =
@@ -500,15 +491,9 @@ __global__ __launch_bounds__(PairGeom<D>::THREADS, 1) void flash_fwd_pair_kernel
                     acc[4 * q4 + 3] += v.w * wq[q + 1];
                 }
             }
-            if (row_ok) {
 #pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) {
-                    const int d0 = 32 * dt + 8 * q4 + 4 * hh;
-                    const uint32_t lo = M::pack(acc[4 * q4] * inv, acc[4 * q4 + 1] * inv);
-                    const uint32_t hi = M::pack(acc[4 * q4 + 2] * inv, acc[4 * q4 + 3] * inv);
-                    *reinterpret_cast<uint2*>(out_row + d0) = make_uint2(lo, hi);
-                }
-            }
+            for (int i = 0; i < 16; ++i) acc[i] *= inv;
+            StoreTile<M>(out_row + 32 * dt, hh, row_ok, acc);
         }
         if (row_ok && p.lse != nullptr && hh == 0) {
             p.lse[(b * p.num_heads + h) * p.seq_q + row] =

@@ -38,14 +38,11 @@ __global__ __launch_bounds__(FlashGeom<D>::THREADS, 1) void flash_fwd_kernel(
     const int kh = wave / kRowGroups;  // which 32 keys of every tile this wave owns
 
     // Block -> (tile, batch*head). Causal: longest row tiles are dispatched first.
-    const int64_t bh_count = p.batch * p.num_heads;
-    int64_t tile_linear, bh;
-    XcdOrder(p, bh_count, &tile_linear, &bh);
-    const int64_t qt = kCausal ? (num_q_tiles - 1 - tile_linear) : tile_linear;
-    const int64_t b = bh / p.num_heads;
-    const int64_t h = bh % p.num_heads;
-    const int64_t h_kv = h / (p.num_heads / p.num_kv_heads);
-    const int q0 = static_cast<int>(qt) * kBlockM;
+    int tile_linear, b_, h_, h_kv_;
+    XcdOrder(p, &tile_linear, &b_, &h_, &h_kv_);
+    const int qt = kCausal ? (num_q_tiles - 1 - tile_linear) : tile_linear;
+    const int64_t b = b_, h = h_, h_kv = h_kv_;
+    const int q0 = qt * kBlockM;
     const int wave_q0 = q0 + rg * kRowsPerWave;
     const int my_q = wave_q0 + lr;
     const int seq_q = static_cast<int>(p.seq_q);

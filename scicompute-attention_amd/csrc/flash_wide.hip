@@ -21,6 +21,10 @@
 // head dims before: D = 160 causal 398 -> 173 us (432 -> 996 TF/s), non-causal 723 -> 333 us (1,032);
 // D = 96 causal 175 -> 122 us (847), non-causal 315 -> 221 us (932); D = 32 causal 78 -> 57 us,
 // non-causal 141 -> 102 us (672: the softmax VALU bounds it, at 4 MFMAs per 56 VALU operations).
+//
+// With one workgroup per CU its fixed part is not hidden: 8,192 workgroups of one key tile (D = 128)
+// took 322 us, 9.2 us each beside the step; with the K/V DMAs ahead of the wait for Q, 32-bit index
+// arithmetic, no rescale of the zero O and both key halves sharing the merge and the stores 246 us.
 // ============================================================================================
 
 #include <hip/hip_runtime.h>
@@ -52,15 +56,12 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     const int rg = wave & 1;   // row group: rows 64*rg .. +64 of the row tile
     const int kq = wave >> 1;  // key half: keys 32*kq .. +32 of every key tile
 
-    const int64_t bh_count = p.batch * p.num_heads;
-    int64_t tile_linear, bh;
-    XcdOrder(p, bh_count, &tile_linear, &bh);
-    const int64_t b = bh / p.num_heads;
-    const int64_t h = bh % p.num_heads;
-    const int64_t h_kv = h / (p.num_heads / p.num_kv_heads);
+    int tile_linear, b_, h_, h_kv_;
+    XcdOrder(p, &tile_linear, &b_, &h_, &h_kv_);
+    const int64_t b = b_, h = h_, h_kv = h_kv_;
     // Causal: longest row tiles first. A packed varlen launch takes the sequence and row tile of
     // work entry tile_linear (the list is longest first); tok_*: the sequence's first token.
-    int qt = static_cast<int>(kCausal ? (num_q_tiles - 1 - tile_linear) : tile_linear);
+    int qt = kCausal ? (num_q_tiles - 1 - tile_linear) : tile_linear;
     int seq_q = static_cast<int>(p.seq_q);
     int seq_kv = static_cast<int>(p.seq_kv);
     int diag = static_cast<int>(p.diagonal);
@@ -89,21 +90,6 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
         if (plain < n_plain) n_plain = plain;
     }
     if (n_plain > n_tiles) n_plain = n_tiles;
-
-    // ---- Q fragments (B operand of S^T = K Q^T): subtile r, k-step ks ----
-    vec8 qf[G::RT][G::KS];
-#pragma unroll
-    for (int r = 0; r < G::RT; ++r) {
-        const int row = row0 + 32 * r;
-        const uint16_t* q_row = static_cast<const uint16_t*>(p.q) + b * p.q_sb + h * p.q_sh +
-                                (tok_q + row) * p.q_ss + 8 * hh;
-#pragma unroll
-        for (int ks = 0; ks < G::KS; ++ks) {
-            uint4 raw = make_uint4(0, 0, 0, 0);
-            if (row < seq_q) raw = *reinterpret_cast<const uint4*>(q_row + 16 * ks);
-            qf[r][ks] = __builtin_bit_cast(vec8, raw);
-        }
-    }
 
     // ---- DMA (buffer resources bounded at the sequence's last row) ----
     const uint8_t* k_bytes = reinterpret_cast<const uint8_t*>(
@@ -185,11 +171,6 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
             PinAgpr(o[r][dt]);
         }
     }
-#pragma unroll
-    for (int r = 0; r < G::RT; ++r) {
-#pragma unroll
-        for (int ks = 0; ks < G::KS; ++ks) PinAgpr(qf[r][ks]);
-    }
     // Row state (RowState); the denominator is summed in two halves (rs.l and l2), which keeps
     // the two dependency chains of its additions apart.
     RowState rs[G::RT];
@@ -269,12 +250,31 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     // ---- prologue: K(0..3), V(0..2) in flight; S(0), its maxima and rescale; K(1) and V(0)
     //      fragments read for step 0; K(2) and V(1) landed before step 0 ----
     issue_k(0, 0);
+    // Q fragments (B operand of S^T = K Q^T): subtile r, k-step ks. Rows past seq_q repeat the last
+    // one (their results are not stored). Requested behind K(0) and pinned only after the other
+    // tiles' DMAs are issued, so that nothing waits for them but the first QK.
+    vec8 qf[G::RT][G::KS];
+#pragma unroll
+    for (int r = 0; r < G::RT; ++r) {
+        const int row = min(row0 + 32 * r, seq_q - 1);
+        const uint16_t* q_row = static_cast<const uint16_t*>(p.q) + b * p.q_sb + h * p.q_sh +
+                                (tok_q + row) * p.q_ss + 8 * hh;
+#pragma unroll
+        for (int ks = 0; ks < G::KS; ++ks) {
+            qf[r][ks] = __builtin_bit_cast(vec8, *reinterpret_cast<const uint4*>(q_row + 16 * ks));
+        }
+    }
     issue_k(1, 1);
     issue_v(0, 0);
     issue_k(2, 2);
     issue_v(1, 1);
     issue_k(3, 3);
     issue_v(2, 2);
+#pragma unroll
+    for (int r = 0; r < G::RT; ++r) {
+#pragma unroll
+        for (int ks = 0; ks < G::KS; ++ks) PinAgpr(qf[r][ks]);
+    }
     WaitVm<4 * G::IPW>();  // K(0), K(1), V(0)
     __builtin_amdgcn_s_barrier();
     floatx16 s0[G::RT], s1[G::RT];
@@ -290,9 +290,13 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     }
     asm volatile("s_nop 15\n\ts_nop 15");  // the QK results are complete; kf has been read
     {
-        const float lm0 = mask_max(s0[0], 0, 0, n_plain == 0);
-        const float lm1 = mask_max(s0[1], 1, 0, n_plain == 0);
-        rescale_if_grown(lm0, lm1);
+        // The first maxima; O and l are zero, so nothing is rescaled.
+#pragma unroll
+        for (int r = 0; r < G::RT; ++r) {
+            rs[r].m = HalfMax(mask_max(s0[r], r, 0, n_plain == 0)) * scale2;
+            rs[r].thr = (rs[r].m + kRescaleSlack) * inv_scale2;
+            rs[r].neg_mu = (rs[r].m == neg_inf()) ? 0.0f : -rs[r].m;
+        }
     }
     StaticFor<G::KS>([&](auto ks) { read_k1.template operator()<1, ks>(); });
     StaticFor<4 * G::DT>([&](auto i) { read_v1.template operator()<0, 0, i>(); });
@@ -487,63 +491,63 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     WaitVm<0>();
     SettleO(o);
     __builtin_amdgcn_s_barrier();
-    float* const mbuf = reinterpret_cast<float*>(lds8) + rg * kWave * G::MERGE_FLOATS;
-    if (kq == 1) {
-        // O as quads, quad k of lane L at k*64 + L (conflict-free 16-byte accesses).
-        float4* q4 = reinterpret_cast<float4*>(mbuf) + lane;
+    // Wave kq finishes subtile kq: it hands its O and (m, l) of the other subtile to its partner,
+    // as quads (quad k of lane L at k*64 + L: conflict-free 16-byte accesses).
+    auto region = [&](int w) { return reinterpret_cast<float*>(lds8) + w * kWave * G::MERGE_FLOATS; };
+    auto hand_over = [&]<int R>() __attribute__((always_inline)) {
+        float4* q4 = reinterpret_cast<float4*>(region(wave)) + lane;
 #pragma unroll
-        for (int r = 0; r < G::RT; ++r) {
+        for (int dt = 0; dt < G::DT; ++dt) {
 #pragma unroll
-            for (int dt = 0; dt < G::DT; ++dt) {
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    q4[((r * G::DT + dt) * 4 + g) * kWave] =
-                        make_float4(o[r][dt][4 * g], o[r][dt][4 * g + 1], o[r][dt][4 * g + 2],
-                                    o[r][dt][4 * g + 3]);
-                }
+            for (int g = 0; g < 4; ++g) {
+                q4[(dt * 4 + g) * kWave] = make_float4(o[R][dt][4 * g], o[R][dt][4 * g + 1],
+                                                       o[R][dt][4 * g + 2], o[R][dt][4 * g + 3]);
             }
         }
-        float2* st = reinterpret_cast<float2*>(mbuf + G::RT * G::DT * 16 * kWave) + lane;
-#pragma unroll
-        for (int r = 0; r < G::RT; ++r) st[r * kWave] = make_float2(rs[r].m, rs[r].l + l2[r]);
-    }
-    __syncthreads();
-    if (kq == 1) return;
-
-    const float4* q4 = reinterpret_cast<const float4*>(mbuf) + lane;
-    const float2* st = reinterpret_cast<const float2*>(mbuf + G::RT * G::DT * 16 * kWave) + lane;
-#pragma unroll
-    for (int r = 0; r < G::RT; ++r) {
-        const float2 other = st[r * kWave];
-        const float mm = fmaxf(rs[r].m, other.x);
-        const float w0 = (rs[r].m == neg_inf()) ? 0.0f : fast_exp2(rs[r].m - mm);
+        reinterpret_cast<float2*>(region(wave) + G::DT * 16 * kWave)[lane] =
+            make_float2(rs[R].m, rs[R].l + l2[R]);
+    };
+    auto finish = [&]<int R>() __attribute__((always_inline)) {
+        const float* from = region(wave ^ 2);
+        const float4* q4 = reinterpret_cast<const float4*>(from) + lane;
+        const float2 other = reinterpret_cast<const float2*>(from + G::DT * 16 * kWave)[lane];
+        const float mm = fmaxf(rs[R].m, other.x);
+        const float w0 = (rs[R].m == neg_inf()) ? 0.0f : fast_exp2(rs[R].m - mm);
         const float w1 = (other.x == neg_inf()) ? 0.0f : fast_exp2(other.x - mm);
-        const float l_tot = HalfSum((rs[r].l + l2[r]) * w0) + HalfSum(other.y * w1);
+        const float l_tot = HalfSum((rs[R].l + l2[R]) * w0) + HalfSum(other.y * w1);
         const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-        const int row = row0 + 32 * r;
+        const int row = row0 + 32 * R;
         const bool row_ok = row < seq_q;
         uint16_t* out_row = static_cast<uint16_t*>(p.out) + b * p.o_sb + h * p.o_sh +
                             (tok_q + row) * p.o_ss;
 #pragma unroll
         for (int dt = 0; dt < G::DT; ++dt) {
+            float a[16];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const float4 v = q4[((r * G::DT + dt) * 4 + g) * kWave];
-                const float a0 = (o[r][dt][4 * g] * w0 + v.x * w1) * inv;
-                const float a1 = (o[r][dt][4 * g + 1] * w0 + v.y * w1) * inv;
-                const float a2 = (o[r][dt][4 * g + 2] * w0 + v.z * w1) * inv;
-                const float a3 = (o[r][dt][4 * g + 3] * w0 + v.w * w1) * inv;
-                if (row_ok) {
-                    const int d0 = 32 * dt + 8 * g + 4 * hh;
-                    *reinterpret_cast<uint2*>(out_row + d0) =
-                        make_uint2(M::pack(a0, a1), M::pack(a2, a3));
-                }
+                const float4 v = q4[(dt * 4 + g) * kWave];
+                a[4 * g] = (o[R][dt][4 * g] * w0 + v.x * w1) * inv;
+                a[4 * g + 1] = (o[R][dt][4 * g + 1] * w0 + v.y * w1) * inv;
+                a[4 * g + 2] = (o[R][dt][4 * g + 2] * w0 + v.z * w1) * inv;
+                a[4 * g + 3] = (o[R][dt][4 * g + 3] * w0 + v.w * w1) * inv;
             }
+            StoreTile<M>(out_row + 32 * dt, hh, row_ok, a);
         }
         if (row_ok && p.lse != nullptr && hh == 0) {
             p.lse[(b * p.num_heads + h) * p.seq_q + row] =
                 l_tot > 0.0f ? (mm + __log2f(l_tot)) * kLn2 : neg_inf();
         }
+    };
+    if (kq == 0) {
+        hand_over.template operator()<1>();
+    } else {
+        hand_over.template operator()<0>();
+    }
+    __syncthreads();
+    if (kq == 0) {
+        finish.template operator()<0>();
+    } else {
+        finish.template operator()<1>();
     }
 }
 
