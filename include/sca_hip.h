@@ -111,6 +111,9 @@ SCA_HIP_API int sca_hip_device_synchronize(void);
 SCA_HIP_API int sca_hip_stream_create(void** stream);
 SCA_HIP_API int sca_hip_stream_destroy(void* stream);
 SCA_HIP_API int sca_hip_stream_synchronize(void* stream);
+/* *capturing = 1 while work launched on `stream` is recorded into a graph. */
+SCA_HIP_API int sca_hip_stream_is_capturing(void* stream, int* capturing);
+SCA_HIP_API int sca_hip_stream_wait_event(void* stream, void* event);
 SCA_HIP_API int sca_hip_event_create(void** event);
 SCA_HIP_API int sca_hip_event_destroy(void* event);
 SCA_HIP_API int sca_hip_event_record(void* event, void* stream);
@@ -150,6 +153,15 @@ SCA_HIP_API int64_t sca_hip_flash_lds_bytes(int32_t head_dim, int64_t elem_bytes
 SCA_HIP_API int sca_hip_flash_tile(int32_t head_dim, int32_t* block_m, int32_t* block_n,
                                    int32_t* waves, int32_t* stages);
 SCA_HIP_API int sca_hip_flash_fwd(const sca_flash_params* params, void* stream);
+/* The same with caller-provided scratch (device memory, 16 B aligned): calls whose query rows do not
+ * fill the GPU (few new tokens or a chunk over a long context) then run several workgroups per row
+ * tile, each over a range of the keys, and merge their fp32 states from the scratch. The first
+ * function gives the bytes such a run wants (0: it would not split, at most 64 MiB); with less
+ * scratch, or none, the second runs as sca_hip_flash_fwd does. The scratch is in use until the
+ * launch has completed on `stream`. */
+SCA_HIP_API int64_t sca_hip_flash_split_bytes(const sca_flash_params* params);
+SCA_HIP_API int sca_hip_flash_fwd_split(const sca_flash_params* params, void* scratch,
+                                        int64_t scratch_bytes, void* stream);
 
 /* Packed variable-length prefill in one launch (no reference counterpart: the reference's
  * FlashBackend::ForwardVarlen, flash_backend.cpp:226-376, launches once per sequence).

@@ -47,8 +47,8 @@ HIP_FLAGS = [
 # Per-file additions. The flash kernels never produce NaN from finite inputs (masked logits are
 # -inf, fully masked rows are handled explicitly), so NaN-preserving max operations are not needed.
 FILE_FLAGS = {name: ["-fno-honor-nans"] for name in
-              ("flash_fwd.hip", "flash_reg.hip", "flash_pair.hip", "flash_wide.hip",
-               "flash_dsplit.hip")}
+              ("flash_fwd.hip", "flash_reg.hip", "flash_pair.hip", "flash_wide_fp16.hip",
+               "flash_wide_bf16.hip", "flash_dsplit.hip")}
 
 HOST_FLAGS = [
     "-std=c++20",

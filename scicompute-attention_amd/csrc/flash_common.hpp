@@ -1,4 +1,4 @@
-// Shared pieces of the flash prefill kernels (flash_reg.hip, flash_pair.hip, flash_wide.hip) and of
+// Shared pieces of the flash prefill kernels (flash_reg.hip, flash_pair.hip, flash_wide.hpp) and of
 // their dispatch (flash_fwd.hip): MFMA wrappers, the workgroup order, the LDS-DMA pipeline's
 // helpers, the online-softmax row state, the tile geometries and the launchers' declarations.
 //
@@ -144,6 +144,27 @@ struct VarlenArgs {
     const int32_t* tiles;
 };
 
+// How the rows and keys of a launch are cut (wide and split-dims kernels).
+//   pack   query heads of one KV head whose rows share row tiles (1, or the whole GQA group): packed
+//          row R is query R / pack of head R % pack of the group;
+//   splits key ranges per row tile, each in a workgroup of its own. With more than one, workgroup
+//          (tile, split) writes the unnormalised fp32 state of its rows - O, m (log2 units), l - to
+//          part_o [split][row][D] and part_ml [split][row][2] (row = (b*H_q + h)*S_q + q), and
+//          flash_combine_kernel merges them.
+struct SplitArgs {
+    int pack;
+    int splits;
+    float* part_o;
+    float* part_ml;
+};
+
+// The key tiles [first, first + count) of `n_tiles` that split `split` of `splits` takes.
+__device__ __forceinline__ void SplitRange(int n_tiles, int splits, int split, int* first, int* count) {
+    const int chunk = (n_tiles + splits - 1) / splits;
+    *first = split * chunk;
+    *count = max(0, min(n_tiles - *first, chunk));
+}
+
 // Launchers, instantiated in the file of their kernel. Every one validates its grid and returns 0
 // or a status.
 template <typename E, int D, bool kCausal>
@@ -151,11 +172,11 @@ int LaunchFlashReg(const sca_flash_params& p, hipStream_t s);   // flash_reg.hip
 template <typename E, int D>
 int LaunchFlashPair(const sca_flash_params& p, hipStream_t s);  // flash_pair.hip (causal)
 template <typename E, int D, bool kCausal>
-int LaunchFlashWide(const sca_flash_params& p, hipStream_t s);  // flash_wide.hip
+int LaunchFlashWide(const sca_flash_params& p, const SplitArgs& sp, hipStream_t s);  // flash_wide.hpp
 template <typename E, int D, bool kCausal>
-int LaunchFlashDsplit(const sca_flash_params& p, hipStream_t s);  // flash_dsplit.hip
+int LaunchFlashDsplit(const sca_flash_params& p, const SplitArgs& sp, hipStream_t s);  // flash_dsplit.hip
 template <typename E, int D, bool kCausal>
-int LaunchFlashVarlen(const sca_flash_varlen_params& v, hipStream_t s);  // flash_wide.hip
+int LaunchFlashVarlen(const sca_flash_varlen_params& v, hipStream_t s);  // flash_wide.hpp
 
 namespace {
 
@@ -204,10 +225,10 @@ struct Mfma<BF16> {
 // orders survive), and the mapping is a bijection on [0, tiles * bh_count).
 // In 32 bits (the launchers bound the grid, and with it every factor, below 2^31): a 64-bit division
 // takes about 130 instructions on this chip, and eight of them cost each workgroup 0.4 us.
-__device__ __forceinline__ void XcdOrder(const sca_flash_params& p, int* tile_linear, int* b, int* h,
-                                         int* h_kv) {
+// `heads` is the number of head units per batch entry: H_q, or H_kv when a unit packs a whole group.
+__device__ __forceinline__ void XcdOrder(const sca_flash_params& p, uint32_t heads, int* tile_linear,
+                                         int* b, int* h) {
     const uint32_t w = blockIdx.x;
-    const uint32_t heads = static_cast<uint32_t>(p.num_heads);
     const uint32_t kv_heads = static_cast<uint32_t>(p.num_kv_heads);
     const uint32_t groups = static_cast<uint32_t>(p.batch) * kv_heads;
     const uint32_t gsz = heads / kv_heads;
@@ -225,7 +246,6 @@ __device__ __forceinline__ void XcdOrder(const sca_flash_params& p, int* tile_li
     }
     *b = static_cast<int>(bh / heads);
     *h = static_cast<int>(bh % heads);
-    *h_kv = *h / static_cast<int>(gsz);
 }
 
 // Scheduling-group masks of __builtin_amdgcn_sched_group_barrier.
@@ -320,6 +340,16 @@ __device__ __forceinline__ void StoreTile(uint16_t* dst, int hh, bool row_ok, co
         asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1"
                      : "+v"(a0), "+v"(a1), "+v"(b0), "+v"(b1));
         if (row_ok) *reinterpret_cast<u32x4*>(dst + 8 * (g + hh)) = u32x4{a0, a1, b0, b1};
+    }
+}
+
+// The same tile unnormalised and in fp32, for a merge over key splits.
+__device__ __forceinline__ void StorePartialTile(float* dst, int hh, bool row_ok, const float (&v)[16]) {
+    if (!row_ok) return;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        *reinterpret_cast<float4*>(dst + 8 * g + 4 * hh) =
+            make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
     }
 }
 

@@ -34,9 +34,10 @@
 namespace sca_hip {
 namespace {
 
-template <typename E, int D, bool kCausal>
+// kCut: rows packed and / or keys split (SplitArgs).
+template <typename E, int D, bool kCausal, bool kCut>
 __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_kernel(
-    const sca_flash_params p, int num_q_tiles) {
+    const sca_flash_params p, int num_q_tiles, const SplitArgs sp) {
     using G = DsplitGeom<D>;
     using M = Mfma<E>;
     using A = MfmaAsm<E>;
@@ -54,35 +55,80 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
     const int rg = wave & 1;   // rows 64*rg .. +64 of the row tile
     const int dh = wave >> 1;  // QK: rows 32*dh of those; PV: dims D/2*dh .. +D/2
 
-    int tile_linear, b_, h_, h_kv_;
-    XcdOrder(p, &tile_linear, &b_, &h_, &h_kv_);
-    const int64_t b = b_, h = h_, h_kv = h_kv_;
+    const int pack = kCut ? sp.pack : 1;
+    const int splits = kCut ? sp.splits : 1;
+    int tile_linear, b_, unit;
+    XcdOrder(p, static_cast<uint32_t>(p.num_heads) / static_cast<uint32_t>(pack), &tile_linear, &b_,
+             &unit);
+    int split = 0;
+    if (splits > 1) {
+        split = tile_linear % splits;
+        tile_linear /= splits;
+    }
+    const int64_t b = b_;
+    const int64_t h0 = static_cast<int64_t>(unit) * pack;  // first query head
+    const int64_t h_kv =
+        static_cast<int>(h0) / (static_cast<int>(p.num_heads) / static_cast<int>(p.num_kv_heads));
     const int qt = kCausal ? (num_q_tiles - 1 - tile_linear) : tile_linear;
     const int seq_q = static_cast<int>(p.seq_q);
-    const int seq_kv = static_cast<int>(p.seq_kv);
-    const int diag = static_cast<int>(p.diagonal);
+    int seq_kv = static_cast<int>(p.seq_kv);
+    int diag = static_cast<int>(p.diagonal);
     const float scale2 = p.scale * kLog2e;
     const float inv_scale2 = 1.0f / scale2;
     const int q0 = qt * BM;
-    const int row0 = q0 + 64 * rg + lr;   // this lane's row of subtile 0 (subtile 1: +32)
-    const int my_q = row0 + 32 * dh;      // its row of the owned subtile
+    // This lane's rows, of the owned subtile and of the partner's: query position and head offset
+    // within the unit.
+    int qi[2], hl[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        qi[r] = q0 + 64 * rg + 32 * (dh ^ r) + lr;
+        hl[r] = 0;
+        if (pack > 1) {
+            const int row = qi[r];
+            qi[r] = static_cast<int>(static_cast<uint32_t>(row) / static_cast<uint32_t>(pack));
+            hl[r] = row - qi[r] * pack;
+        }
+    }
 
     int n_tiles = (seq_kv + BN - 1) / BN;
     int n_plain = seq_kv / BN;
     if (kCausal) {
-        const int last_key = q0 + BM - 1 + diag;
+        const int q_first = pack > 1 ? q0 / pack : q0;
+        const int q_last = pack > 1 ? (q0 + BM - 1) / pack : q0 + BM - 1;
+        const int last_key = q_last + diag;
         const int causal_tiles = last_key < 0 ? 0 : last_key / BN + 1;
         if (causal_tiles < n_tiles) n_tiles = causal_tiles;
-        const int plain = (q0 + diag + 1) / BN;
+        const int plain = (q_first + diag + 1) / BN;
         if (plain < n_plain) n_plain = plain;
     }
     if (n_plain > n_tiles) n_plain = n_tiles;
+    int64_t key0 = 0;
+    const int64_t rows_all = p.batch * p.num_heads * seq_q;
+    const int64_t flat_own = (b * p.num_heads + h0 + hl[0]) * seq_q + qi[0];
+    if (splits > 1) {
+        // Key tiles [first, first + count): the keys, the causal diagonal and K/V start there.
+        int first, count;
+        SplitRange(n_tiles, splits, split, &first, &count);
+        if (count == 0) {  // fewer key tiles than splits: a state that the merge skips
+            if (hh == 0 && qi[0] < seq_q) {
+                float* ml = sp.part_ml + 2 * (split * rows_all + flat_own);
+                ml[0] = neg_inf();
+                ml[1] = 0.0f;
+            }
+            return;
+        }
+        key0 = static_cast<int64_t>(first) * BN;
+        seq_kv = min(seq_kv - first * BN, count * BN);
+        diag -= first * BN;
+        n_tiles = count;
+        n_plain = max(0, min(n_plain - first, count));
+    }
 
     // ---- DMA (buffer resources bounded at the last row any row of this tile attends) ----
     const uint8_t* k_bytes = reinterpret_cast<const uint8_t*>(
-        static_cast<const uint16_t*>(p.k) + b * p.k_sb + h_kv * p.k_sh);
+        static_cast<const uint16_t*>(p.k) + b * p.k_sb + h_kv * p.k_sh + key0 * p.k_ss);
     const uint8_t* v_bytes = reinterpret_cast<const uint8_t*>(
-        static_cast<const uint16_t*>(p.v) + b * p.v_sb + h_kv * p.v_sh);
+        static_cast<const uint16_t*>(p.v) + b * p.v_sb + h_kv * p.v_sh + key0 * p.v_ss);
     const int k_row_bytes = static_cast<int>(p.k_ss) * 2;
     const int v_row_bytes = static_cast<int>(p.v_ss) * 2;
     const int rows = min(seq_kv, n_tiles * BN);
@@ -174,7 +220,7 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
     auto mask_max = [&](floatx16& sr, int t, bool masked) __attribute__((always_inline)) -> float {
         if (masked) {
             const int kbase = t * BN + 4 * hh;
-            const int lim = kCausal ? min(seq_kv - 1, my_q + diag) : seq_kv - 1;
+            const int lim = kCausal ? min(seq_kv - 1, qi[0] + diag) : seq_kv - 1;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int key = kbase + 8 * (i / 4) + (i % 4);
@@ -268,8 +314,9 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
     // nothing waits for them but the first QK.
     vec8 qf[G::KS];
     {
-        const uint16_t* q_row = static_cast<const uint16_t*>(p.q) + b * p.q_sb + h * p.q_sh +
-                                static_cast<int64_t>(min(my_q, seq_q - 1)) * p.q_ss + 8 * hh;
+        const uint16_t* q_row = static_cast<const uint16_t*>(p.q) + b * p.q_sb +
+                                (h0 + hl[0]) * p.q_sh +
+                                static_cast<int64_t>(min(qi[0], seq_q - 1)) * p.q_ss + 8 * hh;
 #pragma unroll
         for (int ks = 0; ks < G::KS; ++ks) {
             qf[ks] = __builtin_bit_cast(vec8, *reinterpret_cast<const uint4*>(q_row + 16 * ks));
@@ -425,27 +472,44 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
     WaitVm<0>();
     SettleO(o);
     const float l_tot = HalfSum(rs.l + l2);
+    if (splits > 1) {
+        // The unnormalised state: both subtiles' O at the scale of their owner's m.
+        if (hh == 0 && qi[0] < seq_q) {
+            *reinterpret_cast<float2*>(sp.part_ml + 2 * (split * rows_all + flat_own)) =
+                make_float2(rs.m, l_tot);
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const int64_t flat = (b * p.num_heads + h0 + hl[r]) * seq_q + qi[r];
+            float* dst = sp.part_o + (split * rows_all + flat) * D + dh * (D / 2);
+#pragma unroll
+            for (int dt = 0; dt < G::DT; ++dt) {
+                float a[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) a[i] = o[r][dt][i];
+                StorePartialTile(dst + 32 * dt, hh, qi[r] < seq_q, a);
+            }
+        }
+        return;
+    }
     if (hh == 0) {
         s_alpha[(rg * 2 + dh) * 32 + lr] = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-        if (my_q < seq_q && p.lse != nullptr) {
-            p.lse[(b * p.num_heads + h) * p.seq_q + my_q] =
-                l_tot > 0.0f ? (rs.m + __log2f(l_tot)) * kLn2 : neg_inf();
+        if (qi[0] < seq_q && p.lse != nullptr) {
+            p.lse[flat_own] = l_tot > 0.0f ? (rs.m + __log2f(l_tot)) * kLn2 : neg_inf();
         }
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-        const int sub = dh ^ r;
-        const float inv = s_alpha[(rg * 2 + sub) * 32 + lr];
-        const int row = row0 + 32 * sub;
-        uint16_t* out_row = static_cast<uint16_t*>(p.out) + b * p.o_sb + h * p.o_sh +
-                            static_cast<int64_t>(row) * p.o_ss + dh * (D / 2);
+        const float inv = s_alpha[(rg * 2 + (dh ^ r)) * 32 + lr];
+        uint16_t* out_row = static_cast<uint16_t*>(p.out) + b * p.o_sb + (h0 + hl[r]) * p.o_sh +
+                            static_cast<int64_t>(qi[r]) * p.o_ss + dh * (D / 2);
 #pragma unroll
         for (int dt = 0; dt < G::DT; ++dt) {
             float a[16];
 #pragma unroll
             for (int i = 0; i < 16; ++i) a[i] = o[r][dt][i] * inv;
-            StoreTile<M>(out_row + 32 * dt, hh, row < seq_q, a);
+            StoreTile<M>(out_row + 32 * dt, hh, qi[r] < seq_q, a);
         }
     }
 }
@@ -453,33 +517,32 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
 }  // namespace
 
 template <typename E, int D, bool kCausal>
-int LaunchFlashDsplit(const sca_flash_params& p, hipStream_t s) {
+int LaunchFlashDsplit(const sca_flash_params& p, const SplitArgs& sp, hipStream_t s) {
     using G = DsplitGeom<D>;
-    // Buffer offsets are unsigned 32-bit: rows up to seq_kv plus the ring's overrun must fit.
-    const int64_t extent_k = (p.seq_kv + 8 * G::BN) * p.k_ss * 2;
-    const int64_t extent_v = (p.seq_kv + 8 * G::BN) * p.v_ss * 2;
-    if (extent_k >= (1LL << 31) || extent_v >= (1LL << 31) || p.k_ss < 0 || p.v_ss < 0) {
-        return LaunchFlashReg<E, D, kCausal>(p, s);
-    }
-    const int64_t num_q_tiles = (p.seq_q + G::BM - 1) / G::BM;
-    const int64_t blocks = num_q_tiles * p.batch * p.num_heads;
+    const int64_t num_q_tiles = (p.seq_q * sp.pack + G::BM - 1) / G::BM;
+    const int64_t blocks = num_q_tiles * p.batch * (p.num_heads / sp.pack) * sp.splits;
     if (blocks <= 0) return 0;
     if (blocks > 0x7fffffffLL) {
         return SetError(SCA_E_SEQ_TOO_LONG, "flash: grid of " + std::to_string(blocks) +
                                                 " workgroups exceeds the launch limit");
     }
-    if (const int rc = EnsureLdsLimit<&flash_fwd_dsplit_kernel<E, D, kCausal>>(G::LDS_BYTES,
-                                                                             "flash LDS limit")) {
-        return rc;
-    }
-    hipLaunchKernelGGL((flash_fwd_dsplit_kernel<E, D, kCausal>), dim3(static_cast<unsigned>(blocks)),
-                       dim3(G::THREADS), G::LDS_BYTES, s, p, static_cast<int>(num_q_tiles));
-    return CheckLaunch("flash_fwd_dsplit_kernel", s);
+    auto launch = [&]<bool kCut>() -> int {
+        if (const int rc = EnsureLdsLimit<&flash_fwd_dsplit_kernel<E, D, kCausal, kCut>>(
+                G::LDS_BYTES, "flash LDS limit")) {
+            return rc;
+        }
+        hipLaunchKernelGGL((flash_fwd_dsplit_kernel<E, D, kCausal, kCut>),
+                           dim3(static_cast<unsigned>(blocks)), dim3(G::THREADS), G::LDS_BYTES, s, p,
+                           static_cast<int>(num_q_tiles), sp);
+        return CheckLaunch("flash_fwd_dsplit_kernel", s);
+    };
+    return sp.pack == 1 && sp.splits == 1 ? launch.template operator()<false>()
+                                          : launch.template operator()<true>();
 }
 
 #define SCA_INSTANTIATE(E, D)                                                     \
-    template int LaunchFlashDsplit<E, D, false>(const sca_flash_params&, hipStream_t); \
-    template int LaunchFlashDsplit<E, D, true>(const sca_flash_params&, hipStream_t);
+    template int LaunchFlashDsplit<E, D, false>(const sca_flash_params&, const SplitArgs&, hipStream_t); \
+    template int LaunchFlashDsplit<E, D, true>(const sca_flash_params&, const SplitArgs&, hipStream_t);
 SCA_INSTANTIATE(F16, 192)
 SCA_INSTANTIATE(F16, 256)
 SCA_INSTANTIATE(BF16, 192)

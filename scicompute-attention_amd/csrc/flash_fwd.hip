@@ -8,7 +8,7 @@
 // out = O / l (0 when l == 0), LSE = m + ln(l) (-inf when l == 0).
 //
 // Three kernels share one formulation (flash_common.hpp); this file validates and picks:
-//   * flash_wide.hip (head_dim 32 to 160: every non-causal grid, large causal grids and, at 64 and
+//   * flash_wide.hpp (head_dim 32 to 160: every non-causal grid, large causal grids and, at 64 and
 //     128, packed variable-length batches in one launch): 4 waves of 64 query rows, K/V tiles
 //     DMA'd into LDS;
 //   * flash_pair.hip (head_dim 64 and 128, causal grids too small to balance 128-row tiles);
@@ -27,12 +27,7 @@
 namespace sca_hip {
 namespace {
 
-// Causal grids with at most one 128-row tile per CU run the pair kernel (64-row tiles in
-// complementary pairs, so every workgroup holds the same share of the triangle); larger causal
-// grids and every non-causal grid run the wide kernel (longest tiles first when causal). Measured
-// warm: at 320-448 tiles on 256 CUs the longest-first 128-row grid is 20-30% faster than a
-// second partial wave of pairs; at 256 tiles the pairs are 30% faster.
-bool UsePairs(const sca_flash_params& p) {
+int CuCount() {
     static int cu_count = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -42,28 +37,186 @@ bool UsePairs(const sca_flash_params& p) {
         }
         return n > 0 ? n : 256;
     }();
-    const int64_t tiles128 = (p.seq_q + 127) / 128 * p.batch * p.num_heads;
-    return tiles128 <= static_cast<int64_t>(cu_count);
+    return cu_count;
+}
+
+// Whether the DMA kernels' unsigned 32-bit buffer offsets reach every row (plus the rings' overrun).
+bool DmaReach(const sca_flash_params& p) {
+    constexpr int64_t kOverrun = 8 * 64;
+    return p.k_ss >= 0 && p.v_ss >= 0 && (p.seq_kv + kOverrun) * p.k_ss * 2 < (1LL << 31) &&
+           (p.seq_kv + kOverrun) * p.v_ss * 2 < (1LL << 31);
+}
+
+// ---- Which kernel, and how its rows and keys are cut -------------------------------------------
+struct FlashPlan {
+    bool pair;
+    int pack;
+    int splits;
+};
+
+constexpr int64_t kMaxSplitBytes = int64_t{64} << 20;
+
+int64_t SplitBytes(const sca_flash_params& p, int splits) {
+    return splits <= 1 ? 0 : p.batch * p.num_heads * p.seq_q * splits * (p.head_dim + 2) * 4;
+}
+
+// Causal grids with at most one 128-row tile per CU run the pair kernel at head_dim 64 and 128 (64-row
+// tiles in complementary pairs, so every workgroup holds the same share of the triangle); larger
+// causal grids and every non-causal grid run the wide kernel (longest tiles first when causal).
+// Measured warm: at 320-448 tiles on 256 CUs the longest-first 128-row grid is 20-30% faster than a
+// second partial wave of pairs; at 256 tiles the pairs are 30% faster.
+//
+// Packing (a GQA group's rows share row tiles) is taken where it leaves fewer row tiles: with few
+// query rows a tile per head is mostly empty and K/V are streamed once per query head.
+//
+// Splitting the keys (allow_split: the caller has scratch for the partial states) pays where the row
+// tiles do not fill the CUs and the keys are many. The estimate below, in microseconds, weighs it
+// against the unsplit kernel: a wide or split-dims workgroup (one per CU) takes about 0.1 + 0.0068 D
+// per 64 keys and 4 + 0.022 D beside them, a pair workgroup 1.19 times the step per 64 keys of two
+// groups and 5 beside them (both fitted to measurements at D = 32 .. 256), and the merge 5 plus its
+// partials' write and read at 4.5 TB/s.
+FlashPlan PlanFlash(const sca_flash_params& p, bool allow_split) {
+    const int64_t cus = CuCount();
+    const int64_t group = p.num_heads / p.num_kv_heads;
+    const int64_t tiles = (p.seq_q + 127) / 128;
+    FlashPlan plan{false, 1, 1};
+    plan.pair = p.causal && (p.head_dim == 64 || p.head_dim == 128) &&
+                tiles * p.batch * p.num_heads <= cus;
+    const int64_t packed_tiles = (p.seq_q * group + 127) / 128;
+    const int pack = packed_tiles < tiles * group && p.seq_q * group < (1LL << 30)
+                         ? static_cast<int>(group) : 1;
+    if (!plan.pair) plan.pack = pack;
+    if (!allow_split) return plan;
+
+    const double step = 0.1 + 0.0068 * static_cast<double>(p.head_dim);
+    const double fixed = 4.0 + 0.022 * static_cast<double>(p.head_dim);
+    const int64_t keys_max = p.seq_kv;
+    const double keys_avg = p.causal ? static_cast<double>(p.diagonal) + 0.5 * static_cast<double>(p.seq_q)
+                                     : static_cast<double>(p.seq_kv);
+    auto wide_us = [&](int64_t units, int64_t splits) {
+        const double longest = static_cast<double>((keys_max + 64 * splits - 1) / (64 * splits)) * step + fixed;
+        const double rounds = static_cast<double>((units * splits + cus - 1) / cus);
+        const double all = rounds * (keys_avg / 64.0 / static_cast<double>(splits) * step + fixed);
+        return longest > all ? longest : all;
+    };
+    double best;
+    const int64_t units_pack = (pack > 1 ? packed_tiles : tiles) * p.batch * p.num_heads / pack;
+    if (plan.pair) {
+        const int64_t t64 = (p.seq_q + 63) / 64;
+        const int64_t n_a = (p.seq_kv + 63) / 64;
+        const int64_t n_b = t64 > 1 ? (p.diagonal + 64 + 63) / 64 + 4 : 0;
+        const int64_t wgs = (t64 + 1) / 2 * p.batch * p.num_heads;
+        best = static_cast<double>((wgs + cus - 1) / cus) *
+               (0.5 * static_cast<double>(n_a + n_b) * 1.19 * step + 5.0);
+    } else {
+        best = wide_us(units_pack, 1);
+    }
+    best *= 0.93;  // a split has to promise more than the estimate's error
+    for (int64_t splits = 2; splits <= 16 && splits * 4 * 64 <= p.seq_kv; ++splits) {
+        const int64_t bytes = SplitBytes(p, static_cast<int>(splits));
+        if (bytes > kMaxSplitBytes) break;
+        const double us = wide_us(units_pack, splits) + 5.0 + 2.0 * static_cast<double>(bytes) / 4.5e6;
+        if (us < best) {
+            best = us;
+            plan = FlashPlan{false, pack, static_cast<int>(splits)};
+        }
+    }
+    return plan;
+}
+
+// Merges the partial states of `splits` key ranges: out = sum_s O_s 2^(m_s - m*) / sum_s l_s 2^(m_s - m*)
+// with m* = max_s m_s (log2 units), states with m_s = -inf skipped and out = 0 when the denominator
+// is 0; LSE = m* + log2 of the denominator, in natural units. One thread per row and 4 dims; bound by
+// the partials' bytes.
+constexpr int kCombineThreads = 256;
+
+template <typename E>
+__global__ __launch_bounds__(kCombineThreads) void flash_combine_kernel(const sca_flash_params p,
+                                                                        const SplitArgs sp) {
+    using M = Mfma<E>;
+    const uint32_t quads = static_cast<uint32_t>(p.head_dim) / 4;
+    const uint32_t rows = static_cast<uint32_t>(p.batch * p.num_heads * p.seq_q);
+    const uint32_t idx = blockIdx.x * kCombineThreads + threadIdx.x;
+    const uint32_t row = idx / quads;
+    if (row >= rows) return;
+    const uint32_t d0 = (idx % quads) * 4;
+    const float2* ml = reinterpret_cast<const float2*>(sp.part_ml) + row;
+    const float* po = sp.part_o + static_cast<int64_t>(row) * p.head_dim + d0;
+    float m = neg_inf();
+#pragma unroll 4
+    for (int s = 0; s < sp.splits; ++s) m = fmaxf(m, ml[static_cast<int64_t>(s) * rows].x);
+    float l = 0.0f;
+    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int s = 0; s < sp.splits; ++s) {
+        const float2 st = ml[static_cast<int64_t>(s) * rows];
+        if (st.x == neg_inf()) continue;  // its O was not written
+        const float w = fast_exp2(st.x - m);
+        l = fmaf(st.y, w, l);
+        const float4 v = *reinterpret_cast<const float4*>(po + static_cast<int64_t>(s) * rows * p.head_dim);
+        a[0] = fmaf(v.x, w, a[0]);
+        a[1] = fmaf(v.y, w, a[1]);
+        a[2] = fmaf(v.z, w, a[2]);
+        a[3] = fmaf(v.w, w, a[3]);
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const uint32_t seq_q = static_cast<uint32_t>(p.seq_q), heads = static_cast<uint32_t>(p.num_heads);
+    const uint32_t bh = row / seq_q;
+    uint16_t* out = static_cast<uint16_t*>(p.out) + static_cast<int64_t>(bh / heads) * p.o_sb +
+                    static_cast<int64_t>(bh % heads) * p.o_sh +
+                    static_cast<int64_t>(row % seq_q) * p.o_ss + d0;
+    *reinterpret_cast<uint2*>(out) =
+        make_uint2(M::pack(a[0] * inv, a[1] * inv), M::pack(a[2] * inv, a[3] * inv));
+    if (p.lse != nullptr && d0 == 0) {
+        p.lse[row] = l > 0.0f ? (m + __log2f(l)) * kLn2 : neg_inf();
+    }
 }
 
 template <typename E, bool kCausal>
-int LaunchForDim(const sca_flash_params& p, hipStream_t s) {
+int LaunchForDim(const sca_flash_params& p, const FlashPlan& plan, const SplitArgs& sp, hipStream_t s) {
+    const bool reach = DmaReach(p);
     switch (p.head_dim) {
-        case 32: return LaunchFlashWide<E, 32, kCausal>(p, s);
+        case 32:
+            return reach ? LaunchFlashWide<E, 32, kCausal>(p, sp, s) : LaunchFlashReg<E, 32, kCausal>(p, s);
         case 64:
-            if (kCausal && UsePairs(p)) return LaunchFlashPair<E, 64>(p, s);
-            return LaunchFlashWide<E, 64, kCausal>(p, s);
-        case 96: return LaunchFlashWide<E, 96, kCausal>(p, s);
+            if (!reach) return LaunchFlashReg<E, 64, kCausal>(p, s);
+            if (kCausal && plan.pair) return LaunchFlashPair<E, 64>(p, s);
+            return LaunchFlashWide<E, 64, kCausal>(p, sp, s);
+        case 96:
+            return reach ? LaunchFlashWide<E, 96, kCausal>(p, sp, s) : LaunchFlashReg<E, 96, kCausal>(p, s);
         case 128:
-            if (kCausal && UsePairs(p)) return LaunchFlashPair<E, 128>(p, s);
-            return LaunchFlashWide<E, 128, kCausal>(p, s);
-        case 160: return LaunchFlashWide<E, 160, kCausal>(p, s);
-        case 192: return LaunchFlashDsplit<E, 192, kCausal>(p, s);
-        case 256: return LaunchFlashDsplit<E, 256, kCausal>(p, s);
+            if (!reach) return LaunchFlashReg<E, 128, kCausal>(p, s);
+            if (kCausal && plan.pair) return LaunchFlashPair<E, 128>(p, s);
+            return LaunchFlashWide<E, 128, kCausal>(p, sp, s);
+        case 160:
+            return reach ? LaunchFlashWide<E, 160, kCausal>(p, sp, s) : LaunchFlashReg<E, 160, kCausal>(p, s);
+        case 192:
+            return reach ? LaunchFlashDsplit<E, 192, kCausal>(p, sp, s) : LaunchFlashReg<E, 192, kCausal>(p, s);
+        case 256:
+            return reach ? LaunchFlashDsplit<E, 256, kCausal>(p, sp, s) : LaunchFlashReg<E, 256, kCausal>(p, s);
         default: break;
     }
     return SetError(SCA_E_UNSUPPORTED_HEAD_DIM,
                     "flash: head_dim=" + std::to_string(p.head_dim) + " is not instantiated");
+}
+
+template <typename E>
+int LaunchTyped(const sca_flash_params& p, void* scratch, int64_t scratch_bytes, hipStream_t s) {
+    FlashPlan plan = PlanFlash(p, scratch != nullptr && DmaReach(p));
+    if (SplitBytes(p, plan.splits) > scratch_bytes) plan = PlanFlash(p, false);
+    SplitArgs sp{plan.pack, plan.splits, nullptr, nullptr};
+    const int64_t rows = p.batch * p.num_heads * p.seq_q;
+    if (plan.splits > 1) {
+        sp.part_o = static_cast<float*>(scratch);
+        sp.part_ml = sp.part_o + rows * plan.splits * p.head_dim;
+    }
+    const int rc = p.causal ? LaunchForDim<E, true>(p, plan, sp, s) : LaunchForDim<E, false>(p, plan, sp, s);
+    if (rc != 0 || plan.splits == 1) return rc;
+    const int64_t threads = rows * (p.head_dim / 4);
+    hipLaunchKernelGGL((flash_combine_kernel<E>),
+                       dim3(static_cast<unsigned>((threads + kCombineThreads - 1) / kCombineThreads)),
+                       dim3(kCombineThreads), 0, s, p, sp);
+    return CheckLaunch("flash_combine_kernel", s);
 }
 
 bool Aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
@@ -193,7 +346,11 @@ int sca_hip_flash_fwd_varlen(const sca_flash_varlen_params* v, void* stream) {
                                      : sca_hip::LaunchVarlenTyped<sca_hip::BF16>(*v, s);
 }
 
-int sca_hip_flash_fwd(const sca_flash_params* p, void* stream) {
+}  // extern "C"
+
+namespace sca_hip {
+namespace {
+int ValidateFlash(const sca_flash_params* p) {
     if (p == nullptr) return SetError(SCA_E_SHAPE_MISMATCH, "flash: null params");
     if (p->q == nullptr || p->k == nullptr || p->v == nullptr || p->out == nullptr) {
         return SetError(SCA_E_SHAPE_MISMATCH, "flash: null pointer");
@@ -231,13 +388,33 @@ int sca_hip_flash_fwd(const sca_flash_params* p, void* stream) {
         return SetError(SCA_E_LAYOUT_MISMATCH,
                         "flash: q/k/v/out must be 16 B aligned with 16 B-multiple row strides");
     }
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (p->dtype == SCA_DTYPE_F16) {
-        return p->causal ? sca_hip::LaunchForDim<sca_hip::F16, true>(*p, s)
-                         : sca_hip::LaunchForDim<sca_hip::F16, false>(*p, s);
+    return 0;
+}
+}  // namespace
+}  // namespace sca_hip
+
+extern "C" {
+
+int64_t sca_hip_flash_split_bytes(const sca_flash_params* p) {
+    if (sca_hip::ValidateFlash(p) != 0 || !sca_hip::DmaReach(*p)) return 0;
+    return sca_hip::SplitBytes(*p, sca_hip::PlanFlash(*p, true).splits);
+}
+
+int sca_hip_flash_fwd_split(const sca_flash_params* p, void* scratch, int64_t scratch_bytes,
+                            void* stream) {
+    const int rc = sca_hip::ValidateFlash(p);
+    if (rc != 0) return rc;
+    if (!sca_hip::Aligned16(scratch)) {
+        return SetError(SCA_E_LAYOUT_MISMATCH, "flash: scratch must be 16 B aligned");
     }
-    return p->causal ? sca_hip::LaunchForDim<sca_hip::BF16, true>(*p, s)
-                     : sca_hip::LaunchForDim<sca_hip::BF16, false>(*p, s);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    return p->dtype == SCA_DTYPE_F16
+               ? sca_hip::LaunchTyped<sca_hip::F16>(*p, scratch, scratch_bytes, s)
+               : sca_hip::LaunchTyped<sca_hip::BF16>(*p, scratch, scratch_bytes, s);
+}
+
+int sca_hip_flash_fwd(const sca_flash_params* p, void* stream) {
+    return sca_hip_flash_fwd_split(p, nullptr, 0, stream);
 }
 
 }  // extern "C"

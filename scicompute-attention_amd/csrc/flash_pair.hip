@@ -42,9 +42,10 @@ __global__ __launch_bounds__(PairGeom<D>::THREADS, 1) void flash_fwd_pair_kernel
         ++syncs;
     };
 
-    int tile_linear, b_, h_, h_kv_;
-    XcdOrder(p, &tile_linear, &b_, &h_, &h_kv_);
-    const int64_t b = b_, h = h_, h_kv = h_kv_;
+    int tile_linear, b_, h_;
+    XcdOrder(p, static_cast<uint32_t>(p.num_heads), &tile_linear, &b_, &h_);
+    const int64_t b = b_, h = h_;
+    const int64_t h_kv = h_ / (static_cast<int>(p.num_heads) / static_cast<int>(p.num_kv_heads));
     const int seq_q = static_cast<int>(p.seq_q);
     const int seq_kv = static_cast<int>(p.seq_kv);
     const int diag = static_cast<int>(p.diagonal);
@@ -507,11 +508,6 @@ __global__ __launch_bounds__(PairGeom<D>::THREADS, 1) void flash_fwd_pair_kernel
 template <typename E, int D>
 int LaunchFlashPair(const sca_flash_params& p, hipStream_t s) {
     using G = PairGeom<D>;
-    const int64_t extent_k = (p.seq_kv + 4 * G::BN) * p.k_ss * 2;
-    const int64_t extent_v = (p.seq_kv + 4 * G::BN) * p.v_ss * 2;
-    if (extent_k >= (1LL << 31) || extent_v >= (1LL << 31) || p.k_ss < 0 || p.v_ss < 0) {
-        return LaunchFlashReg<E, D, true>(p, s);
-    }
     const int64_t num_q_tiles = (p.seq_q + G::BM - 1) / G::BM;
     const int64_t blocks = (num_q_tiles + 1) / 2 * p.batch * p.num_heads;
     if (blocks <= 0) return 0;

@@ -38,10 +38,11 @@ __global__ __launch_bounds__(FlashGeom<D>::THREADS, 1) void flash_fwd_kernel(
     const int kh = wave / kRowGroups;  // which 32 keys of every tile this wave owns
 
     // Block -> (tile, batch*head). Causal: longest row tiles are dispatched first.
-    int tile_linear, b_, h_, h_kv_;
-    XcdOrder(p, &tile_linear, &b_, &h_, &h_kv_);
+    int tile_linear, b_, h_;
+    XcdOrder(p, static_cast<uint32_t>(p.num_heads), &tile_linear, &b_, &h_);
     const int qt = kCausal ? (num_q_tiles - 1 - tile_linear) : tile_linear;
-    const int64_t b = b_, h = h_, h_kv = h_kv_;
+    const int64_t b = b_, h = h_;
+    const int64_t h_kv = h_ / (static_cast<int>(p.num_heads) / static_cast<int>(p.num_kv_heads));
     const int q0 = qt * kBlockM;
     const int wave_q0 = q0 + rg * kRowsPerWave;
     const int my_q = wave_q0 + lr;

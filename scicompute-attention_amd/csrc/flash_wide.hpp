@@ -27,6 +27,8 @@
 // arithmetic, no rescale of the zero O and both key halves sharing the merge and the stores 246 us.
 // ============================================================================================
 
+#pragma once
+
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -36,9 +38,12 @@
 namespace sca_hip {
 namespace {
 
-template <typename E, int D, bool kCausal, bool kVarlen>
+// kMode: plain, packed varlen, or cut (rows packed and / or keys split: SplitArgs).
+enum WideMode { kPlain, kPackedVarlen, kCut };
+
+template <typename E, int D, bool kCausal, WideMode kMode>
 __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel(
-    const sca_flash_params p, int num_q_tiles, const VarlenArgs vl) {
+    const sca_flash_params p, int num_q_tiles, const VarlenArgs vl, const SplitArgs sp) {
     using G = WideGeom<D>;
     using M = Mfma<E>;
     using A = MfmaAsm<E>;
@@ -46,6 +51,7 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     constexpr int BN = G::BN;
     constexpr int BM = G::BM;
     constexpr int RB = G::ROW_BYTES;
+    constexpr bool kVarlen = kMode == kPackedVarlen;
 
     extern __shared__ __align__(16) uint8_t lds8[];
     const int tid = threadIdx.x;
@@ -56,9 +62,20 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     const int rg = wave & 1;   // row group: rows 64*rg .. +64 of the row tile
     const int kq = wave >> 1;  // key half: keys 32*kq .. +32 of every key tile
 
-    int tile_linear, b_, h_, h_kv_;
-    XcdOrder(p, &tile_linear, &b_, &h_, &h_kv_);
-    const int64_t b = b_, h = h_, h_kv = h_kv_;
+    const int pack = kMode == kCut ? sp.pack : 1;
+    const int splits = kMode == kCut ? sp.splits : 1;
+    int tile_linear, b_, unit;
+    XcdOrder(p, static_cast<uint32_t>(p.num_heads) / static_cast<uint32_t>(pack), &tile_linear, &b_,
+             &unit);
+    int split = 0;
+    if (splits > 1) {
+        split = tile_linear % splits;
+        tile_linear /= splits;
+    }
+    const int64_t b = b_;
+    const int64_t h0 = static_cast<int64_t>(unit) * pack;  // first query head
+    const int64_t h_kv =
+        static_cast<int>(h0) / (static_cast<int>(p.num_heads) / static_cast<int>(p.num_kv_heads));
     // Causal: longest row tiles first. A packed varlen launch takes the sequence and row tile of
     // work entry tile_linear (the list is longest first); tok_*: the sequence's first token.
     int qt = kCausal ? (num_q_tiles - 1 - tile_linear) : tile_linear;
@@ -78,18 +95,54 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     const float scale2 = p.scale * kLog2e;
     const float inv_scale2 = 1.0f / scale2;
     const int q0 = qt * BM;
-    const int row0 = q0 + 64 * rg + lr;  // row of subtile 0 (subtile 1: +32)
+    // This lane's rows (subtile 0, subtile 1): query position and head offset within the unit.
+    int qi[G::RT], hl[G::RT];
+#pragma unroll
+    for (int r = 0; r < G::RT; ++r) {
+        qi[r] = q0 + 64 * rg + 32 * r + lr;
+        hl[r] = 0;
+        if (pack > 1) {
+            const int row = qi[r];
+            qi[r] = static_cast<int>(static_cast<uint32_t>(row) / static_cast<uint32_t>(pack));
+            hl[r] = row - qi[r] * pack;
+        }
+    }
 
     int n_tiles = (seq_kv + BN - 1) / BN;
     int n_plain = seq_kv / BN;
     if (kCausal) {
-        const int last_key = q0 + BM - 1 + diag;
+        const int q_first = pack > 1 ? q0 / pack : q0;
+        const int q_last = pack > 1 ? (q0 + BM - 1) / pack : q0 + BM - 1;
+        const int last_key = q_last + diag;
         const int causal_tiles = last_key < 0 ? 0 : last_key / BN + 1;
         if (causal_tiles < n_tiles) n_tiles = causal_tiles;
-        const int plain = (q0 + diag + 1) / BN;
+        const int plain = (q_first + diag + 1) / BN;
         if (plain < n_plain) n_plain = plain;
     }
     if (n_plain > n_tiles) n_plain = n_tiles;
+    if (splits > 1) {
+        // Key tiles [first, first + count): the keys, the causal diagonal and K/V start there.
+        int first, count;
+        SplitRange(n_tiles, splits, split, &first, &count);
+        if (count == 0) {  // fewer key tiles than splits: a state that the merge skips
+            if (hh == 0) {
+                const int r = kq;  // each of the two waves of a row group covers one subtile
+                const int q = r == 0 ? qi[0] : qi[1];
+                const int64_t row = (b * p.num_heads + h0 + (r == 0 ? hl[0] : hl[1])) * seq_q + q;
+                if (q < seq_q) {
+                    float* ml = sp.part_ml + 2 * (split * p.batch * p.num_heads * seq_q + row);
+                    ml[0] = neg_inf();
+                    ml[1] = 0.0f;
+                }
+            }
+            return;
+        }
+        tok_kv = static_cast<int64_t>(first) * BN;
+        seq_kv = min(seq_kv - first * BN, count * BN);
+        diag -= first * BN;
+        n_tiles = count;
+        n_plain = max(0, min(n_plain - first, count));
+    }
 
     // ---- DMA (buffer resources bounded at the sequence's last row) ----
     const uint8_t* k_bytes = reinterpret_cast<const uint8_t*>(
@@ -210,7 +263,7 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     auto mask_max = [&](floatx16& sr, int r, int t, bool masked) __attribute__((always_inline)) -> float {
         if (masked) {
             const int kbase = t * BN + 32 * kq + 4 * hh;
-            const int lim = kCausal ? min(seq_kv - 1, row0 + 32 * r + diag) : seq_kv - 1;
+            const int lim = kCausal ? min(seq_kv - 1, qi[r] + diag) : seq_kv - 1;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int key = kbase + 8 * (i / 4) + (i % 4);
@@ -256,9 +309,9 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     vec8 qf[G::RT][G::KS];
 #pragma unroll
     for (int r = 0; r < G::RT; ++r) {
-        const int row = min(row0 + 32 * r, seq_q - 1);
-        const uint16_t* q_row = static_cast<const uint16_t*>(p.q) + b * p.q_sb + h * p.q_sh +
-                                (tok_q + row) * p.q_ss + 8 * hh;
+        const int row = min(qi[r], seq_q - 1);
+        const uint16_t* q_row = static_cast<const uint16_t*>(p.q) + b * p.q_sb +
+                                (h0 + hl[r]) * p.q_sh + (tok_q + row) * p.q_ss + 8 * hh;
 #pragma unroll
         for (int ks = 0; ks < G::KS; ++ks) {
             qf[r][ks] = __builtin_bit_cast(vec8, *reinterpret_cast<const uint4*>(q_row + 16 * ks));
@@ -516,8 +569,30 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
         const float w1 = (other.x == neg_inf()) ? 0.0f : fast_exp2(other.x - mm);
         const float l_tot = HalfSum((rs[R].l + l2[R]) * w0) + HalfSum(other.y * w1);
         const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-        const int row = row0 + 32 * R;
+        const int row = qi[R];
         const bool row_ok = row < seq_q;
+        const int64_t h = h0 + hl[R];
+        const int64_t flat = (b * p.num_heads + h) * seq_q + row;  // not used by varlen launches
+        if (splits > 1) {
+            const int64_t at = split * p.batch * p.num_heads * seq_q + flat;
+#pragma unroll
+            for (int dt = 0; dt < G::DT; ++dt) {
+                float a[16];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float4 v = q4[(dt * 4 + g) * kWave];
+                    a[4 * g] = o[R][dt][4 * g] * w0 + v.x * w1;
+                    a[4 * g + 1] = o[R][dt][4 * g + 1] * w0 + v.y * w1;
+                    a[4 * g + 2] = o[R][dt][4 * g + 2] * w0 + v.z * w1;
+                    a[4 * g + 3] = o[R][dt][4 * g + 3] * w0 + v.w * w1;
+                }
+                StorePartialTile(sp.part_o + at * D + 32 * dt, hh, row_ok, a);
+            }
+            if (row_ok && hh == 0) {
+                *reinterpret_cast<float2*>(sp.part_ml + 2 * at) = make_float2(mm, l_tot);
+            }
+            return;
+        }
         uint16_t* out_row = static_cast<uint16_t*>(p.out) + b * p.o_sb + h * p.o_sh +
                             (tok_q + row) * p.o_ss;
 #pragma unroll
@@ -534,8 +609,7 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
             StoreTile<M>(out_row + 32 * dt, hh, row_ok, a);
         }
         if (row_ok && p.lse != nullptr && hh == 0) {
-            p.lse[(b * p.num_heads + h) * p.seq_q + row] =
-                l_tot > 0.0f ? (mm + __log2f(l_tot)) * kLn2 : neg_inf();
+            p.lse[flat] = l_tot > 0.0f ? (mm + __log2f(l_tot)) * kLn2 : neg_inf();
         }
     };
     if (kq == 0) {
@@ -554,29 +628,27 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
 }  // namespace
 
 template <typename E, int D, bool kCausal>
-int LaunchFlashWide(const sca_flash_params& p, hipStream_t s) {
+int LaunchFlashWide(const sca_flash_params& p, const SplitArgs& sp, hipStream_t s) {
     using G = WideGeom<D>;
-    // Buffer offsets are unsigned 32-bit: rows up to seq_kv plus the ring's overrun must fit.
-    const int64_t extent_k = (p.seq_kv + 8 * G::BN) * p.k_ss * 2;
-    const int64_t extent_v = (p.seq_kv + 8 * G::BN) * p.v_ss * 2;
-    if (extent_k >= (1LL << 31) || extent_v >= (1LL << 31) || p.k_ss < 0 || p.v_ss < 0) {
-        return LaunchFlashReg<E, D, kCausal>(p, s);
-    }
-    const int64_t num_q_tiles = (p.seq_q + G::BM - 1) / G::BM;
-    const int64_t blocks = num_q_tiles * p.batch * p.num_heads;
+    const int64_t num_q_tiles = (p.seq_q * sp.pack + G::BM - 1) / G::BM;
+    const int64_t blocks = num_q_tiles * p.batch * (p.num_heads / sp.pack) * sp.splits;
     if (blocks <= 0) return 0;
     if (blocks > 0x7fffffffLL) {
         return SetError(SCA_E_SEQ_TOO_LONG, "flash: grid of " + std::to_string(blocks) +
                                                 " workgroups exceeds the launch limit");
     }
-    if (const int rc =
-            EnsureLdsLimit<&flash_fwd_wide_kernel<E, D, kCausal, false>>(G::LDS_BYTES, "flash LDS limit")) {
-        return rc;
-    }
-    hipLaunchKernelGGL((flash_fwd_wide_kernel<E, D, kCausal, false>),
-                       dim3(static_cast<unsigned>(blocks)), dim3(G::THREADS), G::LDS_BYTES, s, p,
-                       static_cast<int>(num_q_tiles), VarlenArgs{nullptr, nullptr, nullptr});
-    return CheckLaunch("flash_fwd_wide_kernel", s);
+    auto launch = [&]<WideMode kMode>() -> int {
+        if (const int rc = EnsureLdsLimit<&flash_fwd_wide_kernel<E, D, kCausal, kMode>>(
+                G::LDS_BYTES, "flash LDS limit")) {
+            return rc;
+        }
+        hipLaunchKernelGGL((flash_fwd_wide_kernel<E, D, kCausal, kMode>),
+                           dim3(static_cast<unsigned>(blocks)), dim3(G::THREADS), G::LDS_BYTES, s, p,
+                           static_cast<int>(num_q_tiles), VarlenArgs{nullptr, nullptr, nullptr}, sp);
+        return CheckLaunch("flash_fwd_wide_kernel", s);
+    };
+    return sp.pack == 1 && sp.splits == 1 ? launch.template operator()<kPlain>()
+                                          : launch.template operator()<kCut>();
 }
 
 // One launch over a packed batch: the wide kernel, one workgroup per (work entry, head).
@@ -613,27 +685,15 @@ int LaunchFlashVarlen(const sca_flash_varlen_params& v, hipStream_t s) {
     p.scale = v.scale;
     p.causal = v.causal;
     p.dtype = v.dtype;
-    if (const int rc = EnsureLdsLimit<&flash_fwd_wide_kernel<E, D, kCausal, true>>(
+    if (const int rc = EnsureLdsLimit<&flash_fwd_wide_kernel<E, D, kCausal, kPackedVarlen>>(
             G::LDS_BYTES, "flash LDS limit")) {
         return rc;
     }
-    hipLaunchKernelGGL((flash_fwd_wide_kernel<E, D, kCausal, true>),
+    hipLaunchKernelGGL((flash_fwd_wide_kernel<E, D, kCausal, kPackedVarlen>),
                        dim3(static_cast<unsigned>(blocks)), dim3(G::THREADS), G::LDS_BYTES, s, p,
-                       0, VarlenArgs{v.cu_seqlens_q, v.cu_seqlens_kv, v.tiles});
+                       0, VarlenArgs{v.cu_seqlens_q, v.cu_seqlens_kv, v.tiles},
+                       SplitArgs{1, 1, nullptr, nullptr});
     return CheckLaunch("flash_fwd_wide_kernel (varlen)", s);
 }
-
-#define SCA_INSTANTIATE_VARLEN(E, D)                                                      \
-    template int LaunchFlashVarlen<E, D, false>(const sca_flash_varlen_params&, hipStream_t); \
-    template int LaunchFlashVarlen<E, D, true>(const sca_flash_varlen_params&, hipStream_t);
-#define SCA_INSTANTIATE(E, D)                                                   \
-    template int LaunchFlashWide<E, D, false>(const sca_flash_params&, hipStream_t); \
-    template int LaunchFlashWide<E, D, true>(const sca_flash_params&, hipStream_t);
-#define SCA_INSTANTIATE_DIMS(E)                                                    \
-    SCA_INSTANTIATE(E, 32) SCA_INSTANTIATE(E, 64) SCA_INSTANTIATE(E, 96)              \
-    SCA_INSTANTIATE(E, 128) SCA_INSTANTIATE(E, 160) SCA_INSTANTIATE_VARLEN(E, 64)        \
-    SCA_INSTANTIATE_VARLEN(E, 128)
-SCA_INSTANTIATE_DIMS(F16)
-SCA_INSTANTIATE_DIMS(BF16)
 
 }  // namespace sca_hip

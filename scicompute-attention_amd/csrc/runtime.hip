@@ -234,6 +234,23 @@ int sca_hip_stream_synchronize(void* stream) {
                    "hipStreamSynchronize");
 }
 
+int sca_hip_stream_is_capturing(void* stream, int* capturing) {
+    if (capturing == nullptr) {
+        return SetError(SCA_E_SHAPE_MISMATCH, "sca_hip_stream_is_capturing: null");
+    }
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    const int rc = FromHip(hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status),
+                           "hipStreamIsCapturing");
+    *capturing = status != hipStreamCaptureStatusNone ? 1 : 0;
+    return rc;
+}
+
+int sca_hip_stream_wait_event(void* stream, void* event) {
+    return FromHip(hipStreamWaitEvent(static_cast<hipStream_t>(stream),
+                                      static_cast<hipEvent_t>(event), 0),
+                   "hipStreamWaitEvent");
+}
+
 int sca_hip_event_create(void** event) {
     if (event == nullptr) return SetError(SCA_E_SHAPE_MISMATCH, "sca_hip_event_create: null");
     hipEvent_t e = nullptr;

@@ -140,8 +140,15 @@ public:
         p.causal = cfg.causal ? 1 : 0;
         p.dtype = runtime::KernelDtype(q.dtype());
         p.diagonal = cfg.causal ? shape.seq_kv - shape.seq_q : 0;
-        status = runtime::StatusFromHip(sca_hip_flash_fwd(&p, runtime::StreamHandle(cfg.stream)),
-                                        "flash forward");
+        void* stream = runtime::StreamHandle(cfg.stream);
+        {
+            // Partial states of a run that splits the keys (no score scratch; none for most calls).
+            const int64_t split_bytes = sca_hip_flash_split_bytes(&p);
+            const runtime::StreamScratch scratch(static_cast<size_t>(split_bytes), device.id(), stream);
+            status = runtime::StatusFromHip(
+                sca_hip_flash_fwd_split(&p, scratch.ptr, scratch.ptr != nullptr ? split_bytes : 0, stream),
+                "flash forward");
+        }
         if (!status.ok()) return sci::MakeUnexpected<AttentionResult>(status);
 
         const TileConfig tile = RecommendTile(cfg, shape);

@@ -4,6 +4,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <string>
 
 #include "core/status.hpp"
@@ -58,6 +59,25 @@ size_t ScratchHighWaterMarkBytes();
 // staging that is reused once the previous copy has completed; returns the device pointer.
 sci::Result<void*> UploadToScratch(ScratchKind kind, const void* host, size_t bytes,
                                    int device_id, void* stream);
+
+// Scratch of one launch sequence on `stream`, safe with any number of threads and streams: at most
+// four buffers per device (64 MiB each), one per stream where possible; a buffer that changes streams
+// waits for the event recorded after its last use, and the lease excludes other threads until its
+// launches are queued. `ptr` is null when there is none to be had (allocation failure, a request above
+// the bound, a stream being captured into a graph): the caller then runs without scratch.
+class StreamScratch {
+public:
+    StreamScratch(size_t bytes, int device_id, void* stream);
+    ~StreamScratch();  // records the event behind the launches queued meanwhile
+    StreamScratch(const StreamScratch&) = delete;
+    StreamScratch& operator=(const StreamScratch&) = delete;
+    void* ptr{nullptr};
+
+private:
+    std::unique_lock<std::mutex> lock_;
+    void* slot_{nullptr};
+    void* stream_{nullptr};
+};
 
 }  // namespace runtime
 }  // namespace sca

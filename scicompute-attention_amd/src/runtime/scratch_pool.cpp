@@ -1,4 +1,5 @@
-// Split-K partial scratch: one FP32 buffer per (device, kind), reused across calls.
+// Split-K partial scratch: one FP32 buffer per (device, kind), reused across calls; and the flash
+// key-split scratch, one buffer per stream (StreamScratch).
 // Growth rule as in the reference's src/runtime/scratch_pool.cpp:38-60 (x1.25 + 1024 elements).
 
 #include <algorithm>
@@ -6,6 +7,7 @@
 #include <map>
 #include <mutex>
 #include <utility>
+#include <vector>
 
 #include "device/device.hpp"
 #include "runtime/internal.hpp"
@@ -67,7 +69,96 @@ sci::Result<float*> AcquireScratchFp32(ScratchKind kind, size_t elements, int de
     return sci::Ok(static_cast<float*>(entry.ptr));
 }
 
+namespace {
+
+constexpr size_t kMaxStreamSlots = 4;
+constexpr size_t kMaxStreamScratchBytes = size_t{64} << 20;
+
+struct StreamSlot {
+    int device_id{0};
+    void* stream{nullptr};  // of the last use
+    void* ptr{nullptr};
+    size_t bytes{0};
+    void* event{nullptr};   // recorded after the last use
+    uint64_t used{0};       // order of last uses
+};
+
+std::mutex& StreamMutex() {
+    static std::mutex mu;
+    return mu;
+}
+
+std::vector<StreamSlot*>& StreamSlots() {  // leaked on purpose, like the scratch pool
+    static auto* slots = new std::vector<StreamSlot*>();
+    return *slots;
+}
+
+void FreeSlotBuffer(StreamSlot* slot) {
+    if (slot->ptr == nullptr) return;
+    if (slot->event != nullptr) sca_hip_event_synchronize(slot->event);
+    sci::GpuDevice(slot->device_id).deallocate(slot->ptr);
+    slot->ptr = nullptr;
+    slot->bytes = 0;
+}
+
+}  // namespace
+
+StreamScratch::StreamScratch(size_t bytes, int device_id, void* stream) : stream_(stream) {
+    if (bytes == 0 || bytes > kMaxStreamScratchBytes) return;
+    int capturing = 0;
+    // A graph would keep the buffer's address beyond this lease.
+    if (sca_hip_stream_is_capturing(stream, &capturing) != 0 || capturing != 0) return;
+    static uint64_t uses = 0;  // guarded by the mutex
+    lock_ = std::unique_lock<std::mutex>(StreamMutex());
+    StreamSlot* slot = nullptr;
+    StreamSlot* oldest = nullptr;
+    size_t on_device = 0;
+    for (StreamSlot* s : StreamSlots()) {
+        if (s->device_id != device_id) continue;
+        ++on_device;
+        if (s->stream == stream && s->used != 0) slot = s;
+        if (oldest == nullptr || s->used < oldest->used) oldest = s;
+    }
+    if (slot == nullptr && on_device < kMaxStreamSlots) {
+        slot = new StreamSlot();
+        slot->device_id = device_id;
+        if (sca_hip_event_create(&slot->event) != 0) {
+            delete slot;
+            return;
+        }
+        StreamSlots().push_back(slot);
+    }
+    if (slot == nullptr) slot = oldest;
+    if (slot->used != 0 && slot->stream != stream &&
+        sca_hip_stream_wait_event(stream, slot->event) != 0) {
+        return;
+    }
+    if (slot->bytes < bytes) {
+        FreeSlotBuffer(slot);
+        size_t want = size_t{1} << 20;
+        while (want < bytes) want *= 2;
+        slot->ptr = sci::GpuDevice(device_id).allocate(want);
+        if (slot->ptr == nullptr) return;
+        slot->bytes = want;
+        std::lock_guard<std::mutex> pool(PoolMutex());
+        g_high_water_bytes = std::max(g_high_water_bytes, want);
+    }
+    slot->stream = stream;
+    slot->used = ++uses;
+    slot_ = slot;
+    ptr = slot->ptr;
+}
+
+StreamScratch::~StreamScratch() {
+    if (slot_ == nullptr) return;
+    sca_hip_event_record(static_cast<StreamSlot*>(slot_)->event, stream_);
+}
+
 sci::Status ReleaseScratch() {
+    {
+        std::lock_guard<std::mutex> streams(StreamMutex());
+        for (StreamSlot* slot : StreamSlots()) FreeSlotBuffer(slot);
+    }
     std::lock_guard<std::mutex> lock(PoolMutex());
     for (auto& kv : Pool()) {
         if (kv.second.ptr != nullptr) {

@@ -347,3 +347,58 @@ def test_split_dims_kernel(hip, D, causal):
     out, _ = run_flash(qb, kb, vb, "bf16", causal, B=1, Hq=2, Hkv=2, Sq=sq, Skv=skv, D=D)
     ref, _ = orc.reference_attention(qd, kd, vd, causal)
     check_attention(out.reshape(-1, D), ref, "bf16", f"growing maxima D={D}")
+
+
+def _split_params(bufs, dtype, causal, B, Hq, Hkv, Sq, Skv, D):
+    p = H.FlashParams()
+    p.q, p.k, p.v, p.out, p.lse = (b.ptr for b in bufs)
+    p.batch, p.num_heads, p.num_kv_heads = B, Hq, Hkv
+    p.seq_q, p.seq_kv, p.head_dim = Sq, Skv, D
+    p.q_sb, p.q_sh, p.q_ss = Hq * Sq * D, Sq * D, D
+    p.k_sb, p.k_sh, p.k_ss = Hkv * Skv * D, Skv * D, D
+    p.v_sb, p.v_sh, p.v_ss = p.k_sb, p.k_sh, p.k_ss
+    p.o_sb, p.o_sh, p.o_ss = Sq * Hq * D, D, Hq * D  # token-major output
+    p.scale = float(np.float32(1.0 / np.sqrt(D)))
+    p.causal, p.dtype, p.diagonal = int(causal), DTYPE_ID[dtype], (Skv - Sq) if causal else 0
+    return p
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal", [
+    (1, 8, 2, 6, 4102, 128, True),     # packed groups of 4, many splits
+    (2, 7, 1, 5, 2900, 64, True),      # a group that does not divide the row tile
+    (1, 4, 4, 1, 3000, 128, False),    # one row, no group
+    (1, 8, 8, 130, 2600, 128, True),   # two row tiles, the second nearly empty
+    (1, 6, 2, 43, 1111, 256, True),    # split-dims kernel: packed 129 rows, ragged last split
+    (2, 4, 2, 2, 2048, 192, False),
+    (1, 8, 2, 33, 1700, 96, True),
+    (1, 4, 1, 100, 1030, 160, True),
+    (1, 4, 2, 1100, 2900, 32, True),   # the early row tiles leave the last splits without keys
+])
+def test_key_splits_and_packed_groups(hip, B, Hq, Hkv, Sq, Skv, D, causal):
+    """The same call with scratch (key ranges in workgroups of their own, merged) and without, both
+    against the oracle, output and LSE; the scratch holds NaN before, so a state that was not written
+    would show."""
+    for dtype in ("bf16", "f16"):
+        qb, qd = quantize(uniform((B, Hq, Sq, D), 96001 + D), dtype)
+        kb, kd = quantize(uniform((B, Hkv, Skv, D), 96002 + D), dtype)
+        vb, vd = quantize(uniform((B, Hkv, Skv, D), 96003 + D), dtype)
+        ref, ref_lse = orc.reference_attention(qd, kd, vd, causal)
+        ref = ref.reshape(B, Hq, Sq, D)
+        inputs = [H.DeviceBuffer.from_array(x) for x in (qb, kb, vb)]
+        want = hip.sca_hip_flash_split_bytes
+        want.restype = H.c_i64
+        for scratch in (True, False):
+            out = H.DeviceBuffer.from_array(np.full(B * Hq * Sq * D, 0x7fff, np.uint16))
+            lse = H.DeviceBuffer.from_array(np.full(B * Hq * Sq, np.nan, np.float32))
+            p = _split_params([*inputs, out, lse], dtype, causal, B, Hq, Hkv, Sq, Skv, D)
+            n = want(H.ctypes.byref(p)) if scratch else 0
+            assert n > 0 or not scratch, "these shapes leave most of the GPU idle unsplit"
+            buf = H.DeviceBuffer.from_array(np.full(max(n // 4, 1), np.nan, np.float32))
+            tag = f"B={B} Hq={Hq} Hkv={Hkv} Sq={Sq} Skv={Skv} D={D} {dtype} scratch={n}"
+            print(tag, flush=True)
+            H.check(hip.sca_hip_flash_fwd_split(H.ctypes.byref(p), H.c_vp(buf.ptr), H.c_i64(n), None))
+            sca_amd.synchronize()
+            got = to_float(out.download(np.uint16), dtype).reshape(B, Sq, Hq, D).transpose(0, 2, 1, 3)
+            check_attention(got.reshape(-1, D), ref.reshape(-1, D), dtype, tag, abs_gate=True)
+            err = np.max(np.abs(lse.download(np.float32).astype(np.float64) - ref_lse.reshape(-1)))
+            assert err <= 1e-2, f"{tag}: LSE err {err}"
