@@ -11,12 +11,12 @@
 // m in natural-log units.
 //
 // MI355X design (HBM-bound kernels):
-//   * fp16/bf16 with head_dim 64 or 128 (power-of-two page sizes when paged) run
-//     decode_mfma_kernel: the query heads of a GQA group are the 16 columns of
+//   * fp16/bf16 (power-of-two page sizes when paged; small groups at other head dims than 64 and
+//     128 excepted, see LaunchForDim) run decode_mfma_kernel: the query heads of a GQA group are the 16 columns of
 //     v_mfma_f32_16x16x32 tiles, K goes straight into A-operand registers, V through a small LDS
 //     ring read with transposed loads; ragged batches run longest sequence first. Described at
 //     its definition;
-//   * every other shape (fp32, other head dims) runs decode_partial_kernel: one workgroup per
+//   * every other shape (fp32, odd page sizes) runs decode_partial_kernel: one workgroup per
 //     (b, kv head, split) streams its K/V chunk exactly once and serves kHeads query heads of the
 //     group from registers; a lane owns 16 B of one token row (8 fp16/bf16 elements), QK uses
 //     v_dot2_f32_{f16,bf16} and a DPP row sum, the online softmax is updated once per chunk of
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(const s
 
 constexpr int kRankBatch = 256;  // ragged batches up to this size are ranked in the kernel
 
-// ---- MFMA partial kernel (fp16/bf16, head_dim 64 or 128, power-of-two pages) -----------------
+// ---- MFMA partial kernel (fp16/bf16, power-of-two pages) ---------------------------------------
 // One workgroup per (b, kv head, 16-head chunk of its q group, split); four waves take the
 // 32-token tiles of the split in turn and are merged through LDS at the end.
 //   S^T[32 tokens x 16 heads] = K . Q^T on v_mfma_f32_16x16x32 (two 16-token row tiles; the
@@ -505,24 +505,29 @@ struct DecMfma<DecBF16> {
 
 template <int D>
 struct MfmaDecGeom {
-    static_assert(D == 64 || D == 128, "MFMA decode covers head_dim 64 and 128");
+    static_assert(D % 32 == 0 && D <= 256, "MFMA decode covers multiples of 32");
+    // Head dims other than 64 and 128 keep the precision of the fp32 probabilities that they had on
+    // the VALU: P = hi + lo, two values of the input type and two PV MFMAs. The K/V stream hides them.
+    static constexpr bool SPLIT_P = D != 64 && D != 128;
     static constexpr int NK = D / 32;                    // QK k steps
     static constexpr int ND = D / 16;                    // PV output tiles
     static constexpr int RB = 2 * D;                     // row bytes
     static constexpr int CPR = D / 8;                    // 16-byte chunks per row
     static constexpr int TILE_BYTES = kMfmaTile * RB;    // one V tile of one wave
     static constexpr int DMA = TILE_BYTES / 1024;        // DMA instructions per V tile
-    static constexpr int ROWS_PER_DMA = 64 / CPR;
     static constexpr int SLOT_BYTES = kDecodeWaves * TILE_BYTES;  // one LDS object
     static constexpr int LOADS = DMA + 2 * NK;           // vector memory instructions per tile
     static_assert(kDecodeWaves * kMfmaHeads * D * 4 <= SLOT_BYTES, "merge buffer fits one slot");
 };
 
-// 32-byte segment swizzle of V row t (rows t and t + 16 share it, which the two transposed
-// reads of a lane rely on).
+// 32-byte segment swizzle of V row t, so that the 8 rows one half of a transposed read touches land on
+// distinct segments of the 256-byte bank window: a row is D/16 segments, so rows of 0 mod 8 segments
+// all start alike, of 4 mod 8 every other one, and of 2 or 6 mod 8 every fourth. (Rows t and t + 16
+// share it, which the two transposed reads of a lane rely on.)
 template <int D>
 __device__ __forceinline__ int VSwz(int t) {
-    return D == 128 ? (t & 7) : ((t >> 1) & 3);
+    constexpr int kStart = (D / 16) % 8;
+    return kStart == 0 ? (t & 7) : kStart == 4 ? ((t >> 1) & 3) : ((t >> 2) & 1);
 }
 
 // kWaveHeads: each wave owns one (kv head, head chunk) slot and all tiles of the split (the
@@ -626,10 +631,8 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
     const int64_t k_row_bytes = p.k_ss * 2;
     const int64_t v_row_bytes = p.v_ss * 2;
 
-    // Per-lane constants: DMA row/chunk within one instruction and the V transposed read
-    // (row 4*grp + col/4, byte 8*(col%4) of a 32-byte segment).
-    const int dma_row = lane / G::CPR;
-    const int dma_pc = lane % G::CPR;
+    // Per-lane constants of the V transposed read (row 4*grp + col/4, byte 8*(col%4) of a 32-byte
+    // segment).
     const int wave_off = wave * G::TILE_BYTES;
     const int tr_row = 4 * grp + col / 4;
     const int tr_rd = wave_off + tr_row * G::RB + 8 * (col % 4);
@@ -682,10 +685,11 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
             const int64_t base = seg + static_cast<int64_t>(tile) * kMfmaTile;
 #pragma unroll
             for (int i = 0; i < G::DMA; ++i) {
-                const int t = i * G::ROWS_PER_DMA + dma_row;
+                const int t = (i * kWave + lane) / G::CPR;  // row and 16-byte chunk of the tile
+                const int pc = (i * kWave + lane) % G::CPR;
                 int64_t r = row_of(base + t);
                 r = r < 0 ? safe_row : r;
-                const int vc = (((dma_pc >> 1) ^ VSwz<D>(t)) << 1) | (dma_pc & 1);
+                const int vc = (((pc >> 1) ^ VSwz<D>(t)) << 1) | (pc & 1);
                 __builtin_amdgcn_global_load_lds(
                     v_base + r * v_row_bytes + vc * 16,
                     (__attribute__((address_space(3))) void*)(vdst + wave_off + i * 1024), 16, 0, 0);
@@ -751,6 +755,20 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
             const vec8 pb = __builtin_bit_cast(
                 vec8, make_uint4(M::pack(pr[0][0], pr[0][1]), M::pack(pr[0][2], pr[0][3]),
                                  M::pack(pr[1][0], pr[1][1]), M::pack(pr[1][2], pr[1][3])));
+            vec8 pb_lo;  // what the rounding of pb lost
+            if constexpr (G::SPLIT_P) {
+                float res[2][4];
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        res[rt][i] = pr[rt][i] - static_cast<float>(pb[4 * rt + i]);
+                    }
+                }
+                pb_lo = __builtin_bit_cast(
+                    vec8, make_uint4(M::pack(res[0][0], res[0][1]), M::pack(res[0][2], res[0][3]),
+                                     M::pack(res[1][0], res[1][1]), M::pack(res[1][2], res[1][3])));
+            }
             if (valid_mask != 0xffffffffu) {
                 // Clear the V rows of masked tokens: their probabilities are zero, but the rows
                 // may hold any bit pattern.
@@ -769,8 +787,9 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
                 const uint8_t* a = vs + tr_rd + ((dt * 32) ^ tr_x);
                 const uint2 lo = M::Tr::read(a);
                 const uint2 hi = M::Tr::read(a + 16 * G::RB);
-                o[dt] = M::mma(__builtin_bit_cast(vec8, make_uint4(lo.x, lo.y, hi.x, hi.y)), pb,
-                               o[dt]);
+                const vec8 vt = __builtin_bit_cast(vec8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+                o[dt] = M::mma(vt, pb, o[dt]);
+                if constexpr (G::SPLIT_P) o[dt] = M::mma(vt, pb_lo, o[dt]);
             }
         };
 
@@ -908,11 +927,12 @@ __global__ __launch_bounds__(256) void decode_order_kernel(const int32_t* seq_le
 }
 
 // One wave per head slot (true) or four waves per slot (false): the caller's slot_waves when
-// set, else one wave per slot for paged KV and four for contiguous KV.
-bool MfmaWaveHeads(bool paged, int32_t slot_waves) {
+// set, else one wave per slot for paged KV at head_dim 64 and 128, whose default split counts are
+// made for it, and four otherwise (a workgroup per slot, as the other split rules count).
+bool MfmaWaveHeads(bool paged, int64_t head_dim, int32_t slot_waves) {
     if (slot_waves == 1) return true;
     if (slot_waves == kDecodeWaves) return false;
-    return paged;
+    return paged && (head_dim == 64 || head_dim == 128);
 }
 
 template <typename E, int D, bool kPaged>
@@ -923,9 +943,18 @@ int LaunchForDim(const sca_decode_params& p, hipStream_t s) {
     if constexpr (kPaged) {
         while ((int64_t{1} << block_shift) < p.block_size) ++block_shift;
     }
-    const bool mfma_ok = !std::is_same_v<E, DecF32> && (D == 64 || D == 128) &&
+    // Contiguous KV with one query head per KV head, or two from head_dim 160 on, stays on the VALU
+    // kernel: with so little reuse it is as fast, and for D >= 160 four of its workgroups share a CU
+    // where the MFMA kernel's rings allow one (bf16: D 96, 16 x 32/32 x 2000 68.5 us against 69.5;
+    // D 256, 16 x 16/16 x 4096 176 against 180, 4 x 16/8 x 8192 54 against 60 at the same 16 splits).
+    // Larger groups and paged KV gain from 1% to 5.6x (64 x 64/8 x 4096, D 192: 536 -> 271 us;
+    // 128 x 28/4 x 2000, D 32: 127 -> 23; 64 x 512..16384 paged, D 256: 1,377 -> 689).
+    // Paged D 256 with one head per KV head too (4 x 4000..9000, 16 heads: 76 us against 81 at its best).
+    const bool valu_group = kPaged ? D == 256 && group == 1
+                                   : D != 64 && D != 128 && (group == 1 || (group == 2 && D >= 160));
+    const bool mfma_ok = !std::is_same_v<E, DecF32> && !valu_group &&
                          (!kPaged || (int64_t{1} << block_shift) == p.block_size);
-    if constexpr (!std::is_same_v<E, DecF32> && (D == 64 || D == 128)) {
+    if constexpr (!std::is_same_v<E, DecF32>) {
         if (mfma_ok) {
             sca_decode_params q = p;
             if (q.seq_lens == nullptr || q.batch <= kRankBatch || q.batch > kMaxOrderedBatch) {
@@ -940,7 +969,7 @@ int LaunchForDim(const sca_decode_params& p, hipStream_t s) {
             }
             const int h_chunks = static_cast<int>((group + kMfmaHeads - 1) / kMfmaHeads);
             const int64_t slots = p.num_kv_heads * h_chunks;
-            if (MfmaWaveHeads(kPaged, p.slot_waves)) {
+            if (MfmaWaveHeads(kPaged, D, p.slot_waves)) {
                 const dim3 grid(static_cast<unsigned>(p.num_splits),
                                 static_cast<unsigned>((slots + kDecodeWaves - 1) / kDecodeWaves),
                                 static_cast<unsigned>(p.batch));

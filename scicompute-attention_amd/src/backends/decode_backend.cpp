@@ -26,11 +26,11 @@ int64_t PartialElements(int64_t batch, int64_t heads, int64_t splits, int64_t he
 
 // Explicit split counts are honoured up to the table's cap; otherwise the table decides.
 int64_t ResolveSplits(int64_t requested, int64_t batch, int64_t num_heads, int64_t num_kv_heads,
-                      int64_t seq_kv, int64_t head_dim, int slot_waves = 4) {
+                      int64_t seq_kv, int64_t head_dim, int slot_waves = 4, bool half = false) {
     const auto& th = detail::kDispatchThresholds;
     if (requested > 0) return requested < th.max_splits ? requested : th.max_splits;
     return detail::DecodeSplits(batch, num_heads, num_kv_heads, seq_kv,
-                                DeviceCapability::ForDevice(0).sm_count, slot_waves, head_dim);
+                                DeviceCapability::ForDevice(0).sm_count, slot_waves, head_dim, half);
 }
 
 // Points the partial pointers of `p` into the pooled FP32 scratch (m | l | O).
@@ -130,7 +130,8 @@ public:
             return fail(AttnStatusCode::kUnsupportedFeature, "decode backend: no GPU device");
         }
         const int64_t splits = ResolveSplits(cfg.num_splits, shape.batch, shape.num_heads,
-                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim);
+                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim,
+                                             /*slot_waves=*/4, q.dtype() != sci::DType::kFloat32);
 
         AttentionResult result;
         result.out = sci::Tensor(sci::TensorShape({shape.batch, shape.num_heads, shape.seq_q,
@@ -322,20 +323,21 @@ sci::Result<AttentionResult> RunPaged(const sci::Tensor& q, const PagedKVCache& 
                       head_dim, /*slot_waves=*/1);
     int32_t slot_waves = 0;
     // With the cache's own page table, its host-side lengths say how ragged the batch is; the
-    // MFMA kernel (fp16/bf16, head_dim 64 or 128, power-of-two pages) then takes the split count
+    // MFMA kernel (fp16/bf16, power-of-two pages) then takes the split count
     // and slot work split of the length-aware plan. Lengths the caller passes in
     // params.seq_lens (device memory) do not feed the plan: the kernel reads them, so results
     // follow them exactly, while the plan is fitted to the cache's host lengths (which a decode
     // loop passing its own lengths, with this step's token, tracks to within a token).
+    // (One query head per KV head at head_dim 256 runs the VALU kernel, with its own split rule.)
     const bool mfma_shape = kv_cfg.dtype != sci::DType::kFloat32 &&
-                            (head_dim == 64 || head_dim == 128) &&
+                            !(head_dim == 256 && num_heads == kv_cfg.num_kv_heads) &&
                             (block_size & (block_size - 1)) == 0;
     if (cfg.num_splits <= 0 && params.page_table == nullptr && mfma_shape) {
         std::vector<int64_t> lengths(static_cast<size_t>(num_seqs));
         for (int64_t b = 0; b < num_seqs; ++b) lengths[static_cast<size_t>(b)] = kv.SeqLength(b);
-        const auto plan = detail::PagedDecodePlan(lengths.data(), num_seqs, num_heads,
-                                                  kv_cfg.num_kv_heads,
-                                                  DeviceCapability::ForDevice(0).sm_count);
+        const auto plan = detail::PagedDecodePlanFor(head_dim, lengths.data(), num_seqs, num_heads,
+                                                     kv_cfg.num_kv_heads,
+                                                     DeviceCapability::ForDevice(0).sm_count);
         if (plan.slot_waves != 0) {
             splits = plan.splits;
             slot_waves = plan.slot_waves;

@@ -44,16 +44,21 @@ inline constexpr DispatchThresholds kDispatchThresholds{
 //    8 splits, 5.95 against 5.47 at 64; 4 x 16384: 8, 5.84 against 5.66 at 32; 1 x 65536: 32,
 //    5.60 against 5.22 at 64).
 //  - One wave per slot: splits are added until every CU holds `workgroups_per_cu` workgroups.
-//  - head_dim outside {64, 128} (the VALU kernel, a workgroup per (sequence, split, 1-8 heads)):
-//    unsplit once the batch gives every CU a workgroup, else splits until every CU holds four,
-//    with no cap at 8 (fp16, H_q 32, H_kv 8, D 96: 4 x 16384 keys 32 splits, 4.34 TB/s against
-//    3.37 at 8; 16 x 4096 8 splits, 4.63, the best of 1..32; 64 x 4096 unsplit 5.05 against
-//    5.10 at 4). fp32 with D 64 or 128 runs the VALU kernel under the MFMA rule (16 x 4096,
-//    D 128: 5.21 TB/s at 8 splits against 5.52 at 4).
+//  - head_dim outside {64, 128}: unsplit once the batch gives every CU a workgroup, else splits
+//    until every CU holds four, with no cap at 8 (made for the VALU kernel, a workgroup per
+//    (sequence, split, 1-8 heads): fp16, H_q 32, H_kv 8, D 96: 4 x 16384 keys 32 splits, 4.34 TB/s
+//    against 3.37 at 8; 16 x 4096 8 splits, 4.63, the best of 1..32; 64 x 4096 unsplit 5.05 against
+//    5.10 at 4; the MFMA kernel at D 96 and 32 is within 6% of its best there: 16 x 4096 4.80 TB/s
+//    against 4.88 at 4). fp32 with D 64 or 128 runs the VALU kernel under the MFMA rule (16 x 4096,
+//    D 128: 5.21 TB/s at 8 splits against 5.52 at 4);
+//  - 16-bit types (`half`) with head_dim >= 160 and groups above 2, where the MFMA kernel's rings
+//    leave room for one workgroup per CU: one workgroup per CU (bf16, H_q 32, H_kv 8: D 192, 16 x
+//    4096 2 splits 5.23 TB/s against 4.45 at 8; D 160, 4 x 8192 8 splits 4.77 against 4.10 at 16;
+//    D 256, 2 x 16384 16 splits 4.82 against 4.25 at 32).
 // Each split keeps at least `min_tokens_per_split` keys.
 inline int64_t DecodeSplits(int64_t batch, int64_t num_heads, int64_t num_kv_heads,
                             int64_t seq_kv, int64_t cu_count, int slot_waves = 4,
-                            int64_t head_dim = 128) {
+                            int64_t head_dim = 128, bool half = false) {
     const auto& th = kDispatchThresholds;
     if (batch < 1 || num_kv_heads < 1 || seq_kv < 1) return 1;
     const int64_t group = num_heads / num_kv_heads;
@@ -63,7 +68,8 @@ inline int64_t DecodeSplits(int64_t batch, int64_t num_heads, int64_t num_kv_hea
     const bool mfma = head_dim == 64 || head_dim == 128;
     if (!mfma) {
         const int64_t jobs = batch * slots;
-        splits = jobs >= cus ? 1 : (4 * cus + jobs - 1) / jobs;
+        const bool one_per_cu = half && head_dim >= 160 && group > 2;
+        splits = jobs >= cus ? 1 : one_per_cu ? cus / jobs : (4 * cus + jobs - 1) / jobs;
     } else if (slot_waves == 1) {
         const int64_t wgs_per_split = batch * ((slots + 3) / 4);
         splits = (th.workgroups_per_cu * cus + wgs_per_split - 1) / wgs_per_split;
@@ -135,6 +141,37 @@ inline PagedDecodePlanResult PagedDecodePlan(const int64_t* lengths, int64_t bat
     if (splits > by_length) splits = by_length;
     if (splits > th.max_splits) splits = th.max_splits;
     return {splits < 1 ? 1 : splits, slot_waves};
+}
+
+// What the paged backend runs: the plan above, except
+//  - one wave per slot that would leave half the CUs without a workgroup (few sequences, splits at
+//    their minimum length) becomes four waves per slot at the same splits: four times the
+//    workgroups, each with a quarter of the tiles per wave;
+//  - head_dim >= 160, where the kernel's rings leave room for one workgroup per CU: four waves per
+//    slot, unsplit from two slots per CU on, two workgroups per CU down to half a slot per CU and one
+//    below (bf16, H_kv 8: D 256, 16 x 512..16384 4 splits 5.52 TB/s against 5.00 at 12; D 160, 128 x
+//    128..4000 1 split 5.01 against 2.95 at 6; D 256, 4 x 4000..9000 x 16 heads 4 splits 4.73 against
+//    3.95 at 12).
+inline PagedDecodePlanResult PagedDecodePlanFor(int64_t head_dim, const int64_t* lengths,
+                                                int64_t batch, int64_t num_heads,
+                                                int64_t num_kv_heads, int64_t cu_count) {
+    PagedDecodePlanResult plan = PagedDecodePlan(lengths, batch, num_heads, num_kv_heads, cu_count);
+    if (plan.slot_waves == 0) return plan;
+    const int64_t slots = num_kv_heads * ((num_heads / num_kv_heads + 15) / 16);
+    const int64_t jobs = batch * slots;
+    const int64_t cus = cu_count > 0 ? cu_count : 256;
+    if (head_dim >= 160) {
+        const auto& th = kDispatchThresholds;
+        int64_t longest = 0;
+        for (int64_t b = 0; b < batch; ++b) longest = lengths[b] > longest ? lengths[b] : longest;
+        const int64_t by_length = (longest + th.min_tokens_per_split - 1) / th.min_tokens_per_split;
+        int64_t splits = jobs >= 2 * cus ? 1 : 2 * jobs >= cus ? 2 * cus / jobs : cus / jobs;
+        splits = splits < by_length ? splits : by_length;
+        splits = splits < th.max_splits ? splits : th.max_splits;
+        return {splits < 1 ? 1 : splits, 4};
+    }
+    if (plan.slot_waves == 1 && 2 * plan.splits * batch * ((slots + 3) / 4) <= cus) plan.slot_waves = 4;
+    return plan;
 }
 
 }  // namespace detail

@@ -137,3 +137,30 @@ def test_contiguous_slot_layouts(hip, slot_waves):
     _case("bf16", 2, 8, 8, 700, 64, 1, 76002, slot_waves=slot_waves)
     _case("f16", 4, 8, 2, 600, 128, 16, 76003, seq_lens=[600, 3, 1, 257], slot_waves=slot_waves)
     _case("bf16", 1, 32, 1, 900, 128, 2, 76004, slot_waves=slot_waves)
+
+
+@pytest.mark.parametrize("d", [32, 96, 160, 192, 256])
+@pytest.mark.parametrize("group", [1, 2, 3, 8, 20])
+def test_other_head_dims_across_groups(hip, d, group):
+    """Both kernels that serve these head dims (small groups the VALU one), odd lengths around the 32-token
+    tile, ragged batches, both work splits of the MFMA kernel."""
+    for i, (skv, splits, waves) in enumerate([(1, 1, 0), (33, 2, 4), (127, 1, 1), (1000, 5, 0)]):
+        _case("bf16" if i % 2 else "f16", 2, 2 * group, 2, skv, d, splits, 83000 + d + skv + group,
+              slot_waves=waves)
+    _case("f16", 3, group, 1, 500, d, 4, 84000 + d + group, seq_lens=[500, 2, 130])
+
+
+def test_decode_splits_follow_the_kernel(hip):
+    """Host decode at head_dim >= 160: one workgroup per CU where the MFMA kernel runs (16-bit types,
+    groups above 2), the VALU kernel's count otherwise; outputs as ever."""
+    from sca_amd import host
+    for dtype, hq, want in [("bf16", 8, 16), ("bf16", 4, 16), ("f32", 8, 16)]:
+        q, k, v = uniform((2, hq, 1, 192), 1), uniform((2, 2, 8192, 192), 2), uniform((2, 2, 8192, 192), 3)
+        enc = [quantize(x, dtype) if dtype != "f32" else (x.astype(np.float32), x) for x in (q, k, v)]
+        t = [host.Tensor.from_numpy(b, dtype) for b, _ in enc]
+        res = host.decode_attention(*t)
+        assert res.stats["num_splits"] == want, (dtype, hq, res.stats)
+        ref, _ = orc.reference_attention(*[d for _, d in enc], True)
+        out = res.out.numpy()
+        got = orc.decode_bits(out, dtype) if dtype != "f32" else out
+        check_attention(got.reshape(-1, 192), ref, dtype, f"host decode {dtype} hq={hq}")

@@ -265,3 +265,25 @@ def test_splits_spanning_several_page_segments(hip, bs, L, splits, D, dtype, slo
           f"slot_waves={slot_waves}", flush=True)
     _case([L, 3], bs, 8, 2, D, dtype, 87000 + bs + splits + D, splits=splits,
           slot_waves=slot_waves)
+
+
+@pytest.mark.parametrize("D", [32, 96, 160, 192, 256])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_other_head_dims_keep_fp32_weights(hip, D, dtype):
+    """The MFMA kernel at head dims other than 64 and 128 carries the softmax weights as two values of
+    the input type: each output is within the rounding of the output type (unit roundoff u = 2^-11 for
+    fp16, 2^-8 for bf16) plus what two values lose of a weight (u^2, times max |v|, as the weights sum
+    to 1) and the fp32 sums (4e-6). Weights rounded once would be off by up to u * max |v|."""
+    u = 2.0 ** -11 if dtype == "f16" else 2.0 ** -8
+    for Hq, Hkv, bs, waves, splits, lengths in [(8, 2, 16, 4, 3, [1, 31, 33, 700]),
+                                                (14, 2, 32, 1, 2, [64, 129, 5]),
+                                                (17, 1, 8, 4, 5, [400, 17]), (6, 2, 16, 0, 1, [95, 96])]:
+        nb, mb, table, kb, kd, vb, vd = build_pool(lengths, bs, Hkv, D, dtype, 81000 + D + Hq)
+        qb, qd = quantize(2.0 * uniform((len(lengths), Hq, 1, D), 82000 + D), dtype)
+        got = run_paged(qb, kb, vb, table, lengths, dtype, Hq=Hq, Hkv=Hkv, D=D, bs=bs, num_blocks=nb,
+                        splits=splits, slot_waves=waves).reshape(-1, D)
+        ref = reference(qd, kd, vd, table, lengths, bs, nb).reshape(-1, D)
+        print(f"paged {dtype} D={D} Hq={Hq} Hkv={Hkv} bs={bs} waves={waves} splits={splits}", flush=True)
+        limit = 1.01 * u * np.abs(ref) + (4 * u * u + 4e-6) * float(np.max(np.abs(vd)))
+        worst = float(np.max(np.abs(got - ref) / limit))
+        assert worst <= 1.0, f"{worst:.2f} times the bound"
