@@ -185,6 +185,16 @@ __device__ __forceinline__ void MergeWeights(float m_a, float m_b, float* m_out,
     *w_b = (m_b == neg_inf()) ? 0.0f : fast_exp2(m_b - mm);
 }
 
+// Keys per split, ceil(len / splits).
+__device__ __forceinline__ int64_t SplitChunk(int64_t len, int64_t splits) {
+    if (len <= 0) return 0;
+    if (len < (int64_t{1} << 31)) {
+        return (static_cast<uint32_t>(len) + static_cast<uint32_t>(splits) - 1) /
+               static_cast<uint32_t>(splits);
+    }
+    return (len + splits - 1) / splits;
+}
+
 template <typename E, int D, int kHeads, bool kPaged>
 __global__ __launch_bounds__(kDecodeThreads) void decode_partial_kernel(const sca_decode_params p,
                                                                         int h_chunks) {
@@ -207,10 +217,10 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_partial_kernel(const sc
     const bool active = sub < NV;
 
     const int64_t split = blockIdx.x;
-    const int64_t h_kv = blockIdx.y / h_chunks;
-    const int64_t h_chunk = blockIdx.y % h_chunks;
+    const int64_t h_kv = blockIdx.y / static_cast<uint32_t>(h_chunks);
+    const int64_t h_chunk = blockIdx.y % static_cast<uint32_t>(h_chunks);
     const int64_t b = blockIdx.z;
-    const int64_t group = p.num_heads / p.num_kv_heads;
+    const int64_t group = static_cast<uint32_t>(p.num_heads) / static_cast<uint32_t>(p.num_kv_heads);
     const int64_t h0 = h_kv * group + h_chunk * kHeads;  // first q head of this workgroup
 
     const float scale2 = p.scale * kLog2e;
@@ -235,7 +245,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_partial_kernel(const sc
     }
 
     const int64_t len = p.seq_lens != nullptr ? static_cast<int64_t>(p.seq_lens[b]) : p.seq_kv;
-    const int64_t chunk = len > 0 ? (len + p.num_splits - 1) / p.num_splits : 0;
+    const int64_t chunk = SplitChunk(len, p.num_splits);
     const int64_t t_begin = split * chunk;
     const int64_t t_end = (t_begin + chunk < len) ? (t_begin + chunk) : len;
 
@@ -284,9 +294,21 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_partial_kernel(const sc
                 int64_t row = tok;
                 if constexpr (kPaged) {
                     if (ok) {
-                        const int32_t id = s_pages[tok / p.block_size - page0];
+                        // Tokens of a segment in 32 bits where its pages allow (below 2^20 tokens
+                        // each): the 64-bit division per key was what bounded paged fp32.
+                        int64_t page, off;
+                        if (p.block_size < (1 << 20)) {
+                            const uint32_t rel = static_cast<uint32_t>(tok - page0 * p.block_size);
+                            const uint32_t bs = static_cast<uint32_t>(p.block_size);
+                            page = rel / bs;
+                            off = rel - static_cast<uint32_t>(page) * bs;
+                        } else {
+                            page = tok / p.block_size - page0;
+                            off = tok % p.block_size;
+                        }
+                        const int32_t id = s_pages[page];
                         ok = id >= 0;
-                        row = static_cast<int64_t>(id) * p.block_size + tok % p.block_size;
+                        row = static_cast<int64_t>(id) * p.block_size + off;
                     }
                 }
                 valid[c] = ok;
@@ -418,12 +440,15 @@ template <typename E, int D>
 __global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(const sca_decode_params p) {
     constexpr int64_t kElemBytes = 16 / E::VE;
     constexpr int kQuads = D / 4;
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * kCombineThreads + threadIdx.x;
-    const int64_t flat_bh = idx / kQuads;
+    // batch * heads fits 32 bits (each is below 2^16); kQuads is a constant.
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kCombineThreads;
+    const int64_t first_row = first / kQuads;
+    const uint32_t within = static_cast<uint32_t>(first - first_row * kQuads) + threadIdx.x;
+    const int64_t flat_bh = first_row + within / kQuads;
     if (flat_bh >= p.batch * p.num_heads) return;
-    const int d0 = static_cast<int>(idx % kQuads) * 4;
-    const int64_t b = flat_bh / p.num_heads;
-    const int64_t h = flat_bh % p.num_heads;
+    const int d0 = static_cast<int>(within % kQuads) * 4;
+    const int64_t b = static_cast<uint32_t>(flat_bh) / static_cast<uint32_t>(p.num_heads);
+    const int64_t h = static_cast<uint32_t>(flat_bh) % static_cast<uint32_t>(p.num_heads);
     const int ns = static_cast<int>(p.num_splits);
     const float* pm = p.partial_m + flat_bh * ns;
     const float* pl = p.partial_l + flat_bh * ns;
@@ -559,8 +584,11 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
     const int64_t hh = kWaveHeads ? static_cast<int64_t>(blockIdx.y) * kDecodeWaves + wave
                                   : static_cast<int64_t>(blockIdx.y);
     const bool slot_ok = hh < slots;  // false only for trailing waves of a kWaveHeads grid
-    const int64_t h_kv = (slot_ok ? hh : 0) / h_chunks;
-    const int64_t h_chunk = (slot_ok ? hh : 0) % h_chunks;
+    // 32-bit divisions (heads are below 2^16; lengths almost always): a 64-bit one takes about 130
+    // instructions, and four of them cost every workgroup 1 us.
+    const uint32_t slot = slot_ok ? static_cast<uint32_t>(hh) : 0;
+    const int64_t h_kv = slot / static_cast<uint32_t>(h_chunks);
+    const int64_t h_chunk = slot % static_cast<uint32_t>(h_chunks);
     // Sequence of this workgroup. Ragged batches run longest first: grid row z takes the
     // sequence of rank z (descending length, ties by index), ranked here for batches of up to
     // kRankBatch sequences and by decode_order_kernel through batch_order above that.
@@ -593,7 +621,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
     } else if (p.seq_lens != nullptr) {
         len = p.seq_lens[b];
     }
-    const int64_t group = p.num_heads / p.num_kv_heads;
+    const int64_t group = static_cast<uint32_t>(p.num_heads) / static_cast<uint32_t>(p.num_kv_heads);
     const int64_t h0 = h_kv * group + h_chunk * kMfmaHeads;
     const int hc = static_cast<int>(group - h_chunk * kMfmaHeads < kMfmaHeads
                                         ? group - h_chunk * kMfmaHeads
@@ -620,7 +648,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
     float m = neg_inf();  // running max of head `col` (log2 units, identical across lane groups)
     float l = 0.0f;       // this lane's share of the running denominator
 
-    const int64_t chunk = len > 0 ? (len + p.num_splits - 1) / p.num_splits : 0;
+    const int64_t chunk = SplitChunk(len, p.num_splits);
     const int64_t t_begin = split * chunk;
     const int64_t t_end = (t_begin + chunk < len) ? (t_begin + chunk) : len;
 

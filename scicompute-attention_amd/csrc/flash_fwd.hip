@@ -27,19 +27,6 @@
 namespace sca_hip {
 namespace {
 
-int CuCount() {
-    static int cu_count = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-            (void)hipGetLastError();
-            n = 256;
-        }
-        return n > 0 ? n : 256;
-    }();
-    return cu_count;
-}
-
 // Whether the DMA kernels' unsigned 32-bit buffer offsets reach every row (plus the rings' overrun).
 bool DmaReach(const sca_flash_params& p) {
     constexpr int64_t kOverrun = 8 * 64;

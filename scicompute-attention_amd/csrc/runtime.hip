@@ -58,6 +58,19 @@ int FromHip(hipError_t err, const char* what) {
                         hipGetErrorString(err) + ")");
 }
 
+int CuCount() {
+    static int cu_count = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+            (void)hipGetLastError();
+            n = 256;
+        }
+        return n > 0 ? n : 256;
+    }();
+    return cu_count;
+}
+
 int CheckLaunch(const char* what, hipStream_t stream) {
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return FromHip(err, what);

@@ -113,6 +113,7 @@ namespace sca_hip {
 int SetError(int code, const std::string& message);
 int CheckLaunch(const char* what, hipStream_t stream);
 int FromHip(hipError_t err, const char* what);
+int CuCount();  // compute units of the first device used (256 when it cannot be read)
 
 // Raises the dynamic LDS limit of kernel `Kernel` to `bytes` the first time it is launched in
 // the process. Safe to call from several threads; a failed attribute call is reported as an

@@ -29,8 +29,12 @@ int64_t ResolveSplits(int64_t requested, int64_t batch, int64_t num_heads, int64
                       int64_t seq_kv, int64_t head_dim, int slot_waves = 4, bool half = false) {
     const auto& th = detail::kDispatchThresholds;
     if (requested > 0) return requested < th.max_splits ? requested : th.max_splits;
-    return detail::DecodeSplits(batch, num_heads, num_kv_heads, seq_kv,
-                                DeviceCapability::ForDevice(0).sm_count, slot_waves, head_dim, half);
+    const int cus = DeviceCapability::ForDevice(0).sm_count;
+    const int64_t splits = detail::DecodeSplits(batch, num_heads, num_kv_heads, seq_kv, cus,
+                                                slot_waves, head_dim, half);
+    if (slot_waves != 4 || batch < 1 || num_kv_heads < 1 || (half && head_dim < 160)) return splits;
+    const int64_t slots = num_kv_heads * ((num_heads / num_kv_heads + 15) / 16);
+    return detail::FillSplits(splits, batch * slots, seq_kv, cus);
 }
 
 // Points the partial pointers of `p` into the pooled FP32 scratch (m | l | O).
@@ -71,7 +75,8 @@ public:
         CapabilityReport report;
         report.recommended_backend = BackendKind::kDecode;
         const int64_t splits = ResolveSplits(cfg.num_splits, shape.batch, shape.num_heads,
-                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim);
+                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim,
+                                             /*slot_waves=*/4, /*half=*/true);
         report.workspace_bytes = WorkspaceBytes(cfg, shape);
         std::string reason;
         if (!DeviceCapability::GpuAvailable()) {
@@ -98,7 +103,8 @@ public:
 
     size_t WorkspaceBytes(const AttentionConfig& cfg, const AttentionShape& shape) const override {
         const int64_t splits = ResolveSplits(cfg.num_splits, shape.batch, shape.num_heads,
-                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim);
+                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim,
+                                             /*slot_waves=*/4, /*half=*/true);
         if (splits <= 1) return 0;
         return static_cast<size_t>(
                    PartialElements(shape.batch, shape.num_heads, splits, shape.head_dim)) *

@@ -89,6 +89,22 @@ inline int64_t DecodeSplits(int64_t batch, int64_t num_heads, int64_t num_kv_hea
     return splits < 1 ? 1 : splits;
 }
 
+// What the contiguous backend runs for fp32 and for head_dim >= 160: the count above, except that a
+// batch whose workgroups would leave half the CUs idle (few sequences, splits at their minimum length)
+// takes shorter splits, down to 128 keys, until every CU has a workgroup: one CU streams about 60 GB/s,
+// and 500 such keys take it 8 us and more (fp32 D 128, 1 x 3000 30.3 -> 14.8 us, 4 x 16/4 x 2000 29.6 ->
+// 14.8; bf16 D 256, 2 x 1000 34 -> 13). Up to head_dim 128 in 16 bits the two launches bound the call
+// and the longer merge costs 3% (4 x 700, D 128: 12.4 -> 12.8), so the count stays.
+inline int64_t FillSplits(int64_t splits, int64_t jobs, int64_t longest, int64_t cu_count) {
+    const int64_t cus = cu_count > 0 ? cu_count : 256;
+    if (2 * splits * jobs > cus) return splits;
+    int64_t fill = cus / jobs;
+    const int64_t by_length = (longest + 127) / 128;
+    fill = fill < by_length ? fill : by_length;
+    fill = fill < kDispatchThresholds.max_splits ? fill : kDispatchThresholds.max_splits;
+    return fill > splits ? fill : splits;
+}
+
 // Work split of the paged MFMA decode kernel for a batch whose host-side lengths are known.
 // slot_waves = 1: one wave per head slot, a workgroup serves four slots; 4: four waves share one
 // slot's key tiles. Measured on MI355X over 48-step decode loops (bf16, H_q 32, H_kv 8, D 128):
@@ -146,7 +162,8 @@ inline PagedDecodePlanResult PagedDecodePlan(const int64_t* lengths, int64_t bat
 // What the paged backend runs: the plan above, except
 //  - one wave per slot that would leave half the CUs without a workgroup (few sequences, splits at
 //    their minimum length) becomes four waves per slot at the same splits: four times the
-//    workgroups, each with a quarter of the tiles per wave;
+//    workgroups, each with a quarter of the tiles per wave, and shorter splits where that still
+//    leaves CUs idle (FillSplits);
 //  - head_dim >= 160, where the kernel's rings leave room for one workgroup per CU: four waves per
 //    slot, unsplit from two slots per CU on, two workgroups per CU down to half a slot per CU and one
 //    below (bf16, H_kv 8: D 256, 16 x 512..16384 4 splits 5.52 TB/s against 5.00 at 12; D 160, 128 x
@@ -160,17 +177,20 @@ inline PagedDecodePlanResult PagedDecodePlanFor(int64_t head_dim, const int64_t*
     const int64_t slots = num_kv_heads * ((num_heads / num_kv_heads + 15) / 16);
     const int64_t jobs = batch * slots;
     const int64_t cus = cu_count > 0 ? cu_count : 256;
+    int64_t longest = 0;
+    for (int64_t b = 0; b < batch; ++b) longest = lengths[b] > longest ? lengths[b] : longest;
     if (head_dim >= 160) {
         const auto& th = kDispatchThresholds;
-        int64_t longest = 0;
-        for (int64_t b = 0; b < batch; ++b) longest = lengths[b] > longest ? lengths[b] : longest;
         const int64_t by_length = (longest + th.min_tokens_per_split - 1) / th.min_tokens_per_split;
         int64_t splits = jobs >= 2 * cus ? 1 : 2 * jobs >= cus ? 2 * cus / jobs : cus / jobs;
         splits = splits < by_length ? splits : by_length;
         splits = splits < th.max_splits ? splits : th.max_splits;
-        return {splits < 1 ? 1 : splits, 4};
+        return {FillSplits(splits < 1 ? 1 : splits, jobs, longest, cus), 4};
     }
-    if (plan.slot_waves == 1 && 2 * plan.splits * batch * ((slots + 3) / 4) <= cus) plan.slot_waves = 4;
+    if (plan.slot_waves == 1 && 2 * plan.splits * batch * ((slots + 3) / 4) <= cus) {
+        plan.slot_waves = 4;
+        plan.splits = FillSplits(plan.splits, jobs, longest, cus);
+    }
     return plan;
 }
 

@@ -150,17 +150,18 @@ def test_other_head_dims_across_groups(hip, d, group):
     _case("f16", 3, group, 1, 500, d, 4, 84000 + d + group, seq_lens=[500, 2, 130])
 
 
-def test_decode_splits_follow_the_kernel(hip):
-    """Host decode at head_dim >= 160: one workgroup per CU where the MFMA kernel runs (16-bit types,
-    groups above 2), the VALU kernel's count otherwise; outputs as ever."""
+def test_host_decode_splits_fill_the_gpu(hip):
+    """Host decode of few sequences, fp32 or head_dim >= 160: splits down to 128 keys until every CU has
+    a workgroup (at most 64 per slot; 256 CUs); at least 512 keys a split otherwise; outputs as ever."""
     from sca_amd import host
-    for dtype, hq, want in [("bf16", 8, 16), ("bf16", 4, 16), ("f32", 8, 16)]:
-        q, k, v = uniform((2, hq, 1, 192), 1), uniform((2, 2, 8192, 192), 2), uniform((2, 2, 8192, 192), 3)
+    for dtype, hq, seq, d, want in [("bf16", 8, 8192, 192, 64), ("f16", 4, 1000, 128, 2),
+                                    ("f32", 8, 700, 64, 6), ("bf16", 2, 127, 96, 1)]:
+        q, k, v = uniform((2, hq, 1, d), 1), uniform((2, 2, seq, d), 2), uniform((2, 2, seq, d), 3)
         enc = [quantize(x, dtype) if dtype != "f32" else (x.astype(np.float32), x) for x in (q, k, v)]
         t = [host.Tensor.from_numpy(b, dtype) for b, _ in enc]
         res = host.decode_attention(*t)
         assert res.stats["num_splits"] == want, (dtype, hq, res.stats)
-        ref, _ = orc.reference_attention(*[d for _, d in enc], True)
+        ref, _ = orc.reference_attention(*[x for _, x in enc], True)
         out = res.out.numpy()
         got = orc.decode_bits(out, dtype) if dtype != "f32" else out
-        check_attention(got.reshape(-1, 192), ref, dtype, f"host decode {dtype} hq={hq}")
+        check_attention(got.reshape(-1, d), ref, dtype, f"host decode {dtype} hq={hq} seq={seq}")
