@@ -14,7 +14,8 @@
 //   * flash_pair.hip (head_dim 64 and 128, causal grids too small to balance 128-row tiles);
 //   * flash_dsplit.hip (head_dim 192 and 256): the same with the dims of O split over two waves;
 //   * flash_reg.hip (any head_dim whose K/V extent passes the 32-bit buffer offsets of the DMA
-//     kernels, or with negative K/V row strides): K/V staged through registers.
+//     kernels, or with negative K/V row strides; single-tile calls at head dims other than 64 and
+//     128): K/V staged through registers.
 
 #include <hip/hip_runtime.h>
 
@@ -32,6 +33,16 @@ bool DmaReach(const sca_flash_params& p) {
     constexpr int64_t kOverrun = 8 * 64;
     return p.k_ss >= 0 && p.v_ss >= 0 && (p.seq_kv + kOverrun) * p.k_ss * 2 < (1LL << 31) &&
            (p.seq_kv + kOverrun) * p.v_ss * 2 < (1LL << 31);
+}
+
+// One key tile and at most one row tile per CU: latency is all there is, and the register-staged
+// kernel's shorter prologue wins at the head dims that also have it (fp16, D 96, 8 x 24 x 44 6.1 us
+// against 6.8; D 160, 16 x 16 x 64 8.9 against 9.5; D 256, 4 x 16 x 30 7.6 against 8.7; from 44 keys on
+// D 256 is faster in the split-dims kernel, 9.9 against 10.7).
+bool OneTileCall(const sca_flash_params& p) {
+    if (p.head_dim == 64 || p.head_dim == 128) return false;
+    return p.seq_kv <= (p.head_dim > 160 ? 32 : 64) &&
+           (p.seq_q + 127) / 128 * p.batch * p.num_heads <= CuCount();
 }
 
 // ---- Which kernel, and how its rows and keys are cut -------------------------------------------
@@ -54,7 +65,8 @@ int64_t SplitBytes(const sca_flash_params& p, int splits) {
 // second partial wave of pairs; at 256 tiles the pairs are 30% faster.
 //
 // Packing (a GQA group's rows share row tiles) is taken where it leaves fewer row tiles: with few
-// query rows a tile per head is mostly empty and K/V are streamed once per query head.
+// query rows a tile per head is mostly empty and K/V are streamed once per query head. Unsplit only
+// past one row tile per CU: below that the tiles run side by side and fewer of them save nothing.
 //
 // Splitting the keys (allow_split: the caller has scratch for the partial states) pays where the row
 // tiles do not fill the CUs and the keys are many. The estimate below, in microseconds, weighs it
@@ -72,7 +84,7 @@ FlashPlan PlanFlash(const sca_flash_params& p, bool allow_split) {
     const int64_t packed_tiles = (p.seq_q * group + 127) / 128;
     const int pack = packed_tiles < tiles * group && p.seq_q * group < (1LL << 30)
                          ? static_cast<int>(group) : 1;
-    if (!plan.pair) plan.pack = pack;
+    if (!plan.pair && tiles * p.batch * p.num_heads > cus) plan.pack = pack;
     if (!allow_split) return plan;
 
     const double step = 0.1 + 0.0068 * static_cast<double>(p.head_dim);
@@ -161,7 +173,7 @@ __global__ __launch_bounds__(kCombineThreads) void flash_combine_kernel(const sc
 
 template <typename E, bool kCausal>
 int LaunchForDim(const sca_flash_params& p, const FlashPlan& plan, const SplitArgs& sp, hipStream_t s) {
-    const bool reach = DmaReach(p);
+    const bool reach = DmaReach(p) && !OneTileCall(p);
     switch (p.head_dim) {
         case 32:
             return reach ? LaunchFlashWide<E, 32, kCausal>(p, sp, s) : LaunchFlashReg<E, 32, kCausal>(p, s);

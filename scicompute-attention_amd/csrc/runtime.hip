@@ -254,14 +254,17 @@ int sca_hip_stream_is_capturing(void* stream, int* capturing) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     const int rc = FromHip(hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status),
                            "hipStreamIsCapturing");
+    if (rc != 0) (void)hipGetLastError();  // an answer, not an error of the next launch
     *capturing = status != hipStreamCaptureStatusNone ? 1 : 0;
     return rc;
 }
 
 int sca_hip_stream_wait_event(void* stream, void* event) {
-    return FromHip(hipStreamWaitEvent(static_cast<hipStream_t>(stream),
-                                      static_cast<hipEvent_t>(event), 0),
-                   "hipStreamWaitEvent");
+    const int rc = FromHip(hipStreamWaitEvent(static_cast<hipStream_t>(stream),
+                                              static_cast<hipEvent_t>(event), 0),
+                           "hipStreamWaitEvent");
+    if (rc != 0) (void)hipGetLastError();  // the caller has a way on without the wait
+    return rc;
 }
 
 int sca_hip_event_create(void** event) {

@@ -373,3 +373,46 @@ def test_reserved_multi_layer_appends(hip):
     assert e.value.code == 2007
     assert np.array_equal(a.page_table_host(), b.page_table_host()) and a.revision == b.revision
     assert not np.array_equal(before[0], a.page_table_host()) or before[1] != a.revision
+
+
+def test_key_split_scratch_across_streams_and_threads(hip):
+    """Few query rows over many keys through the host API: six streams (more than the scratch has
+    buffers) driven from three threads, each with inputs of its own; every result equals, bit for bit,
+    the same call alone on the default stream, before and after the scratch is released."""
+    import ctypes
+    import threading
+
+    import sca_amd
+    B, Hq, Hkv, Sq, Skv, D = 1, 8, 2, 6, 4102, 128
+    cases = []
+    for i in range(6):
+        t = [tensor(quantize(uniform((B, h, n, D), 600 + 10 * i + j), "bf16")[0], "bf16")
+             for j, (h, n) in enumerate([(Hq, Sq), (Hkv, Skv), (Hkv, Skv)])]
+        s = ctypes.c_void_p()
+        assert hip.sca_hip_stream_create(ctypes.byref(s)) == 0
+        cases.append((t, s.value))
+    want = [H.flash_attention(*t, H.AttentionConfig(causal=True)).out.numpy() for t, _ in cases]
+    sca_amd.synchronize()
+    outs = [[] for _ in cases]
+
+    def drive(mine):
+        for _ in range(5):
+            for i in mine:
+                t, s = cases[i]
+                outs[i].append(H.flash_attention(*t, H.AttentionConfig(causal=True, stream=s)).out)
+
+    threads = [threading.Thread(target=drive, args=(m,)) for m in ([0, 1, 2, 3], [4, 5, 0], [2, 5, 1])]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    sca_amd.synchronize()
+    for i in range(6):
+        for o in outs[i]:
+            assert np.array_equal(o.numpy(), want[i]), i
+    assert H.host_lib().sca_release_scratch() == 0
+    again = H.flash_attention(*cases[0][0], H.AttentionConfig(causal=True, stream=cases[0][1])).out
+    sca_amd.synchronize()
+    assert np.array_equal(again.numpy(), want[0])
+    for _, s in cases:
+        assert hip.sca_hip_stream_destroy(s) == 0
