@@ -402,3 +402,12 @@ def test_key_splits_and_packed_groups(hip, B, Hq, Hkv, Sq, Skv, D, causal):
             check_attention(got.reshape(-1, D), ref.reshape(-1, D), dtype, tag, abs_gate=True)
             err = np.max(np.abs(lse.download(np.float32).astype(np.float64) - ref_lse.reshape(-1)))
             assert err <= 1e-2, f"{tag}: LSE err {err}"
+
+
+@pytest.mark.parametrize("D,causal,dtype", [(128, True, "bf16"), (64, False, "f16"), (96, True, "f16"),
+                                            (256, True, "bf16"), (192, False, "f16")])
+def test_packed_groups_unsplit(hip, D, causal, dtype):
+    """More row tiles than CUs, mostly empty: a GQA group's rows share tiles (160 rows of 4 heads in two
+    tiles, 111 of 3 in one), output and LSE written through the row mapping."""
+    _case(dtype, causal, 12, 32, 8, 40, 90, D, 97000 + D, want_lse=True)
+    _case(dtype, causal, 15, 18, 6, 37, 37 if causal else 70, D, 98000 + D, want_lse=True)
