@@ -72,8 +72,9 @@ int64_t SplitBytes(const sca_flash_params& p, int splits) {
 // tiles do not fill the CUs and the keys are many. The estimate below, in microseconds, weighs it
 // against the unsplit kernel: a wide or split-dims workgroup (one per CU) takes about 0.1 + 0.0068 D
 // per 64 keys and 4 + 0.022 D beside them, a pair workgroup 1.19 times the step per 64 keys of two
-// groups and 5 beside them (both fitted to measurements at D = 32 .. 256), and the merge 5 plus its
-// partials' write and read at 4.5 TB/s.
+// groups and 5 beside them (both fitted to measurements at D = 32 .. 256), and the merge's launch 8 plus
+// its partials' write and read at 4.5 TB/s (with 5 for the launch 24 x 256 over 1,354 keys split, 28.1 us
+// against 26.5 for the pairs).
 FlashPlan PlanFlash(const sca_flash_params& p, bool allow_split) {
     const int64_t cus = CuCount();
     const int64_t group = p.num_heads / p.num_kv_heads;
@@ -105,8 +106,10 @@ FlashPlan PlanFlash(const sca_flash_params& p, bool allow_split) {
         const int64_t n_a = (p.seq_kv + 63) / 64;
         const int64_t n_b = t64 > 1 ? (p.diagonal + 64 + 63) / 64 + 4 : 0;
         const int64_t wgs = (t64 + 1) / 2 * p.batch * p.num_heads;
+        // With half the CUs idle the clock is a quarter higher.
+        const double pair_step = (2 * wgs <= cus ? 0.8 : 1.0) * 1.19 * step;
         best = static_cast<double>((wgs + cus - 1) / cus) *
-               (0.5 * static_cast<double>(n_a + n_b) * 1.19 * step + 5.0);
+               (0.5 * static_cast<double>(n_a + n_b) * pair_step + 5.0);
     } else {
         best = wide_us(units_pack, 1);
     }
@@ -114,7 +117,7 @@ FlashPlan PlanFlash(const sca_flash_params& p, bool allow_split) {
     for (int64_t splits = 2; splits <= 16 && splits * 4 * 64 <= p.seq_kv; ++splits) {
         const int64_t bytes = SplitBytes(p, static_cast<int>(splits));
         if (bytes > kMaxSplitBytes) break;
-        const double us = wide_us(units_pack, splits) + 5.0 + 2.0 * static_cast<double>(bytes) / 4.5e6;
+        const double us = wide_us(units_pack, splits) + 8.0 + 2.0 * static_cast<double>(bytes) / 4.5e6;
         if (us < best) {
             best = us;
             plan = FlashPlan{false, pack, static_cast<int>(splits)};

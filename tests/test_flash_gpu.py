@@ -365,7 +365,7 @@ def _split_params(bufs, dtype, causal, B, Hq, Hkv, Sq, Skv, D):
 
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal", [
     (1, 8, 2, 6, 4102, 128, True),     # packed groups of 4, many splits
-    (2, 7, 1, 5, 2900, 64, True),      # a group that does not divide the row tile
+    (2, 7, 1, 5, 5900, 64, True),      # a group that does not divide the row tile
     (1, 4, 4, 1, 3000, 128, False),    # one row, no group
     (1, 8, 8, 130, 2600, 128, True),   # two row tiles, the second nearly empty
     (1, 6, 2, 43, 1111, 256, True),    # split-dims kernel: packed 129 rows, ragged last split
