@@ -61,8 +61,8 @@ sci::Result<void*> UploadToScratch(ScratchKind kind, const void* host, size_t by
                                    int device_id, void* stream);
 
 // Scratch of one launch sequence on `stream`, safe with any number of threads and streams: at most
-// four buffers per device (64 MiB each), one per stream where possible; a buffer that changes streams
-// waits for the event recorded after its last use, and the lease excludes other threads until its
+// four buffers per device (64 MiB each), one per stream handle where possible; every lease waits on its
+// stream for the event recorded after the buffer's last use, and excludes other threads until its
 // launches are queued. `ptr` is null when there is none to be had (allocation failure, a request above
 // the bound, a stream being captured into a graph): the caller then runs without scratch.
 class StreamScratch {

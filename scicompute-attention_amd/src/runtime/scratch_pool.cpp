@@ -93,12 +93,14 @@ std::vector<StreamSlot*>& StreamSlots() {  // leaked on purpose, like the scratc
     return *slots;
 }
 
-void FreeSlotBuffer(StreamSlot* slot) {
-    if (slot->ptr == nullptr) return;
-    if (slot->event != nullptr) sca_hip_event_synchronize(slot->event);
+// Frees the buffer once its last use has completed; false when that cannot be known (it stays).
+bool FreeSlotBuffer(StreamSlot* slot) {
+    if (slot->ptr == nullptr) return true;
+    if (slot->used != 0 && sca_hip_event_synchronize(slot->event) != 0) return false;
     sci::GpuDevice(slot->device_id).deallocate(slot->ptr);
     slot->ptr = nullptr;
     slot->bytes = 0;
+    return true;
 }
 
 }  // namespace
@@ -129,12 +131,11 @@ StreamScratch::StreamScratch(size_t bytes, int device_id, void* stream) : stream
         StreamSlots().push_back(slot);
     }
     if (slot == nullptr) slot = oldest;
-    if (slot->used != 0 && slot->stream != stream &&
-        sca_hip_stream_wait_event(stream, slot->event) != 0) {
-        return;
-    }
+    // Also when the handles are equal: one value can name several streams (hipStreamPerThread is a
+    // stream per host thread; a handle can be reused after a destroy). On one stream the wait is free.
+    if (slot->used != 0 && sca_hip_stream_wait_event(stream, slot->event) != 0) return;
     if (slot->bytes < bytes) {
-        FreeSlotBuffer(slot);
+        if (!FreeSlotBuffer(slot)) return;
         size_t want = size_t{1} << 20;
         while (want < bytes) want *= 2;
         slot->ptr = sci::GpuDevice(device_id).allocate(want);
@@ -151,13 +152,19 @@ StreamScratch::StreamScratch(size_t bytes, int device_id, void* stream) : stream
 
 StreamScratch::~StreamScratch() {
     if (slot_ == nullptr) return;
-    sca_hip_event_record(static_cast<StreamSlot*>(slot_)->event, stream_);
+    StreamSlot* slot = static_cast<StreamSlot*>(slot_);
+    if (sca_hip_event_record(slot->event, stream_) == 0) return;
+    // The event still stands for an earlier use, which orders nothing: wait here, or give the buffer up.
+    if (sca_hip_stream_synchronize(stream_) != 0) {
+        slot->ptr = nullptr;
+        slot->bytes = 0;
+    }
 }
 
 sci::Status ReleaseScratch() {
     {
         std::lock_guard<std::mutex> streams(StreamMutex());
-        for (StreamSlot* slot : StreamSlots()) FreeSlotBuffer(slot);
+        for (StreamSlot* slot : StreamSlots()) (void)FreeSlotBuffer(slot);
     }
     std::lock_guard<std::mutex> lock(PoolMutex());
     for (auto& kv : Pool()) {

@@ -416,3 +416,32 @@ def test_key_split_scratch_across_streams_and_threads(hip):
     assert np.array_equal(again.numpy(), want[0])
     for _, s in cases:
         assert hip.sca_hip_stream_destroy(s) == 0
+
+
+def test_key_split_scratch_under_the_per_thread_handle(hip):
+    """hipStreamPerThread is one handle value (2) for a stream per host thread: threads that pass it share
+    a buffer by handle and are ordered by its event, so every result equals the call on its own."""
+    import threading
+
+    import sca_amd
+    B, Hq, Hkv, Sq, Skv, D = 1, 8, 2, 6, 4102, 128
+    cases = [[tensor(quantize(uniform((B, h, n, D), 700 + 10 * i + j), "bf16")[0], "bf16")
+              for j, (h, n) in enumerate([(Hq, Sq), (Hkv, Skv), (Hkv, Skv)])] for i in range(4)]
+    want = [H.flash_attention(*t, H.AttentionConfig(causal=True)).out.numpy() for t in cases]
+    sca_amd.synchronize()
+    outs = [[] for _ in cases]
+
+    def drive(i):
+        for _ in range(8):
+            outs[i].append(H.flash_attention(*cases[i], H.AttentionConfig(causal=True, stream=2)).out)
+        assert hip.sca_hip_stream_synchronize(2) == 0  # the thread's stream ends with it
+
+    threads = [threading.Thread(target=drive, args=(i,)) for i in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    sca_amd.synchronize()
+    for i in range(4):
+        for o in outs[i]:
+            assert np.array_equal(o.numpy(), want[i]), i
