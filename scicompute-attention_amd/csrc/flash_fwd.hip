@@ -127,9 +127,11 @@ FlashPlan PlanFlash(const sca_flash_params& p, bool allow_split) {
 }
 
 // Merges the partial states of `splits` key ranges: out = sum_s O_s 2^(m_s - m*) / sum_s l_s 2^(m_s - m*)
-// with m* = max_s m_s (log2 units), states with m_s = -inf skipped and out = 0 when the denominator
-// is 0; LSE = m* + log2 of the denominator, in natural units. One thread per row and 4 dims; bound by
-// the partials' bytes.
+// with m* = max_s m_s (log2 units), states with l_s = 0 (no visible key) skipped and out = 0 when the
+// denominator is 0; LSE = m* + log2 of the denominator, in natural units. A state of NaN scores has
+// l_s = NaN and m_s = NaN or -inf and makes the row NaN, as in the unsplit kernels; this file is
+// therefore compiled with NaN semantics, unlike theirs. One thread per row and 4 dims; bound by the
+// partials' bytes.
 constexpr int kCombineThreads = 256;
 
 template <typename E>
@@ -152,7 +154,7 @@ __global__ __launch_bounds__(kCombineThreads) void flash_combine_kernel(const sc
 #pragma unroll 4
     for (int s = 0; s < sp.splits; ++s) {
         const float2 st = ml[static_cast<int64_t>(s) * rows];
-        if (st.x == neg_inf()) continue;  // its O was not written
+        if (st.y == 0.0f) continue;  // empty: its O may not have been written
         const float w = fast_exp2(st.x - m);
         l = fmaf(st.y, w, l);
         const float4 v = *reinterpret_cast<const float4*>(po + static_cast<int64_t>(s) * rows * p.head_dim);

@@ -404,6 +404,38 @@ def test_key_splits_and_packed_groups(hip, B, Hq, Hkv, Sq, Skv, D, causal):
             assert err <= 1e-2, f"{tag}: LSE err {err}"
 
 
+@pytest.mark.parametrize("D,causal", [(256, True), (192, False), (128, True), (64, False), (96, True)])
+def test_nan_scores_show_with_and_without_key_splits(hip, D, causal):
+    """A query row of NaN, and one NaN key: every row that sees a NaN score comes out as NaN whether the
+    call splits its keys or not, every other row as if there were none."""
+    B, Hq, Hkv, Sq, Skv, dtype = 1, 4, 2, 6, 4100, "f16"
+    qb, qd = quantize(uniform((B, Hq, Sq, D), 99001 + D), dtype)
+    kb, kd = quantize(uniform((B, Hkv, Skv, D), 99002 + D), dtype)
+    vb, vd = quantize(uniform((B, Hkv, Skv, D), 99003 + D), dtype)
+    ref = orc.reference_attention(qd, kd, vd, causal)[0].reshape(Hq, Sq, D)
+    qb[0, 1, 2] = 0x7e00  # head 1 (of KV head 0), query 2
+    kb[0, 1, Skv - 3] = 0x7e00  # KV head 1: seen by all queries, or by the last three
+    bad = np.zeros((Hq, Sq), bool)
+    bad[1, 2] = True
+    bad[2:, Sq - 3 if causal else 0:] = True
+    inputs = [H.DeviceBuffer.from_array(x) for x in (qb, kb, vb)]
+    want = hip.sca_hip_flash_split_bytes
+    want.restype = H.c_i64
+    for split in (True, False):
+        out = H.DeviceBuffer.from_array(np.zeros(B * Hq * Sq * D, np.uint16))
+        lse = H.DeviceBuffer(B * Hq * Sq * 4)
+        p = _split_params([*inputs, out, lse], dtype, causal, B, Hq, Hkv, Sq, Skv, D)
+        n = want(H.ctypes.byref(p)) if split else 0
+        assert n > 0 or not split
+        buf = H.DeviceBuffer(max(n, 16))
+        print(f"D={D} causal={causal} scratch={n}", flush=True)
+        H.check(hip.sca_hip_flash_fwd_split(H.ctypes.byref(p), H.c_vp(buf.ptr), H.c_i64(n), None))
+        sca_amd.synchronize()
+        got = to_float(out.download(np.uint16), dtype).reshape(Sq, Hq, D).transpose(1, 0, 2)
+        assert np.all(np.isnan(got[bad])), f"scratch={n}: a row with NaN scores has finite outputs"
+        check_attention(got[~bad], ref[~bad], dtype, f"D={D} scratch={n}", abs_gate=True)
+
+
 @pytest.mark.parametrize("D,causal,dtype", [(128, True, "bf16"), (64, False, "f16"), (96, True, "f16"),
                                             (256, True, "bf16"), (192, False, "f16")])
 def test_packed_groups_unsplit(hip, D, causal, dtype):
