@@ -491,9 +491,17 @@ constexpr int kRankBatch = 256;  // ragged batches up to this size are ranked in
 // two-stage ring per wave (one LDS object per stage, so the compiler's LDS-DMA tracking waits
 // only for the stage being read); V rows XOR their 32-byte segments so the transposed reads
 // hit distinct banks. A wave always has the next tile in flight while it computes, and the
-// 64 KB ring lets two workgroups share a CU. The probabilities are rounded to fp16/bf16 for the
-// PV MFMA (the reference's decode kernel keeps them in fp32; the denominator here sums the
-// unrounded values), which stays inside the parity tolerance.
+// 64 KB ring lets two workgroups share a CU. At head_dim 64 and 128 the probabilities are rounded to
+// fp16/bf16 for the PV MFMA (the reference's decode kernel keeps them in fp32; the denominator here
+// sums the unrounded values), which stays inside the parity tolerance. At the other head dims no
+// weight loses a bit: P = hi + mid + lo, three values of the input type and three PV MFMAs. The parts
+// of a weight are positive, so an infinite V value stays infinite. fp16 has not the range for small
+// weights: tiles with one below 2^-14 run PV in fp32 instead, V widened in registers and
+// v_mfma_f32_16x16x4 number i (of 8) taking element i of every lane's V fragment and its fp32
+// probability (k = lane group g, token 8g + i of the order above). Measured: bf16, 16 x 32/8 x 4096,
+// D 96 41.7 us, with PV in fp32 throughout 48.3 (5 to 17% more over other shapes too), with two values
+// for a weight 41.4; fp16, 8 x 24/8 x 1994, D 96 15.3, two values 14.7, VALU kernel 20.3. Two values
+// lose fp16 weights below 2^-25, and the second one, 0 or negative, makes NaN of an infinite V.
 constexpr int kMfmaTile = 32;   // tokens per wave iteration
 constexpr int kMfmaHeads = 16;  // query heads per workgroup (MFMA N)
 
@@ -512,6 +520,21 @@ struct DecMfma<DecF16> {
         typedef float f2 __attribute__((ext_vector_type(2)));
         return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){a, b}, pair_t));
     }
+    // Weights from kSplitLeast on, times kScale, have all their 24 bits above fp16's smallest value.
+    static constexpr float kScale = 0x1p15f;
+    static constexpr float kSplitLeast = 0x1p-14f;
+    // Two weights (scaled) as fp16 pairs hi + mid + lo, each rounded towards zero, mid and lo at least
+    // 2^-24 (2^-25 of the smallest weight).
+    static __device__ __forceinline__ void split3(float a, float b, uint32_t* w) {
+        float ra = a, rb = b;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const auto pair = __builtin_amdgcn_cvt_pkrtz(ra, rb);
+            w[i] = __builtin_bit_cast(uint32_t, pair);
+            ra = fmaxf(ra - static_cast<float>(pair[0]), 0x1p-24f);
+            rb = fmaxf(rb - static_cast<float>(pair[1]), 0x1p-24f);
+        }
+    }
 };
 
 template <>
@@ -526,14 +549,28 @@ struct DecMfma<DecBF16> {
         typedef float f2 __attribute__((ext_vector_type(2)));
         return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){a, b}, pair_t));
     }
+    static constexpr float kScale = 1.0f;
+    static constexpr float kSplitLeast = 0.0f;  // bf16 has fp32's range
+    // Two weights as bf16 pairs hi + mid + lo (8 bits each, by truncation), mid and lo at least 2^-126
+    // unless the weight is 0.
+    static __device__ __forceinline__ void split3(float a, float b, uint32_t* w) {
+        float ra = a, rb = b;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const uint32_t ua = __builtin_bit_cast(uint32_t, ra), ub = __builtin_bit_cast(uint32_t, rb);
+            w[i] = (ua >> 16) | (ub & 0xffff0000u);
+            ra = __builtin_amdgcn_fmed3f(ra - __builtin_bit_cast(float, ua & 0xffff0000u), 0x1p-126f, a);
+            rb = __builtin_amdgcn_fmed3f(rb - __builtin_bit_cast(float, ub & 0xffff0000u), 0x1p-126f, b);
+        }
+    }
 };
 
 template <int D>
 struct MfmaDecGeom {
     static_assert(D % 32 == 0 && D <= 256, "MFMA decode covers multiples of 32");
-    // Head dims other than 64 and 128 keep the precision of the fp32 probabilities that they had on
-    // the VALU: P = hi + lo, two values of the input type and two PV MFMAs. The K/V stream hides them.
-    static constexpr bool SPLIT_P = D != 64 && D != 128;
+    // Head dims other than 64 and 128 keep all bits of the fp32 probabilities, which the VALU kernel
+    // gives them (see the kernel's description).
+    static constexpr bool EXACT_P = D != 64 && D != 128;
     static constexpr int NK = D / 32;                    // QK k steps
     static constexpr int ND = D / 16;                    // PV output tiles
     static constexpr int RB = 2 * D;                     // row bytes
@@ -780,22 +817,38 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
                     l += pr[rt][i];
                 }
             }
-            const vec8 pb = __builtin_bit_cast(
-                vec8, make_uint4(M::pack(pr[0][0], pr[0][1]), M::pack(pr[0][2], pr[0][3]),
-                                 M::pack(pr[1][0], pr[1][1]), M::pack(pr[1][2], pr[1][3])));
-            vec8 pb_lo;  // what the rounding of pb lost
-            if constexpr (G::SPLIT_P) {
-                float res[2][4];
+            // P as PV operands: rounded once, or in three parts where every weight of the tile allows it.
+            constexpr int kParts = G::EXACT_P ? 3 : 1;
+            vec8 pb[kParts];
+            bool parts = true;
+            if constexpr (G::EXACT_P && M::kSplitLeast > 0.0f) {
+                float least = 1.0f;
 #pragma unroll
                 for (int rt = 0; rt < 2; ++rt) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        res[rt][i] = pr[rt][i] - static_cast<float>(pb[4 * rt + i]);
+                        // (a masked token's V row is cleared: its parts do not matter)
+                        const int t = 16 * rt + 4 * grp + i;
+                        least = fminf(least, ((valid_mask >> t) & 1u) ? pr[rt][i] : 1.0f);
+                        pr[rt][i] *= M::kScale;
                     }
                 }
-                pb_lo = __builtin_bit_cast(
-                    vec8, make_uint4(M::pack(res[0][0], res[0][1]), M::pack(res[0][2], res[0][3]),
-                                     M::pack(res[1][0], res[1][1]), M::pack(res[1][2], res[1][3])));
+                parts = __builtin_amdgcn_ballot_w64(!(least >= M::kSplitLeast)) == 0;
+            }
+            if constexpr (G::EXACT_P) {
+                uint32_t w[4][3];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    M::split3(pr[i / 2][2 * (i % 2)], pr[i / 2][2 * (i % 2) + 1], w[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    pb[i] = __builtin_bit_cast(vec8, make_uint4(w[0][i], w[1][i], w[2][i], w[3][i]));
+                }
+            } else {
+                pb[0] = __builtin_bit_cast(
+                    vec8, make_uint4(M::pack(pr[0][0], pr[0][1]), M::pack(pr[0][2], pr[0][3]),
+                                     M::pack(pr[1][0], pr[1][1]), M::pack(pr[1][2], pr[1][3])));
             }
             if (valid_mask != 0xffffffffu) {
                 // Clear the V rows of masked tokens: their probabilities are zero, but the rows
@@ -810,14 +863,29 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
                     for (int c = 0; c < kChunksPerLane; ++c) rowp[c] = make_uint4(0, 0, 0, 0);
                 }
             }
-#pragma unroll
-            for (int dt = 0; dt < G::ND; ++dt) {
+            auto v_frag = [&](int dt) __attribute__((always_inline)) {
                 const uint8_t* a = vs + tr_rd + ((dt * 32) ^ tr_x);
                 const uint2 lo = M::Tr::read(a);
                 const uint2 hi = M::Tr::read(a + 16 * G::RB);
-                const vec8 vt = __builtin_bit_cast(vec8, make_uint4(lo.x, lo.y, hi.x, hi.y));
-                o[dt] = M::mma(vt, pb, o[dt]);
-                if constexpr (G::SPLIT_P) o[dt] = M::mma(vt, pb_lo, o[dt]);
+                return __builtin_bit_cast(vec8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+            };
+            if (parts) {
+#pragma unroll
+                for (int dt = 0; dt < G::ND; ++dt) {
+                    const vec8 vt = v_frag(dt);
+#pragma unroll
+                    for (int i = 0; i < kParts; ++i) o[dt] = M::mma(vt, pb[i], o[dt]);
+                }
+            } else {
+#pragma unroll
+                for (int dt = 0; dt < G::ND; ++dt) {
+                    const vec8 vt = v_frag(dt);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(static_cast<float>(vt[e]),
+                                                                     pr[e / 4][e % 4], o[dt], 0, 0, 0);
+                    }
+                }
             }
         };
 
@@ -847,6 +915,10 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_mfma_kernel(const sca_d
         }
     }
 
+    if constexpr (G::EXACT_P && M::kScale != 1.0f) {
+#pragma unroll
+        for (int dt = 0; dt < G::ND; ++dt) o[dt] *= 1.0f / M::kScale;
+    }
     // Lane totals of l over the four lane groups.
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);

@@ -165,3 +165,50 @@ def test_host_decode_splits_fill_the_gpu(hip):
         out = res.out.numpy()
         got = orc.decode_bits(out, dtype) if dtype != "f32" else out
         check_attention(got.reshape(-1, d), ref, dtype, f"host decode {dtype} hq={hq} seq={seq}")
+
+
+@pytest.mark.parametrize("D", [32, 96, 160, 192, 256])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_small_weights_of_a_long_context_count(hip, D, dtype):
+    """One key 17.4 nats above 39,999 equal ones, V = 0 on it and 1 elsewhere: each small weight is
+    2.8e-8 (below fp16's range), together 1.1e-3. Relative bound: the output's rounding u, the share of
+    the small weights that the one lane holding the large one drops from its denominator (1/16 of
+    1.1e-3), chains of up to 2,500 fp32 additions (2,500 * 2^-24) and the exponent's rounding (1e-5)."""
+    B, Hq, Hkv, Skv = 1, 8, 2, 40000
+    qf, kf = np.zeros((B, Hq, 1, D), np.float32), np.zeros((B, Hkv, Skv, D), np.float32)
+    qf[..., 0] = kf[:, :, 0, 0] = np.sqrt(17.4 * np.sqrt(D))
+    vf = np.ones((B, Hkv, Skv, D), np.float32)
+    vf[:, :, 0] = 0.0
+    (qb, qd), (kb, kd), (vb, _) = (quantize(x, dtype) for x in (qf, kf, vf))
+    small = np.exp(-float(qd[0, 0, 0, 0]) * float(kd[0, 0, 0, 0]) / np.sqrt(D))
+    want = (Skv - 1) * small / (1.0 + (Skv - 1) * small)
+    limit = (2.0 ** -11 if dtype == "f16" else 2.0 ** -8) + 7e-5 + 1.5e-4 + 1e-5
+    for splits in (1, 3):
+        print(f"decode {dtype} D={D} splits={splits} dominant key", flush=True)
+        out = run_decode(qb, kb, vb, dtype, B=B, Hq=Hq, Hkv=Hkv, Skv=Skv, D=D, splits=splits)
+        worst = float(np.max(np.abs(out - want))) / want
+        assert worst <= limit, f"off by {worst:.2e} of {want:.2e}"
+
+
+@pytest.mark.parametrize("D", [32, 96, 160, 192, 256])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_infinite_values_stay_infinite(hip, D, dtype):
+    """An infinite V value of a visible key (the dominant one, weight near 1, or any other) gives an
+    infinite output in its dim, and leaves the other dims alone."""
+    B, Hq, Hkv, Skv = 2, 8, 2, 301
+    q, k, v = (uniform(s, 78000 + D + i) for i, s in
+               enumerate([(B, Hq, 1, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)]))
+    k[:, :, 200] = 6.0 * q[:, ::Hq // Hkv, 0]  # close to one weight of 1 for one head per group
+    (qb, qd), (kb, kd), (vb, vd) = (quantize(x, dtype) for x in (q, k, v))
+    ref = orc.reference_attention(qd, kd, vd, True)[0].reshape(B * Hq, D)
+    inf = 0x7c00 if dtype == "f16" else 0x7f80
+    vb[:, :, 200, 3] = vb[:, :, 7, 5] = inf
+    vb[:, :, 200, 17] = vb[:, :, 300, 30] = inf | 0x8000
+    vb[:, :, :, 9] = inf  # also on the keys whose weight is 1 in their tile
+    for splits, waves in ((1, 4), (3, 4), (1, 1), (3, 1)):
+        print(f"decode {dtype} D={D} splits={splits} slot_waves={waves} infinite V", flush=True)
+        out = run_decode(qb, kb, vb, dtype, B=B, Hq=Hq, Hkv=Hkv, Skv=Skv, D=D, splits=splits,
+                         slot_waves=waves).reshape(B * Hq, D)
+        assert np.all(out[:, [3, 5, 9]] == np.inf) and np.all(out[:, [17, 30]] == -np.inf)
+        rest = np.setdiff1d(np.arange(D), [3, 5, 9, 17, 30])
+        check_attention(out[:, rest], ref[:, rest], dtype, f"D={D} splits={splits}")

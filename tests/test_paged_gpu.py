@@ -260,7 +260,7 @@ def test_c5_full_size_against_fp32(hip):
 def test_splits_spanning_several_page_segments(hip, bs, L, splits, D, dtype, slot_waves):
     """Splits longer than one staged page-id segment (2048 pages), starting on and off a page
     boundary: the segment loop restages the page ids of every segment. D=128 bf16 runs the MFMA
-    kernel (one or four waves per KV-head slot), D=96 the VALU kernel."""
+    kernel with one or four waves per KV-head slot, D=96 with four."""
     print(f"paged multi-segment bs={bs} L={L} splits={splits} D={D} {dtype} "
           f"slot_waves={slot_waves}", flush=True)
     _case([L, 3], bs, 8, 2, D, dtype, 87000 + bs + splits + D, splits=splits,
@@ -270,10 +270,10 @@ def test_splits_spanning_several_page_segments(hip, bs, L, splits, D, dtype, slo
 @pytest.mark.parametrize("D", [32, 96, 160, 192, 256])
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_other_head_dims_keep_fp32_weights(hip, D, dtype):
-    """The MFMA kernel at head dims other than 64 and 128 carries the softmax weights as two values of
-    the input type: each output is within the rounding of the output type (unit roundoff u = 2^-11 for
-    fp16, 2^-8 for bf16) plus what two values lose of a weight (u^2, times max |v|, as the weights sum
-    to 1) and the fp32 sums (4e-6). Weights rounded once would be off by up to u * max |v|."""
+    """The MFMA kernel at head dims other than 64 and 128 keeps the softmax weights' fp32 bits: each
+    output is within the rounding of the output type (unit roundoff u = 2^-11 for fp16, 2^-8 for bf16)
+    plus what two 16-bit values would lose of a weight (u^2, times max |v|, as the weights sum to 1)
+    and the fp32 sums (4e-6). Weights rounded once would be off by up to u * max |v|."""
     u = 2.0 ** -11 if dtype == "f16" else 2.0 ** -8
     for Hq, Hkv, bs, waves, splits, lengths in [(8, 2, 16, 4, 3, [1, 31, 33, 700]),
                                                 (14, 2, 32, 1, 2, [64, 129, 5]),
