@@ -102,8 +102,9 @@ struct WideGeom {
     static constexpr int SLOTS = 4;
     static constexpr int V_BASE = SLOTS * TILE_BYTES;
     static constexpr int RING_BYTES = 2 * SLOTS * TILE_BYTES;
-    // Merge: every wave hands one subtile's O (DT*16 floats per lane) and (m, l) to its partner.
-    static constexpr int MERGE_FLOATS = DT * 16 + 2;
+    // Merge: every wave hands one subtile's O (DT*16 floats per lane), m and up to two denominators to
+    // its partner.
+    static constexpr int MERGE_FLOATS = DT * 16 + 3;
     static constexpr int MERGE_BYTES = WAVES * kWave * MERGE_FLOATS * 4;
     static constexpr int LDS_BYTES = RING_BYTES > MERGE_BYTES ? RING_BYTES : MERGE_BYTES;
     static_assert(IPW >= 1 && BN * CPR == IPW * kWave * WAVES, "tile must split evenly");
@@ -370,6 +371,41 @@ __device__ __forceinline__ void ResetRow(RowState& r) {
     r.thr = neg_inf();
     r.neg_mu = 0.0f;
     r.l = 0.0f;
+}
+
+// What the softmax denominator sums. P is rounded to the input type for the PV product, so at head dims
+// other than 64 and 128 the output is divided by the sum of the rounded weights: the rounding cancels
+// (equal values give exactly that value), as in the register-staged kernel. The LSE is made of the
+// unrounded sum, which those kernels add up only when it is asked for. At 64 and 128 one unrounded
+// sum serves both. Against the unrounded sum for all (2 x 16 heads x 4096 causal): D 32 58.8 -> 55.5
+// us, D 96 119.7 -> 121.7, D 160 177 -> 184, D 192 225 -> 218; with LSE, 16/8 heads, D 256 134.7 -> 136.4.
+enum Denominator { kUnrounded, kRounded, kRoundedAndUnrounded };
+template <int D>
+constexpr Denominator DenominatorFor(bool lse) {
+    return D == 64 || D == 128 ? kUnrounded : lse ? kRoundedAndUnrounded : kRounded;
+}
+
+// The VALU operations that turn a lane's 16 scores into P, as codes: 16 exponent arguments
+// s * scale2 - m (0-15), 16 exponentials (16-31), 8 packs to the input type (32-39), 16 additions of
+// the unrounded weights (40-55), 8 pair sums of the rounded ones (56-63). SoftmaxOp gives the n-th of
+// the SoftmaxOps operations of a kernel, in an order that keeps each result at least two operations
+// from its first use (one, for the last pair sum).
+constexpr int SoftmaxOps(Denominator den) {
+    return den == kUnrounded ? 56 : den == kRounded ? 48 : 64;
+}
+__host__ __device__ constexpr int SoftmaxOp(Denominator den, int n) {
+    constexpr int kUn[56] = {0,  1,  2,  3,  16, 17, 4,  5,  18, 19, 6,  7,  20, 21,
+                             32, 33, 8,  9,  22, 23, 34, 10, 11, 24, 25, 35, 40, 41,
+                             12, 13, 26, 27, 36, 42, 43, 14, 15, 28, 29, 37, 44, 45,
+                             30, 31, 46, 47, 38, 39, 48, 49, 50, 51, 52, 53, 54, 55};
+    constexpr int kRo[48] = {0,  1,  2,  3,  16, 17, 4,  5,  18, 19, 6,  7,  20, 21, 32, 33,
+                             8,  9,  22, 23, 34, 56, 10, 11, 24, 25, 35, 57, 12, 13, 26, 27,
+                             36, 58, 14, 15, 28, 29, 37, 59, 30, 31, 38, 60, 39, 61, 62, 63};
+    constexpr int kBo[64] = {0,  1,  2,  3,  16, 17, 4,  5,  18, 19, 6,  7,  20, 21, 32, 33,
+                             8,  9,  22, 23, 34, 56, 10, 11, 24, 25, 35, 57, 40, 41, 12, 13,
+                             26, 27, 36, 58, 42, 43, 14, 15, 28, 29, 37, 59, 44, 45, 30, 31,
+                             60, 46, 47, 38, 39, 61, 48, 49, 50, 51, 62, 52, 53, 63, 54, 55};
+    return den == kUnrounded ? kUn[n < 56 ? n : 0] : den == kRounded ? kRo[n < 48 ? n : 0] : kBo[n];
 }
 
 __device__ __forceinline__ float Max16(const floatx16& s) {

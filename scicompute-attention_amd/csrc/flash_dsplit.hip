@@ -35,7 +35,7 @@ namespace sca_hip {
 namespace {
 
 // kCut: rows packed and / or keys split (SplitArgs).
-template <typename E, int D, bool kCausal, bool kCut>
+template <typename E, int D, bool kCausal, bool kCut, Denominator kDen>
 __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_kernel(
     const sca_flash_params p, int num_q_tiles, const SplitArgs sp) {
     using G = DsplitGeom<D>;
@@ -193,6 +193,7 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
     }
     RowState rs;
     float l2 = 0.0f;  // second half of the denominator (two addition chains)
+    float lw = 0.0f;  // the rounded weights' sum beside the unrounded one (kRoundedAndUnrounded)
     ResetRow(rs);
 
     vec8 kf[G::KS];           // K fragments of the next QK
@@ -239,6 +240,7 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
         rs.m = m_new;
         rs.l *= alpha;
         l2 *= alpha;
+        lw *= alpha;
         rs.thr = (m_new + kRescaleSlack) * inv_scale2;
         rs.neg_mu = (m_new == neg_inf()) ? 0.0f : -m_new;
         if (hh == 0) s_alpha[(par * 4 + rg * 2 + dh) * 32 + lr] = alpha;
@@ -266,21 +268,19 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
         }
         asm volatile("s_nop 4");
     };
-    // The 56 VALU operations that turn the owned scores into P (codes as in the wide kernel: 16
-    // exponent arguments, 16 exponentials, 8 packs, 16 additions of the fp32 weights), in an order
-    // that keeps each result at least two operations from its first use.
+    // The VALU operations that turn the owned scores into P (SoftmaxOp); op(n, ...) runs the n-th.
+    constexpr int kOps = SoftmaxOps(kDen);
     auto op = [&](int n, floatx16& s, uint32_t (&pw)[8]) __attribute__((always_inline)) {
-        constexpr int kOps[56] = {0,  1,  2,  3,  16, 17, 4,  5,  18, 19, 6,  7,  20, 21,
-                                  32, 33, 8,  9,  22, 23, 34, 10, 11, 24, 25, 35, 40, 41,
-                                  12, 13, 26, 27, 36, 42, 43, 14, 15, 28, 29, 37, 44, 45,
-                                  30, 31, 46, 47, 38, 39, 48, 49, 50, 51, 52, 53, 54, 55};
-        const int c = kOps[n];
+        const int c = SoftmaxOp(kDen, n);
         if (c < 16) {
             s[c] = fmaf(s[c], scale2, rs.neg_mu);
         } else if (c < 32) {
             s[c - 16] = fast_exp2(s[c - 16]);
         } else if (c < 40) {
             pw[c - 32] = M::pack(s[2 * (c - 32)], s[2 * (c - 32) + 1]);
+        } else if (c >= 56) {
+            float& sum = kDen == kRoundedAndUnrounded ? lw : c % 2 == 0 ? rs.l : l2;
+            sum = M::sum2(pw[c - 56], sum);
         } else if (c % 2 == 0) {
             rs.l += s[c - 40];
         } else {
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
     {
         uint32_t pw[8];
 #pragma unroll
-        for (int n = 0; n < 56; ++n) op(n, s0, pw);
+        for (int n = 0; n < kOps; ++n) op(n, s0, pw);
         pack_p(pw, pb0);
         write_p.template operator()<0>(pb0);
         const float lm = mask_max(s1, 1, n_plain <= 1);
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
         uint2 flags;
         uint32_t pw[8];
         // ---- A ----
-        constexpr int kOpsA = (56 + G::KS - 1) / G::KS;
+        constexpr int kOpsA = (kOps + G::KS - 1) / G::KS;
         constexpr int kVReads = (4 * G::DT + G::KS - 4) / (G::KS - 3);
         StaticFor<G::KS>([&](auto ks) __attribute__((always_inline)) {
             if constexpr (ks == 0) {
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
             });
 #pragma unroll
             for (int q = 0; q < kOpsA; ++q) {
-                if (ks * kOpsA + q < 56) op(ks * kOpsA + q, s_in, pw);
+                if (ks * kOpsA + q < kOps) op(ks * kOpsA + q, s_in, pw);
             }
             if constexpr (ks % 4 == 2 && ks / 4 < G::IPW) dma_k(ks / 4, (S + 2) & 3, t + 6);
             Fence();
@@ -471,22 +471,30 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
     // ---- epilogue: share 1/l, normalise, store ----
     WaitVm<0>();
     SettleO(o);
-    const float l_tot = HalfSum(rs.l + l2);
+    constexpr bool kBoth = kDen == kRoundedAndUnrounded;
+    const float l_lse = HalfSum(rs.l + l2);
+    const float l_tot = kBoth ? HalfSum(lw) : l_lse;
     if (splits > 1) {
-        // The unnormalised state: both subtiles' O at the scale of their owner's m.
-        if (hh == 0 && qi[0] < seq_q) {
-            *reinterpret_cast<float2*>(sp.part_ml + 2 * (split * rows_all + flat_own)) =
-                make_float2(rs.m, l_tot);
+        // The unnormalised state: both subtiles' O at the scale of their owner's m (and, with two
+        // denominators, to the scale of the unrounded one, which the merge takes).
+        if (hh == 0) {
+            if (kBoth) s_alpha[(rg * 2 + dh) * 32 + lr] = l_tot > 0.0f ? l_lse / l_tot : 0.0f;
+            if (qi[0] < seq_q) {
+                *reinterpret_cast<float2*>(sp.part_ml + 2 * (split * rows_all + flat_own)) =
+                    make_float2(rs.m, l_lse);
+            }
         }
+        if (kBoth) __syncthreads();
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             const int64_t flat = (b * p.num_heads + h0 + hl[r]) * seq_q + qi[r];
             float* dst = sp.part_o + (split * rows_all + flat) * D + dh * (D / 2);
+            const float to_l = kBoth ? s_alpha[(rg * 2 + (dh ^ r)) * 32 + lr] : 1.0f;
 #pragma unroll
             for (int dt = 0; dt < G::DT; ++dt) {
                 float a[16];
 #pragma unroll
-                for (int i = 0; i < 16; ++i) a[i] = o[r][dt][i];
+                for (int i = 0; i < 16; ++i) a[i] = o[r][dt][i] * to_l;
                 StorePartialTile(dst + 32 * dt, hh, qi[r] < seq_q, a);
             }
         }
@@ -495,7 +503,7 @@ __global__ __launch_bounds__(DsplitGeom<D>::THREADS, 1) void flash_fwd_dsplit_ke
     if (hh == 0) {
         s_alpha[(rg * 2 + dh) * 32 + lr] = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
         if (qi[0] < seq_q && p.lse != nullptr) {
-            p.lse[flat_own] = l_tot > 0.0f ? (rs.m + __log2f(l_tot)) * kLn2 : neg_inf();
+            p.lse[flat_own] = l_lse > 0.0f ? (rs.m + __log2f(l_lse)) * kLn2 : neg_inf();
         }
     }
     __syncthreads();
@@ -526,18 +534,23 @@ int LaunchFlashDsplit(const sca_flash_params& p, const SplitArgs& sp, hipStream_
         return SetError(SCA_E_SEQ_TOO_LONG, "flash: grid of " + std::to_string(blocks) +
                                                 " workgroups exceeds the launch limit");
     }
-    auto launch = [&]<bool kCut>() -> int {
-        if (const int rc = EnsureLdsLimit<&flash_fwd_dsplit_kernel<E, D, kCausal, kCut>>(
+    auto launch = [&]<bool kCut, Denominator kDen>() -> int {
+        if (const int rc = EnsureLdsLimit<&flash_fwd_dsplit_kernel<E, D, kCausal, kCut, kDen>>(
                 G::LDS_BYTES, "flash LDS limit")) {
             return rc;
         }
-        hipLaunchKernelGGL((flash_fwd_dsplit_kernel<E, D, kCausal, kCut>),
+        hipLaunchKernelGGL((flash_fwd_dsplit_kernel<E, D, kCausal, kCut, kDen>),
                            dim3(static_cast<unsigned>(blocks)), dim3(G::THREADS), G::LDS_BYTES, s, p,
                            static_cast<int>(num_q_tiles), sp);
         return CheckLaunch("flash_fwd_dsplit_kernel", s);
     };
-    return sp.pack == 1 && sp.splits == 1 ? launch.template operator()<false>()
-                                          : launch.template operator()<true>();
+    const bool cut = sp.pack != 1 || sp.splits != 1;
+    if (p.lse != nullptr) {
+        constexpr Denominator kDen = DenominatorFor<D>(true);
+        return cut ? launch.template operator()<true, kDen>() : launch.template operator()<false, kDen>();
+    }
+    constexpr Denominator kDen = DenominatorFor<D>(false);
+    return cut ? launch.template operator()<true, kDen>() : launch.template operator()<false, kDen>();
 }
 
 #define SCA_INSTANTIATE(E, D)                                                     \

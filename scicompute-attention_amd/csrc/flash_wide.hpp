@@ -20,7 +20,7 @@
 // Measured (MI355X, 2 x 16 heads x 4096 keys) against the register-staged kernel that served these
 // head dims before: D = 160 causal 398 -> 173 us (432 -> 996 TF/s), non-causal 723 -> 333 us (1,032);
 // D = 96 causal 175 -> 122 us (847), non-causal 315 -> 221 us (932); D = 32 causal 78 -> 57 us,
-// non-causal 141 -> 102 us (672: the softmax VALU bounds it, at 4 MFMAs per 56 VALU operations).
+// non-causal 141 -> 102 us (672: the softmax VALU bounds it, at 4 MFMAs per 48 VALU operations).
 //
 // With one workgroup per CU its fixed part is not hidden: 8,192 workgroups of one key tile (D = 128)
 // took 322 us, 9.2 us each beside the step; with the K/V DMAs ahead of the wait for Q, 32-bit index
@@ -41,7 +41,7 @@ namespace {
 // kMode: plain, packed varlen, or cut (rows packed and / or keys split: SplitArgs).
 enum WideMode { kPlain, kPackedVarlen, kCut };
 
-template <typename E, int D, bool kCausal, WideMode kMode>
+template <typename E, int D, bool kCausal, WideMode kMode, Denominator kDen>
 __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel(
     const sca_flash_params p, int num_q_tiles, const VarlenArgs vl, const SplitArgs sp) {
     using G = WideGeom<D>;
@@ -225,13 +225,16 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
         }
     }
     // Row state (RowState); the denominator is summed in two halves (rs.l and l2), which keeps
-    // the two dependency chains of its additions apart.
+    // the two dependency chains of its additions apart. lw: the rounded weights' sum beside the
+    // unrounded one (kRoundedAndUnrounded).
     RowState rs[G::RT];
     float l2[G::RT];
+    float lw[G::RT];
 #pragma unroll
     for (int r = 0; r < G::RT; ++r) {
         ResetRow(rs[r]);
         l2[r] = 0.0f;
+        lw[r] = 0.0f;
     }
 
     // K fragments of the next key tile, and two V^T fragment buffers (tile parity).
@@ -286,6 +289,7 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
             rs[r].m = m_new;
             rs[r].l *= alpha;
             l2[r] *= alpha;
+            if constexpr (kDen == kRoundedAndUnrounded) lw[r] *= alpha;
 #pragma unroll
             for (int dt = 0; dt < G::DT; ++dt) {
                 Fence();  // one O tile at a time through VGPRs
@@ -376,30 +380,27 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
                                            floatx16 (&s_out)[G::RT]) __attribute__((always_inline)) {
         constexpr int VB = S & 1;
         constexpr int NPV = 2 * G::DT;  // PV MFMAs per subtile
+        constexpr int kOps = SoftmaxOps(kDen);  // of each subtile
         // S(j+1) is a real tile. With little register room (D = 160) the QK of a tile past the
         // end runs too (its scores are all masked): merging "computed" and "not computed" scores
         // would make the compiler copy MFMA results it does not know to be in flight.
         const bool next_ok = !kMaskable || D > 128 || j + 1 < n_tiles;
         const bool next_masked = kMaskable && j + 1 >= n_plain;
         uint32_t pw[G::RT][8];
-        // The 56 VALU operations that turn S(j) subtile r into P: 16 exponent arguments
-        // s * scale2 - m (codes 0-15), 16 exponentials (16-31), 8 packs to the input dtype
-        // (32-39) and 16 additions of the fp32 weights into the two denominator halves (40-55),
-        // all in place; op(r, n) runs the n-th in the order of kOps, which keeps each result at
-        // least two operations from its first use. (The sums use v_add: a v_dot2 issued between
-        // MFMAs does not overlap with them.)
+        // The VALU operations that turn S(j) subtile r into P, in place (SoftmaxOp); op(r, n) runs
+        // the n-th. (Unrounded sums use v_add: a v_dot2 issued between MFMAs does not overlap with
+        // them.)
         auto op = [&](int r, int n) __attribute__((always_inline)) {
-            constexpr int kOps[56] = {0,  1,  2,  3,  16, 17, 4,  5,  18, 19, 6,  7,  20, 21,
-                                      32, 33, 8,  9,  22, 23, 34, 10, 11, 24, 25, 35, 40, 41,
-                                      12, 13, 26, 27, 36, 42, 43, 14, 15, 28, 29, 37, 44, 45,
-                                      30, 31, 46, 47, 38, 39, 48, 49, 50, 51, 52, 53, 54, 55};
-            const int c = kOps[n];
+            const int c = SoftmaxOp(kDen, n);
             if (c < 16) {
                 s_in[r][c] = fmaf(s_in[r][c], scale2, rs[r].neg_mu);
             } else if (c < 32) {
                 s_in[r][c - 16] = fast_exp2(s_in[r][c - 16]);
             } else if (c < 40) {
                 pw[r][c - 32] = M::pack(s_in[r][2 * (c - 32)], s_in[r][2 * (c - 32) + 1]);
+            } else if (c >= 56) {
+                float& sum = kDen == kRoundedAndUnrounded ? lw[r] : c % 2 == 0 ? rs[r].l : l2[r];
+                sum = M::sum2(pw[r][c - 56], sum);
             } else if (c % 2 == 0) {
                 rs[r].l += s_in[r][c - 40];
             } else {
@@ -437,14 +438,14 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
         };
 
         // ---- A ----
-        constexpr int kOpsA = (56 + G::KS - 1) / G::KS;  // VALU operations per QK MFMA
+        constexpr int kOpsA = (kOps + G::KS - 1) / G::KS;  // VALU operations per QK MFMA
 #pragma unroll
         for (int ks = 0; ks < G::KS; ++ks) {
             qk(0, ks);
             Fence();
 #pragma unroll
             for (int q = 0; q < kOpsA; ++q) {
-                if (ks * kOpsA + q < 56) op(0, ks * kOpsA + q);
+                if (ks * kOpsA + q < kOps) op(0, ks * kOpsA + q);
             }
             dma(0, ks);
             Fence();
@@ -455,13 +456,13 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
         asm volatile("s_nop 1" : "+v"(pb[0][0]), "+v"(pb[0][1]));
         // ---- B ----
         constexpr int kVReadsB = 4 * G::DT / NPV;  // V reads per PV MFMA
-        constexpr int kOpsB = (28 + NPV - 1) / NPV;  // subtile 1's operations 0-27
+        constexpr int kOpsB = (kOps / 2 + NPV - 1) / NPV;  // subtile 1's operations, first half
         StaticFor<NPV>([&](auto i) __attribute__((always_inline)) {
             pv(0, i);
             Fence();
 #pragma unroll
             for (int q = 0; q < kOpsB; ++q) {
-                if (i * kOpsB + q < 28) op(1, i * kOpsB + q);
+                if (i * kOpsB + q < kOps / 2) op(1, i * kOpsB + q);
             }
             dma(1, i);
             StaticFor<kVReadsB>([&](auto q) __attribute__((always_inline)) {
@@ -471,14 +472,14 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
         });
         // ---- C ----
         float lm0 = neg_inf(), lm1 = neg_inf();
-        constexpr int kOpsC = (28 + G::KS - 1) / G::KS;  // subtile 1's operations 28-55
+        constexpr int kOpsC = (kOps / 2 + G::KS - 1) / G::KS;  // and second half
 #pragma unroll
         for (int ks = 0; ks < G::KS; ++ks) {
             qk(1, ks);
             Fence();
 #pragma unroll
             for (int q = 0; q < kOpsC; ++q) {
-                if (ks * kOpsC + q < 28) op(1, 28 + ks * kOpsC + q);
+                if (ks * kOpsC + q < kOps / 2) op(1, kOps / 2 + ks * kOpsC + q);
             }
             dma(2, ks);
             if (ks == G::KS / 2) {
@@ -544,8 +545,9 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
     WaitVm<0>();
     SettleO(o);
     __builtin_amdgcn_s_barrier();
-    // Wave kq finishes subtile kq: it hands its O and (m, l) of the other subtile to its partner,
-    // as quads (quad k of lane L at k*64 + L: conflict-free 16-byte accesses).
+    // Wave kq finishes subtile kq: it hands its O and (m, denominators) of the other subtile to its
+    // partner, as quads (quad k of lane L at k*64 + L: conflict-free 16-byte accesses).
+    constexpr bool kBoth = kDen == kRoundedAndUnrounded;
     auto region = [&](int w) { return reinterpret_cast<float*>(lds8) + w * kWave * G::MERGE_FLOATS; };
     auto hand_over = [&]<int R>() __attribute__((always_inline)) {
         float4* q4 = reinterpret_cast<float4*>(region(wave)) + lane;
@@ -557,23 +559,35 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
                                                        o[R][dt][4 * g + 2], o[R][dt][4 * g + 3]);
             }
         }
-        reinterpret_cast<float2*>(region(wave) + G::DT * 16 * kWave)[lane] =
-            make_float2(rs[R].m, rs[R].l + l2[R]);
+        const float l = rs[R].l + l2[R];
+        float* st = region(wave) + G::DT * 16 * kWave;
+        reinterpret_cast<float2*>(st)[lane] = make_float2(rs[R].m, kBoth ? lw[R] : l);
+        if constexpr (kBoth) st[2 * kWave + lane] = l;
     };
     auto finish = [&]<int R>() __attribute__((always_inline)) {
         const float* from = region(wave ^ 2);
         const float4* q4 = reinterpret_cast<const float4*>(from) + lane;
         const float2 other = reinterpret_cast<const float2*>(from + G::DT * 16 * kWave)[lane];
         const float mm = fmaxf(rs[R].m, other.x);
-        const float w0 = (rs[R].m == neg_inf()) ? 0.0f : fast_exp2(rs[R].m - mm);
-        const float w1 = (other.x == neg_inf()) ? 0.0f : fast_exp2(other.x - mm);
-        const float l_tot = HalfSum((rs[R].l + l2[R]) * w0) + HalfSum(other.y * w1);
+        float w0 = (rs[R].m == neg_inf()) ? 0.0f : fast_exp2(rs[R].m - mm);
+        float w1 = (other.x == neg_inf()) ? 0.0f : fast_exp2(other.x - mm);
+        const float l = rs[R].l + l2[R];
+        const float l_tot = HalfSum((kBoth ? lw[R] : l) * w0) + HalfSum(other.y * w1);
+        float l_lse = l_tot;
+        if constexpr (kBoth) {
+            l_lse = HalfSum(l * w0) + HalfSum(from[(G::DT * 16 + 2) * kWave + lane] * w1);
+        }
         const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
         const int row = qi[R];
         const bool row_ok = row < seq_q;
         const int64_t h = h0 + hl[R];
         const int64_t flat = (b * p.num_heads + h) * seq_q + row;  // not used by varlen launches
         if (splits > 1) {
+            if constexpr (kBoth) {  // one denominator for the merge: O to the scale of the unrounded one
+                const float c = l_tot > 0.0f ? l_lse / l_tot : 0.0f;
+                w0 *= c;
+                w1 *= c;
+            }
             const int64_t at = split * p.batch * p.num_heads * seq_q + flat;
 #pragma unroll
             for (int dt = 0; dt < G::DT; ++dt) {
@@ -589,7 +603,7 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
                 StorePartialTile(sp.part_o + at * D + 32 * dt, hh, row_ok, a);
             }
             if (row_ok && hh == 0) {
-                *reinterpret_cast<float2*>(sp.part_ml + 2 * at) = make_float2(mm, l_tot);
+                *reinterpret_cast<float2*>(sp.part_ml + 2 * at) = make_float2(mm, l_lse);
             }
             return;
         }
@@ -609,7 +623,7 @@ __global__ __launch_bounds__(WideGeom<D>::THREADS, 1) void flash_fwd_wide_kernel
             StoreTile<M>(out_row + 32 * dt, hh, row_ok, a);
         }
         if (row_ok && p.lse != nullptr && hh == 0) {
-            p.lse[flat] = l_tot > 0.0f ? (mm + __log2f(l_tot)) * kLn2 : neg_inf();
+            p.lse[flat] = l_lse > 0.0f ? (mm + __log2f(l_lse)) * kLn2 : neg_inf();
         }
     };
     if (kq == 0) {
@@ -637,18 +651,23 @@ int LaunchFlashWide(const sca_flash_params& p, const SplitArgs& sp, hipStream_t 
         return SetError(SCA_E_SEQ_TOO_LONG, "flash: grid of " + std::to_string(blocks) +
                                                 " workgroups exceeds the launch limit");
     }
-    auto launch = [&]<WideMode kMode>() -> int {
-        if (const int rc = EnsureLdsLimit<&flash_fwd_wide_kernel<E, D, kCausal, kMode>>(
+    auto launch = [&]<WideMode kMode, Denominator kDen>() -> int {
+        if (const int rc = EnsureLdsLimit<&flash_fwd_wide_kernel<E, D, kCausal, kMode, kDen>>(
                 G::LDS_BYTES, "flash LDS limit")) {
             return rc;
         }
-        hipLaunchKernelGGL((flash_fwd_wide_kernel<E, D, kCausal, kMode>),
+        hipLaunchKernelGGL((flash_fwd_wide_kernel<E, D, kCausal, kMode, kDen>),
                            dim3(static_cast<unsigned>(blocks)), dim3(G::THREADS), G::LDS_BYTES, s, p,
                            static_cast<int>(num_q_tiles), VarlenArgs{nullptr, nullptr, nullptr}, sp);
         return CheckLaunch("flash_fwd_wide_kernel", s);
     };
-    return sp.pack == 1 && sp.splits == 1 ? launch.template operator()<kPlain>()
-                                          : launch.template operator()<kCut>();
+    const bool cut = sp.pack != 1 || sp.splits != 1;
+    if (p.lse != nullptr) {
+        constexpr Denominator kDen = DenominatorFor<D>(true);
+        return cut ? launch.template operator()<kCut, kDen>() : launch.template operator()<kPlain, kDen>();
+    }
+    constexpr Denominator kDen = DenominatorFor<D>(false);
+    return cut ? launch.template operator()<kCut, kDen>() : launch.template operator()<kPlain, kDen>();
 }
 
 // One launch over a packed batch: the wide kernel, one workgroup per (work entry, head).
@@ -656,6 +675,7 @@ template <typename E, int D, bool kCausal>
 int LaunchFlashVarlen(const sca_flash_varlen_params& v, hipStream_t s) {
     using G = WideGeom<D>;
     static_assert(G::BM == 128, "the work list's row tiles are 128 rows");
+    static_assert(DenominatorFor<D>(false) == kUnrounded);
     // 32-bit buffer offsets: a sequence's rows plus the wide kernel's ring overrun must fit.
     const int64_t rows_k = v.max_seq_kv + 8 * G::BN;
     if (rows_k * v.k_ss * 2 >= (1LL << 31) || rows_k * v.v_ss * 2 >= (1LL << 31)) {
@@ -685,11 +705,11 @@ int LaunchFlashVarlen(const sca_flash_varlen_params& v, hipStream_t s) {
     p.scale = v.scale;
     p.causal = v.causal;
     p.dtype = v.dtype;
-    if (const int rc = EnsureLdsLimit<&flash_fwd_wide_kernel<E, D, kCausal, kPackedVarlen>>(
+    if (const int rc = EnsureLdsLimit<&flash_fwd_wide_kernel<E, D, kCausal, kPackedVarlen, kUnrounded>>(
             G::LDS_BYTES, "flash LDS limit")) {
         return rc;
     }
-    hipLaunchKernelGGL((flash_fwd_wide_kernel<E, D, kCausal, kPackedVarlen>),
+    hipLaunchKernelGGL((flash_fwd_wide_kernel<E, D, kCausal, kPackedVarlen, kUnrounded>),
                        dim3(static_cast<unsigned>(blocks)), dim3(G::THREADS), G::LDS_BYTES, s, p,
                        0, VarlenArgs{v.cu_seqlens_q, v.cu_seqlens_kv, v.tiles},
                        SplitArgs{1, 1, nullptr, nullptr});

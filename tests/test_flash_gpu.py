@@ -443,3 +443,39 @@ def test_packed_groups_unsplit(hip, D, causal, dtype):
     tiles, 111 of 3 in one), output and LSE written through the row mapping."""
     _case(dtype, causal, 12, 32, 8, 40, 90, D, 97000 + D, want_lse=True)
     _case(dtype, causal, 15, 18, 6, 37, 37 if causal else 70, D, 98000 + D, want_lse=True)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("D", [32, 96, 160, 192, 256])
+def test_equal_values_come_out_unchanged(hip, D, dtype):
+    """All keys hold one value (just below 2, where a half-ulp is relatively smallest): divided by the
+    sum of the rounded weights the output is that value to the bit, whole, packed or split, with LSE or
+    without; the LSE is that of the unrounded weights (fp32 sums: 2e-5 of values up to 10)."""
+    want = H.hip_lib().sca_hip_flash_split_bytes
+    want.restype = H.c_i64
+    for B, Hq, Hkv, Sq, Skv, causal in [(1, 8, 2, 200, 300, True), (1, 4, 4, 130, 257, False),
+                                        (1, 8, 2, 6, 4100, True)]:
+        qb, qd = quantize(3.0 * uniform((B, Hq, Sq, D), 99101 + D), dtype)
+        kb, kd = quantize(3.0 * uniform((B, Hkv, Skv, D), 99102 + D), dtype)
+        vb = np.full((B, Hkv, Skv, D), 0x3fff, np.uint16)
+        lse_ref = orc.reference_attention(qd, kd, np.ones_like(kd), causal)[1].reshape(Hq, Sq)
+        inputs = [H.DeviceBuffer.from_array(x) for x in (qb, kb, vb)]
+        for with_lse in (False, True):
+            out = H.DeviceBuffer.from_array(np.zeros(B * Hq * Sq * D, np.uint16))
+            lse = H.DeviceBuffer(B * Hq * Sq * 4)
+            p = _split_params([*inputs, out, lse], dtype, causal, B, Hq, Hkv, Sq, Skv, D)
+            if not with_lse:
+                p.lse = None
+            n = want(H.ctypes.byref(p))
+            buf = H.DeviceBuffer(max(n, 16))
+            for scratch in {0, n}:
+                print(f"{dtype} D={D} {Hq}/{Hkv} x {Sq} x {Skv} lse={with_lse} scratch={scratch}",
+                      flush=True)
+                H.check(hip.sca_hip_flash_fwd_split(H.ctypes.byref(p), H.c_vp(buf.ptr),
+                                                    H.c_i64(scratch), None))
+                sca_amd.synchronize()
+                off = int(np.count_nonzero(out.download(np.uint16) != 0x3fff))
+                assert off == 0, f"{off} of {B * Hq * Sq * D} outputs differ from the value"
+                if with_lse:
+                    err = float(np.max(np.abs(lse.download(np.float32).reshape(Hq, Sq) - lse_ref)))
+                    assert err <= 2e-5, f"LSE err {err:.2e}"
