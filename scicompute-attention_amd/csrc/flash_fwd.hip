@@ -7,15 +7,15 @@
 // q head h to kv head h / (H_q / H_kv), P is rounded to the input dtype before the PV product,
 // out = O / l (0 when l == 0), LSE = m + ln(l) (-inf when l == 0).
 //
-// Three kernels share one formulation (flash_common.hpp); this file validates and picks:
+// Four kernels share one formulation (flash_common.hpp); this file validates and picks:
 //   * flash_wide.hpp (head_dim 32 to 160: every non-causal grid, large causal grids and, at 64 and
 //     128, packed variable-length batches in one launch): 4 waves of 64 query rows, K/V tiles
 //     DMA'd into LDS;
 //   * flash_pair.hip (head_dim 64 and 128, causal grids too small to balance 128-row tiles);
 //   * flash_dsplit.hip (head_dim 192 and 256): the same with the dims of O split over two waves;
 //   * flash_reg.hip (any head_dim whose K/V extent passes the 32-bit buffer offsets of the DMA
-//     kernels, or with negative K/V row strides; single-tile calls at head dims other than 64 and
-//     128): K/V staged through registers.
+//     kernels, or with negative K/V row strides; small calls of one or two key tiles at head dims other
+//     than 64 and 128): K/V staged through registers.
 
 #include <hip/hip_runtime.h>
 
@@ -35,14 +35,23 @@ bool DmaReach(const sca_flash_params& p) {
            (p.seq_kv + kOverrun) * p.v_ss * 2 < (1LL << 31);
 }
 
-// One key tile and at most one row tile per CU: latency is all there is, and the register-staged
-// kernel's shorter prologue wins at the head dims that also have it (fp16, D 96, 8 x 24 x 44 6.1 us
-// against 6.8; D 160, 16 x 16 x 64 8.9 against 9.5; D 256, 4 x 16 x 30 7.6 against 8.7; from 44 keys on
-// D 256 is faster in the split-dims kernel, 9.9 against 10.7).
-bool OneTileCall(const sca_flash_params& p) {
+// One or two key tiles and a grid that leaves CUs idle: latency is all there is, and the register-staged
+// kernel's shorter prologue wins at the head dims that also have it. Microseconds, register-staged
+// against the kernel that serves longer calls:
+//   one tile, up to one row tile per CU: D 96, 8 x 24 x 44 6.1 / 6.8; D 160, 16 x 16 x 64 8.9 / 9.5;
+//   D 256, 4 x 16 x 30 7.6 / 8.7, from 44 keys on 10.7 / 9.9;
+//   two, up to half the CUs (16 to 128 workgroups alike; at 192 the order turns): causal D 96 x 70 keys
+//   7.35 / 7.73, x 96 7.58 / 7.82, x 104 7.80 / 7.85, x 120 7.98 / 7.91, D 32 x 80 5.56 / 5.61, D 96 20
+//   rows x 110 keys 7.05 / 7.35 and 5 x 126 7.14 / 7.33; non-causal D 96 x 95 7.62 / 7.39; D 160 x 70 9.55
+//   / 9.81, x 96 9.87 / 9.99, x 128 11.9 / 10.2, non-causal x 96 9.22 / 9.83. With LSE they stay with
+//   the kernels whose LSE sums unrounded weights.
+bool FewTilesCall(const sca_flash_params& p) {
     if (p.head_dim == 64 || p.head_dim == 128) return false;
-    return p.seq_kv <= (p.head_dim > 160 ? 32 : 64) &&
-           (p.seq_q + 127) / 128 * p.batch * p.num_heads <= CuCount();
+    const int64_t row_tiles = (p.seq_q + 127) / 128 * p.batch * p.num_heads;
+    if (p.seq_kv <= (p.head_dim > 160 ? 32 : 64)) return row_tiles <= CuCount();
+    if (p.head_dim > 160 || p.lse != nullptr || 2 * row_tiles > CuCount()) return false;
+    if (p.head_dim == 160) return p.seq_kv <= 96;
+    return p.causal && p.seq_kv <= (p.head_dim == 96 && p.seq_q <= 32 ? 128 : 100);
 }
 
 // ---- Which kernel, and how its rows and keys are cut -------------------------------------------
@@ -178,7 +187,7 @@ __global__ __launch_bounds__(kCombineThreads) void flash_combine_kernel(const sc
 
 template <typename E, bool kCausal>
 int LaunchForDim(const sca_flash_params& p, const FlashPlan& plan, const SplitArgs& sp, hipStream_t s) {
-    const bool reach = DmaReach(p) && !OneTileCall(p);
+    const bool reach = DmaReach(p) && !FewTilesCall(p);
     switch (p.head_dim) {
         case 32:
             return reach ? LaunchFlashWide<E, 32, kCausal>(p, sp, s) : LaunchFlashReg<E, 32, kCausal>(p, s);

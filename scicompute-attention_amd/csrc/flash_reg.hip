@@ -1,8 +1,9 @@
 // Register-staged flash kernel: 4 row groups of 32 query rows, K/V staged through registers into an
 // LDS ring with V transposed on the way in. It addresses K and V with 64-bit pointers per tile, so
 // it serves the calls that the DMA kernels' 32-bit buffer offsets cannot reach (K/V extents of 2 GiB
-// and more, negative row strides), at any head_dim; and, with the shorter prologue, calls of a single
-// key tile at head dims other than 64 and 128 (OneTileCall). The DMA kernels are 1.4-2.5x faster elsewhere.
+// and more, negative row strides), at any head_dim; and, with the shorter prologue, small calls of one
+// or two key tiles at head dims other than 64 and 128 (FewTilesCall). The DMA kernels are 1.4-2.5x
+// faster on long calls.
 
 #include <hip/hip_runtime.h>
 

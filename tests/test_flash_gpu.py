@@ -479,3 +479,24 @@ def test_equal_values_come_out_unchanged(hip, D, dtype):
                 if with_lse:
                     err = float(np.max(np.abs(lse.download(np.float32).reshape(Hq, Sq) - lse_ref)))
                     assert err <= 2e-5, f"LSE err {err:.2e}"
+
+
+@pytest.mark.parametrize("D,Sq,Skv,causal", [
+    (32, 100, 100, True), (32, 101, 101, True), (96, 100, 100, True), (96, 101, 101, True),
+    (96, 32, 128, True), (96, 33, 128, True), (96, 32, 129, True), (96, 70, 70, False),
+    (160, 96, 96, True), (160, 97, 97, True), (160, 20, 96, False), (160, 96, 97, False)])
+def test_two_key_tiles_either_side_of_the_kernel_rule(hip, D, Sq, Skv, causal):
+    """Calls of two key tiles run the register-staged kernel up to half the CUs and the DMA kernels past
+    it, with more keys or with an LSE (of unrounded weights: 2e-5): both sides of each line, on a small
+    grid and on one past half the CUs."""
+    for B, Hq, Hkv, dtype in [(1, 6, 2, "f16"), (5, 32, 8, "bf16")]:
+        q, k, v = (quantize(uniform(s, 99201 + D + i), dtype) for i, s in
+                   enumerate([(B, Hq, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)]))
+        ref, lse_ref = orc.reference_attention(q[1], k[1], v[1], causal)
+        for want_lse in (False, True):
+            print(f"{dtype} {B}x{Hq}/{Hkv} {Sq}x{Skv} D={D} causal={causal} lse={want_lse}", flush=True)
+            out, lse = run_flash(q[0], k[0], v[0], dtype, causal, B=B, Hq=Hq, Hkv=Hkv, Sq=Sq, Skv=Skv,
+                                 D=D, want_lse=want_lse)
+            check_attention(out.reshape(-1, D), ref.reshape(-1, D), dtype, f"D={D} {Sq}x{Skv}")
+        err = float(np.max(np.abs(lse.reshape(-1) - lse_ref.reshape(-1))))
+        assert err <= 2e-5, f"LSE err {err:.1e}"
