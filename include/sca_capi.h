@@ -117,11 +117,16 @@ SCA_CAPI int sca_select(const ScaConfig* cfg, const ScaShape* shape, int32_t* ba
                         int32_t* tile4, uint64_t* workspace_bytes, char* reason, size_t len);
 SCA_CAPI void sca_explain(const ScaConfig* cfg, const ScaShape* shape, char* out, size_t len);
 SCA_CAPI void sca_recommend_tile(const ScaConfig* cfg, const ScaShape* shape, int32_t* tile4);
+/* Split count of the contiguous decode launcher from the shape alone, whatever the type. The backend
+ * itself takes fewer for 16-bit types from head_dim 160 on and, there and for fp32, more for a few
+ * short sequences. */
 SCA_CAPI int64_t sca_decode_splits(const ScaShape* shape, int64_t cu_count);
 /* Length-aware work split of the paged MFMA decode kernel (no reference counterpart: the
  * reference sizes paged splits from the pool alone). lengths = the batch's host-side key counts;
  * writes the split count and the sca_decode_params.slot_waves value (1 or 4; 0 with splits 1
- * when every length is 0) the paged backend uses when the cache's own page table is attended.
+ * when every length is 0) the paged backend uses when the cache's own page table is attended, made
+ * for head_dim up to 128 and batches that fill the GPU: where one wave per slot would leave half the
+ * CUs idle the backend takes four (and shorter splits), and from head_dim 160 on always four.
  * Returns 0, or SCA_E_SHAPE_MISMATCH. */
 SCA_CAPI int sca_paged_decode_plan(const int64_t* lengths, int64_t batch, int64_t num_heads,
                                    int64_t num_kv_heads, int64_t cu_count, int64_t* splits,

@@ -13,6 +13,7 @@ struct DecodeConfig {
     bool use_splitk{true};   // false => one split (no combine pass)
 };
 
+// What a call with num_splits = 0 takes for 16-bit types (fp32 may take more splits).
 SCI_ATTENTION_API DecodeConfig RecommendDecodeConfig(const AttentionShape& shape,
                                                      const DeviceCapability& cap);
 

@@ -4,6 +4,7 @@
 // src/backends/decode/decode_backend.cpp:53-214 and src/backends/paged/paged_backend.cpp:40-253;
 // the split count comes from the MI355X dispatch table (runtime/dispatch_table.hpp).
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -25,16 +26,25 @@ int64_t PartialElements(int64_t batch, int64_t heads, int64_t splits, int64_t he
 }
 
 // Explicit split counts are honoured up to the table's cap; otherwise the table decides.
-int64_t ResolveSplits(int64_t requested, int64_t batch, int64_t num_heads, int64_t num_kv_heads,
-                      int64_t seq_kv, int64_t head_dim, int slot_waves = 4, bool half = false) {
+int64_t CappedSplits(int64_t requested) {
     const auto& th = detail::kDispatchThresholds;
-    if (requested > 0) return requested < th.max_splits ? requested : th.max_splits;
-    const int cus = DeviceCapability::ForDevice(0).sm_count;
-    const int64_t splits = detail::DecodeSplits(batch, num_heads, num_kv_heads, seq_kv, cus,
-                                                slot_waves, head_dim, half);
-    if (slot_waves != 4 || batch < 1 || num_kv_heads < 1 || (half && head_dim < 160)) return splits;
-    const int64_t slots = num_kv_heads * ((num_heads / num_kv_heads + 15) / 16);
-    return detail::FillSplits(splits, batch * slots, seq_kv, cus);
+    return requested < th.max_splits ? requested : th.max_splits;
+}
+int64_t ResolveSplits(const AttentionConfig& cfg, const AttentionShape& s, bool half) {
+    if (cfg.num_splits > 0) return CappedSplits(cfg.num_splits);
+    return detail::ContiguousDecodeSplits(s.batch, s.num_heads, s.num_kv_heads, s.seq_kv,
+                                          DeviceCapability::ForDevice(0).sm_count, s.head_dim, half);
+}
+// The most splits a call of this shape runs: the count depends on the type, which a shape leaves open.
+int64_t MostSplits(const AttentionConfig& cfg, const AttentionShape& shape) {
+    return std::max(ResolveSplits(cfg, shape, /*half=*/false), ResolveSplits(cfg, shape, /*half=*/true));
+}
+// Paged KV without a plan: one wave per slot over `seq_kv` keys.
+int64_t ResolvePagedSplits(int64_t requested, int64_t batch, int64_t num_heads, int64_t num_kv_heads,
+                           int64_t seq_kv, int64_t head_dim) {
+    if (requested > 0) return CappedSplits(requested);
+    return detail::DecodeSplits(batch, num_heads, num_kv_heads, seq_kv,
+                                DeviceCapability::ForDevice(0).sm_count, /*slot_waves=*/1, head_dim);
 }
 
 // Points the partial pointers of `p` into the pooled FP32 scratch (m | l | O).
@@ -74,9 +84,7 @@ public:
                               const AttentionShape& shape) const override {
         CapabilityReport report;
         report.recommended_backend = BackendKind::kDecode;
-        const int64_t splits = ResolveSplits(cfg.num_splits, shape.batch, shape.num_heads,
-                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim,
-                                             /*slot_waves=*/4, /*half=*/true);
+        const int64_t splits = MostSplits(cfg, shape);
         report.workspace_bytes = WorkspaceBytes(cfg, shape);
         std::string reason;
         if (!DeviceCapability::GpuAvailable()) {
@@ -94,7 +102,7 @@ public:
         }
         report.supported = reason.empty();
         report.reason = report.supported
-                            ? "split-K decode with " + std::to_string(splits) +
+                            ? "split-K decode with up to " + std::to_string(splits) +
                                   " splits, workspace " + std::to_string(report.workspace_bytes) +
                                   " B (FP32 partials)"
                             : reason;
@@ -102,9 +110,7 @@ public:
     }
 
     size_t WorkspaceBytes(const AttentionConfig& cfg, const AttentionShape& shape) const override {
-        const int64_t splits = ResolveSplits(cfg.num_splits, shape.batch, shape.num_heads,
-                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim,
-                                             /*slot_waves=*/4, /*half=*/true);
+        const int64_t splits = MostSplits(cfg, shape);
         if (splits <= 1) return 0;
         return static_cast<size_t>(
                    PartialElements(shape.batch, shape.num_heads, splits, shape.head_dim)) *
@@ -135,9 +141,7 @@ public:
         if (!DeviceCapability::GpuAvailable()) {
             return fail(AttnStatusCode::kUnsupportedFeature, "decode backend: no GPU device");
         }
-        const int64_t splits = ResolveSplits(cfg.num_splits, shape.batch, shape.num_heads,
-                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim,
-                                             /*slot_waves=*/4, q.dtype() != sci::DType::kFloat32);
+        const int64_t splits = ResolveSplits(cfg, shape, q.dtype() != sci::DType::kFloat32);
 
         AttentionResult result;
         result.out = sci::Tensor(sci::TensorShape({shape.batch, shape.num_heads, shape.seq_q,
@@ -225,9 +229,8 @@ public:
     // An estimate from the shape alone (one wave per slot over seq_kv keys); a run under the
     // cache's length-aware plan binds, and reports in stats.workspace_bytes, what it uses.
     size_t WorkspaceBytes(const AttentionConfig& cfg, const AttentionShape& shape) const override {
-        const int64_t splits = ResolveSplits(cfg.num_splits, shape.batch, shape.num_heads,
-                                             shape.num_kv_heads, shape.seq_kv, shape.head_dim,
-                                             /*slot_waves=*/1);
+        const int64_t splits = ResolvePagedSplits(cfg.num_splits, shape.batch, shape.num_heads,
+                                                  shape.num_kv_heads, shape.seq_kv, shape.head_dim);
         if (splits <= 1) return 0;
         return static_cast<size_t>(
                    PartialElements(shape.batch, shape.num_heads, splits, shape.head_dim)) *
@@ -325,8 +328,8 @@ sci::Result<AttentionResult> RunPaged(const sci::Tensor& q, const PagedKVCache& 
     // Upper bound of a sequence's length; the kernel reads the true lengths from seq_lens.
     const int64_t seq_kv_bound = kv_cfg.num_blocks * block_size;
     int64_t splits =
-        ResolveSplits(cfg.num_splits, num_seqs, num_heads, kv_cfg.num_kv_heads, seq_kv_bound,
-                      head_dim, /*slot_waves=*/1);
+        ResolvePagedSplits(cfg.num_splits, num_seqs, num_heads, kv_cfg.num_kv_heads, seq_kv_bound,
+                           head_dim);
     int32_t slot_waves = 0;
     // With the cache's own page table, its host-side lengths say how ragged the batch is; the
     // MFMA kernel (fp16/bf16, power-of-two pages) then takes the split count
@@ -408,8 +411,9 @@ const IAttentionBackend* PagedBackendInstance() noexcept { return &kPagedBackend
 DecodeConfig RecommendDecodeConfig(const AttentionShape& shape, const DeviceCapability& cap) {
     DecodeConfig cfg;
     cfg.max_splits = detail::kDispatchThresholds.max_splits;
-    cfg.num_splits = detail::DecodeSplits(shape.batch, shape.num_heads, shape.num_kv_heads,
-                                          shape.seq_kv, cap.sm_count, 4, shape.head_dim);
+    cfg.num_splits = detail::ContiguousDecodeSplits(shape.batch, shape.num_heads, shape.num_kv_heads,
+                                                    shape.seq_kv, cap.sm_count, shape.head_dim,
+                                                    /*half=*/true);
     return cfg;
 }
 

@@ -2,8 +2,8 @@
 // Request checks, output allocation (always contiguous BHSD, optional FP32 LSE) and the varlen
 // contract follow the reference's src/backends/flash/flash_backend.cpp:43-376.
 //
-// Guarantees: the S_q x S_kv score matrix never reaches HBM (workspace_bytes == 0 and
-// materialized_score_bytes == 0 on every result).
+// Guarantees: the S_q x S_kv score matrix never reaches HBM (materialized_score_bytes == 0 on every
+// result); workspace_bytes counts the partial states of a call that splits its keys, 0 for all others.
 
 #include <algorithm>
 #include <vector>
@@ -49,6 +49,31 @@ sci::Status CheckDtype(sci::DType dtype) {
                           " is served by the naive (reference) or tiled backend");
 }
 
+// The kernel's parameters for contiguous tensors of this shape, pointers and type left open.
+sca_flash_params ParamsFor(const AttentionConfig& cfg, const AttentionShape& shape) {
+    const detail::Strides qs =
+        detail::StridesFor(cfg.layout, shape.seq_q, shape.num_heads, shape.head_dim);
+    const detail::Strides ks =
+        detail::StridesFor(cfg.layout, shape.seq_kv, shape.num_kv_heads, shape.head_dim);
+    const detail::Strides os =
+        detail::StridesFor(AttnLayout::kBHSD, shape.seq_q, shape.num_heads, shape.head_dim);
+    sca_flash_params p{};
+    p.batch = shape.batch;
+    p.num_heads = shape.num_heads;
+    p.num_kv_heads = shape.num_kv_heads;
+    p.seq_q = shape.seq_q;
+    p.seq_kv = shape.seq_kv;
+    p.head_dim = shape.head_dim;
+    p.q_sb = qs.s_b, p.q_sh = qs.s_h, p.q_ss = qs.s_s;
+    p.k_sb = ks.s_b, p.k_sh = ks.s_h, p.k_ss = ks.s_s;
+    p.v_sb = ks.s_b, p.v_sh = ks.s_h, p.v_ss = ks.s_s;
+    p.o_sb = os.s_b, p.o_sh = os.s_h, p.o_ss = os.s_s;
+    p.scale = EffectiveScale(cfg, shape);
+    p.causal = cfg.causal ? 1 : 0;
+    p.diagonal = cfg.causal ? shape.seq_kv - shape.seq_q : 0;
+    return p;
+}
+
 void FillStats(AttentionRuntimeStats* stats, const TileConfig& tile, const std::string& note) {
     stats->used_backend = BackendKind::kFlash;
     stats->tile = tile;
@@ -66,12 +91,13 @@ public:
                               const AttentionShape& shape) const override {
         CapabilityReport report;
         report.recommended_backend = BackendKind::kFlash;
-        report.workspace_bytes = 0;
         const std::string refusal = FlashRefusal(cfg, shape);
         report.supported = refusal.empty();
         if (report.supported) {
             report.tile = RecommendTile(cfg, shape);
-            report.reason = "online softmax in registers (workspace 0 B), tile " +
+            report.workspace_bytes = WorkspaceBytes(cfg, shape);
+            report.reason = "online softmax in registers (workspace " +
+                            std::to_string(report.workspace_bytes) + " B), tile " +
                             report.tile.ToString();
         } else {
             report.reason = refusal;
@@ -79,7 +105,14 @@ public:
         return report;
     }
 
-    size_t WorkspaceBytes(const AttentionConfig&, const AttentionShape&) const override { return 0; }
+    // Partial states of a call that splits its keys; a call that finds no scratch runs without.
+    size_t WorkspaceBytes(const AttentionConfig& cfg, const AttentionShape& shape) const override {
+        sca_flash_params p = ParamsFor(cfg, shape);
+        p.dtype = SCA_DTYPE_BF16;
+        p.q = p.k = p.v = p.out = reinterpret_cast<void*>(16);  // any aligned address: nothing is read
+        if (cfg.return_lse) p.lse = static_cast<float*>(p.out);
+        return static_cast<size_t>(sca_hip_flash_split_bytes(&p));
+    }
 
     sci::Result<AttentionResult> Forward(const sci::Tensor& q, const sci::Tensor& k,
                                          const sci::Tensor& v,
@@ -114,39 +147,21 @@ public:
             }
         }
 
-        const detail::Strides qs =
-            detail::StridesFor(cfg.layout, shape.seq_q, shape.num_heads, shape.head_dim);
-        const detail::Strides ks =
-            detail::StridesFor(cfg.layout, shape.seq_kv, shape.num_kv_heads, shape.head_dim);
-        const detail::Strides os =
-            detail::StridesFor(AttnLayout::kBHSD, shape.seq_q, shape.num_heads, shape.head_dim);
-        sca_flash_params p{};
+        sca_flash_params p = ParamsFor(cfg, shape);
         p.q = q.data();
         p.k = k.data();
         p.v = v.data();
         p.out = result.out.data();
         p.lse = cfg.return_lse ? static_cast<float*>(result.lse.data()) : nullptr;
-        p.batch = shape.batch;
-        p.num_heads = shape.num_heads;
-        p.num_kv_heads = shape.num_kv_heads;
-        p.seq_q = shape.seq_q;
-        p.seq_kv = shape.seq_kv;
-        p.head_dim = shape.head_dim;
-        p.q_sb = qs.s_b, p.q_sh = qs.s_h, p.q_ss = qs.s_s;
-        p.k_sb = ks.s_b, p.k_sh = ks.s_h, p.k_ss = ks.s_s;
-        p.v_sb = ks.s_b, p.v_sh = ks.s_h, p.v_ss = ks.s_s;
-        p.o_sb = os.s_b, p.o_sh = os.s_h, p.o_ss = os.s_s;
-        p.scale = EffectiveScale(cfg, shape);
-        p.causal = cfg.causal ? 1 : 0;
         p.dtype = runtime::KernelDtype(q.dtype());
-        p.diagonal = cfg.causal ? shape.seq_kv - shape.seq_q : 0;
         void* stream = runtime::StreamHandle(cfg.stream);
+        int64_t split_bytes = sca_hip_flash_split_bytes(&p);
         {
             // Partial states of a run that splits the keys (no score scratch; none for most calls).
-            const int64_t split_bytes = sca_hip_flash_split_bytes(&p);
             const runtime::StreamScratch scratch(static_cast<size_t>(split_bytes), device.id(), stream);
+            if (scratch.ptr == nullptr) split_bytes = 0;
             status = runtime::StatusFromHip(
-                sca_hip_flash_fwd_split(&p, scratch.ptr, scratch.ptr != nullptr ? split_bytes : 0, stream),
+                sca_hip_flash_fwd_split(&p, scratch.ptr, split_bytes, stream),
                 "flash forward");
         }
         if (!status.ok()) return sci::MakeUnexpected<AttentionResult>(status);
@@ -155,6 +170,7 @@ public:
         FillStats(&result.stats, tile,
                   "flash: gfx950 MFMA 32x32x16, tile " + tile.ToString() +
                       ", S/P in registers; layout=" + LayoutName(cfg.layout));
+        result.stats.workspace_bytes = static_cast<size_t>(split_bytes);
         return sci::Ok(std::move(result));
     }
 

@@ -105,6 +105,16 @@ inline int64_t FillSplits(int64_t splits, int64_t jobs, int64_t longest, int64_t
     return fill > splits ? fill : splits;
 }
 
+// The contiguous backend's split count (four waves per slot); `half`: 16-bit types.
+inline int64_t ContiguousDecodeSplits(int64_t batch, int64_t num_heads, int64_t num_kv_heads,
+                                      int64_t seq_kv, int64_t cu_count, int64_t head_dim, bool half) {
+    const int64_t splits =
+        DecodeSplits(batch, num_heads, num_kv_heads, seq_kv, cu_count, 4, head_dim, half);
+    if (batch < 1 || num_kv_heads < 1 || (half && head_dim < 160)) return splits;
+    const int64_t slots = num_kv_heads * ((num_heads / num_kv_heads + 15) / 16);
+    return FillSplits(splits, batch * slots, seq_kv, cu_count);
+}
+
 // Work split of the paged MFMA decode kernel for a batch whose host-side lengths are known.
 // slot_waves = 1: one wave per head slot, a workgroup serves four slots; 4: four waves share one
 // slot's key tiles. Measured on MI355X over 48-step decode loops (bf16, H_q 32, H_kv 8, D 128):

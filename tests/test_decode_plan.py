@@ -4,6 +4,9 @@ The expected (splits, slot_waves) pairs are the fastest settings measured on an 
 for these batches in 48-step bf16 decode loops (H_q 32, H_kv 8, D 128, bs 16): each row names
 the measured rate of the chosen setting and of the best alternative."""
 
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -97,3 +100,24 @@ def test_contiguous_decode_splits_valu_head_dim(B, S, want):
     # head_dim 96 runs the VALU kernel: splits until every CU holds four workgroups, no cap at
     # 8, and at least min_tokens_per_split keys per split (the 1 x 1024 case)
     assert H.decode_splits(H.AttentionShape(B, 1, S, 32, 8, 96), CUS) == want
+
+
+def test_split_rules_at_their_edges(tmp_path):
+    """tests/cpp/test_decode_rules.cpp: the rules the backends run (idle CUs, head_dim from 160 on)."""
+    repo = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = str(tmp_path / "decode_rules")
+    subprocess.run(["g++", "-std=c++20", "-O1", "-Wall", "-I" + os.path.join(repo, "include"),
+                    "-I" + os.path.join(repo, "scicompute-attention_amd", "src"),
+                    os.path.join(repo, "tests", "cpp", "test_decode_rules.cpp"), "-o", exe], check=True)
+    proc = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,most", [
+    (1, 32, 8, 3000, 128, 24), (4, 16, 4, 2000, 128, 16),  # fp32 takes more splits than 16 bits
+    (4, 32, 8, 8192, 160, 16), (16, 32, 8, 4096, 128, 8), (64, 32, 8, 4096, 128, 1)])
+def test_reported_scratch_covers_every_type(B, Hq, Hkv, S, D, most):
+    """The dispatcher's estimate knows no type: it is that of the type with the most splits."""
+    got = H.select(H.AttentionConfig(backend="decode", allow_fallback=False),
+                   H.AttentionShape(B, 1, S, Hq, Hkv, D))
+    assert got["workspace"] == (0 if most == 1 else B * Hq * most * (D + 2) * 4)

@@ -445,3 +445,33 @@ def test_key_split_scratch_under_the_per_thread_handle(hip):
     for i in range(4):
         for o in outs[i]:
             assert np.array_equal(o.numpy(), want[i]), i
+
+
+@pytest.mark.parametrize("shape", [(1, 32, 8, 3000, 128), (4, 16, 4, 2000, 128), (4, 32, 8, 8192, 160),
+                                   (16, 8, 8, 600, 96)])
+def test_decode_scratch_is_within_the_reported(hip, shape):
+    """stats.workspace_bytes of each type is at most the dispatcher's estimate, and reaches it for one."""
+    B, Hq, Hkv, S, D = shape
+    cfg = H.AttentionConfig(backend="decode")
+    reported = H.select(cfg, H.AttentionShape(B, 1, S, Hq, Hkv, D))["workspace"]
+    used = []
+    for dtype in ("f32", "f16", "bf16"):
+        bits = np.uint32 if dtype == "f32" else np.uint16
+        q, k, v = (tensor(np.zeros(n, bits), dtype) for n in
+                   ((B, Hq, 1, D), (B, Hkv, S, D), (B, Hkv, S, D)))
+        used.append(H.decode_attention(q, k, v, cfg).stats["workspace_bytes"])
+    print(shape, reported, used)
+    assert max(used) == reported
+
+
+@pytest.mark.parametrize("Sq,Skv,splits", [(6, 4102, True), (300, 300, False)])
+def test_flash_scratch_is_reported(hip, Sq, Skv, splits):
+    """A prefill that splits its keys reports the bytes of its partial states, before and after; others 0."""
+    B, Hq, Hkv, D = 1, 8, 2, 128
+    cfg = H.AttentionConfig(causal=True)
+    q, k, v = (tensor(np.zeros(n, np.uint16), "f16") for n in
+               ((B, Hq, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)))
+    used = H.attention(q, k, v, cfg).stats["workspace_bytes"]
+    got = H.select(cfg, H.AttentionShape(B, Sq, Skv, Hq, Hkv, D))
+    assert got["workspace"] == used and (used > 0) == splits and used % (B * Hq * Sq * (D + 2) * 4) == 0
+    assert f"workspace={used} B" in got["reason"]
