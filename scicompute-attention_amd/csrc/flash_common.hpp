@@ -256,7 +256,7 @@ constexpr int kSchedDsRead = 0x100;
 
 
 // ============================================================================================
-// The DMA pipeline of the head_dim 64 / 128 kernels (pair and wide).
+// The DMA pipeline of the pair, wide and split-dims kernels.
 //
 // K and V tiles go straight from global memory to LDS with buffer loads to LDS (16 bytes per
 // lane, no VGPR staging, no transposition) through a buffer resource bounded at the sequence's

@@ -79,8 +79,9 @@ int64_t SplitBytes(const sca_flash_params& p, int splits) {
 //
 // Splitting the keys (allow_split: the caller has scratch for the partial states) pays where the row
 // tiles do not fill the CUs and the keys are many. The estimate below, in microseconds, weighs it
-// against the unsplit kernel: a wide or split-dims workgroup (one per CU) takes about 0.1 + 0.0068 D
-// per 64 keys and 4 + 0.022 D beside them, a pair workgroup 1.19 times the step per 64 keys of two
+// against the unsplit kernel: a wide or split-dims workgroup takes about 0.1 + 0.0068 D per 64 keys and
+// 4 + 0.022 D beside them (modelled one to a CU; at D 32 and 64 two or three share one, so there the
+// rounds are overstated and no split goes past one workgroup per CU), a pair workgroup 1.19 times the step per 64 keys of two
 // groups and 5 beside them (both fitted to measurements at D = 32 .. 256), and the merge's launch 8 plus
 // its partials' write and read at 4.5 TB/s (with 5 for the launch 24 x 256 over 1,354 keys split, 28.1 us
 // against 26.5 for the pairs).

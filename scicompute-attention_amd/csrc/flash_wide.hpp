@@ -22,7 +22,7 @@
 // D = 96 causal 175 -> 122 us (847), non-causal 315 -> 221 us (932); D = 32 causal 78 -> 57 us,
 // non-causal 141 -> 102 us (672: the softmax VALU bounds it, at 4 MFMAs per 48 VALU operations).
 //
-// With one workgroup per CU its fixed part is not hidden: 8,192 workgroups of one key tile (D = 128)
+// With one workgroup per CU (from D = 96 on) its fixed part is not hidden: 8,192 workgroups of one key tile (D = 128)
 // took 322 us, 9.2 us each beside the step; with the K/V DMAs ahead of the wait for Q, 32-bit index
 // arithmetic, no rescale of the zero O and both key halves sharing the merge and the stores 246 us.
 // ============================================================================================
