@@ -62,6 +62,7 @@ struct FlashPlan {
 };
 
 constexpr int64_t kMaxSplitBytes = int64_t{64} << 20;
+constexpr int64_t kMinSplitKeys = 4 * 64;  // of each key range
 
 int64_t SplitBytes(const sca_flash_params& p, int splits) {
     return splits <= 1 ? 0 : p.batch * p.num_heads * p.seq_q * splits * (p.head_dim + 2) * 4;
@@ -124,7 +125,7 @@ FlashPlan PlanFlash(const sca_flash_params& p, bool allow_split) {
         best = wide_us(units_pack, 1);
     }
     best *= 0.93;  // a split has to promise more than the estimate's error
-    for (int64_t splits = 2; splits <= 16 && splits * 4 * 64 <= p.seq_kv; ++splits) {
+    for (int64_t splits = 2; splits <= 16 && splits * kMinSplitKeys <= p.seq_kv; ++splits) {
         const int64_t bytes = SplitBytes(p, static_cast<int>(splits));
         if (bytes > kMaxSplitBytes) break;
         const double us = wide_us(units_pack, splits) + 8.0 + 2.0 * static_cast<double>(bytes) / 4.5e6;
@@ -410,6 +411,8 @@ int ValidateFlash(const sca_flash_params* p) {
 extern "C" {
 
 int64_t sca_hip_flash_split_bytes(const sca_flash_params* p) {
+    // Short calls, which the host's own work bounds, are answered first.
+    if (p != nullptr && p->seq_kv < 2 * sca_hip::kMinSplitKeys) return 0;
     if (sca_hip::ValidateFlash(p) != 0 || !sca_hip::DmaReach(*p)) return 0;
     return sca_hip::SplitBytes(*p, sca_hip::PlanFlash(*p, true).splits);
 }
