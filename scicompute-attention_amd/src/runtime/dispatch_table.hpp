@@ -95,9 +95,14 @@ inline int64_t DecodeSplits(int64_t batch, int64_t num_heads, int64_t num_kv_hea
 // and 500 such keys take it 8 us and more (fp32 D 128, 1 x 3000 30.3 -> 14.8 us, 4 x 16/4 x 2000 29.6 ->
 // 14.8; bf16 D 256, 2 x 1000 34 -> 13). Up to head_dim 128 in 16 bits the two launches bound the call
 // and the longer merge costs 3% (4 x 700, D 128: 12.4 -> 12.8), so the count stays.
-inline int64_t FillSplits(int64_t splits, int64_t jobs, int64_t longest, int64_t cu_count) {
+// An unsplit call stays unsplit while a slot's K and V (`key_bytes` per key) are below 256 KiB: it saves
+// the merge's launch (unsplit / split, us: fp32 D 128, 2 sequences of 130 keys 9.7 / 12.3, of 256 13.7 /
+// 12.5; fp32 D 64 x 511 9.6 / 12.6; bf16 D 256 x 256 12.7 / 12.8, x 300 15.2 / 13.0; paged bf16 D 128,
+// 3 x 130 13.9 / 15.7, x 511 15.3 / 17.6, D 192 x 300 17.3 / 17.2, x 400 19.9 / 17.3).
+inline int64_t FillSplits(int64_t splits, int64_t jobs, int64_t longest, int64_t cu_count,
+                          int64_t key_bytes) {
     const int64_t cus = cu_count > 0 ? cu_count : 256;
-    if (2 * splits * jobs > cus) return splits;
+    if (2 * splits * jobs > cus || (splits == 1 && longest * key_bytes < (256 << 10))) return splits;
     int64_t fill = cus / jobs;
     const int64_t by_length = (longest + 127) / 128;
     fill = fill < by_length ? fill : by_length;
@@ -112,7 +117,7 @@ inline int64_t ContiguousDecodeSplits(int64_t batch, int64_t num_heads, int64_t 
         DecodeSplits(batch, num_heads, num_kv_heads, seq_kv, cu_count, 4, head_dim, half);
     if (batch < 1 || num_kv_heads < 1 || (half && head_dim < 160)) return splits;
     const int64_t slots = num_kv_heads * ((num_heads / num_kv_heads + 15) / 16);
-    return FillSplits(splits, batch * slots, seq_kv, cu_count);
+    return FillSplits(splits, batch * slots, seq_kv, cu_count, 2 * head_dim * (half ? 2 : 4));
 }
 
 // Work split of the paged MFMA decode kernel for a batch whose host-side lengths are known.
@@ -195,11 +200,11 @@ inline PagedDecodePlanResult PagedDecodePlanFor(int64_t head_dim, const int64_t*
         int64_t splits = jobs >= 2 * cus ? 1 : 2 * jobs >= cus ? 2 * cus / jobs : cus / jobs;
         splits = splits < by_length ? splits : by_length;
         splits = splits < th.max_splits ? splits : th.max_splits;
-        return {FillSplits(splits < 1 ? 1 : splits, jobs, longest, cus), 4};
+        return {FillSplits(splits < 1 ? 1 : splits, jobs, longest, cus, 4 * head_dim), 4};
     }
     if (plan.slot_waves == 1 && 2 * plan.splits * batch * ((slots + 3) / 4) <= cus) {
         plan.slot_waves = 4;
-        plan.splits = FillSplits(plan.splits, jobs, longest, cus);
+        plan.splits = FillSplits(plan.splits, jobs, longest, cus, 4 * head_dim);
     }
     return plan;
 }

@@ -30,14 +30,16 @@ void CheckPlan(const char* what, int64_t head_dim, const std::vector<int64_t>& l
 int main() {
     // Splits for idle CUs: not when half of them have a workgroup, at most 128 keys each and the table's
     // cap, never fewer than before, and the default CU count when it is unknown.
-    Check("half busy", FillSplits(8, 17, 100000, 256), 8);
-    Check("half idle", FillSplits(8, 16, 100000, 256), 16);
-    Check("short keys", FillSplits(1, 1, 129, 256), 2);
-    Check("one split of keys", FillSplits(1, 1, 128, 256), 1);
-    Check("no keys", FillSplits(1, 1, 0, 256), 1);
-    Check("the table's cap", FillSplits(1, 1, 1 << 20, 256), 64);
-    Check("never fewer", FillSplits(3, 4, 130, 256), 3);
-    Check("unknown CU count", FillSplits(1, 8, 1 << 20, 0), 32);
+    Check("half busy", FillSplits(8, 17, 100000, 256, 1024), 8);
+    Check("half idle", FillSplits(8, 16, 100000, 256, 1024), 16);
+    Check("short keys", FillSplits(2, 1, 257, 256, 1024), 3);
+    Check("the table's cap", FillSplits(1, 1, 1 << 20, 256, 512), 64);
+    Check("never fewer", FillSplits(3, 4, 130, 256, 1024), 3);
+    Check("unknown CU count", FillSplits(1, 8, 1 << 20, 0, 512), 32);
+    // Unsplit calls stay unsplit below 256 KiB of K and V a slot.
+    Check("below 256 KiB", FillSplits(1, 16, 255, 256, 1024), 1);
+    Check("from 256 KiB", FillSplits(1, 16, 256, 256, 1024), 2);
+    Check("no keys", FillSplits(1, 1, 0, 256, 1024), 1);
 
     // Contiguous KV: the fill is for fp32 and for head_dim >= 160.
     Check("fp32 1 x 3000", ContiguousDecodeSplits(1, 32, 8, 3000, 256, 128, false), 24);
@@ -50,6 +52,10 @@ int main() {
     Check("D 160, fp32: four", ContiguousDecodeSplits(4, 32, 8, 8192, 256, 160, false), 16);
     Check("D 192, a group of two: four", ContiguousDecodeSplits(4, 16, 8, 8192, 256, 192, true), 16);
     Check("D 256, a slot per CU", ContiguousDecodeSplits(32, 32, 8, 4096, 256, 256, true), 1);
+    Check("fp32 2 x 255", ContiguousDecodeSplits(2, 32, 8, 255, 256, 128, false), 1);
+    Check("fp32 2 x 256", ContiguousDecodeSplits(2, 32, 8, 256, 256, 128, false), 2);
+    Check("fp32 1 x 511, D 64", ContiguousDecodeSplits(1, 8, 8, 511, 256, 64, false), 1);
+    Check("16 bits 2 x 300, D 256", ContiguousDecodeSplits(2, 32, 8, 300, 256, 256, true), 3);
     Check("no keys at all", ContiguousDecodeSplits(1, 32, 8, 0, 256, 256, true), 1);
     Check("no batch", ContiguousDecodeSplits(0, 32, 8, 100, 256, 256, true), 1);
 
@@ -62,7 +68,9 @@ int main() {
     CheckPlan("D 160, two slots per CU", 160, std::vector<int64_t>(64, 4000), 32, 8, 1, 4);
     CheckPlan("D 256, half a slot per CU", 256, std::vector<int64_t>(16, 16384), 32, 8, 4, 4);
     CheckPlan("D 256, below", 256, std::vector<int64_t>(4, 9000), 64, 16, 4, 4);
-    CheckPlan("D 192, a few short ones", 192, {300, 5}, 32, 8, 3, 4);
+    CheckPlan("3 x 511", 128, std::vector<int64_t>(3, 511), 16, 16, 1, 4);
+    CheckPlan("D 192, 300 keys", 192, {300, 5}, 32, 8, 1, 4);
+    CheckPlan("D 192, 400 keys", 192, {400, 5}, 32, 8, 4, 4);
     if (failures == 0) std::printf("decode rules: ok\n");
     return failures == 0 ? 0 : 1;
 }
