@@ -126,7 +126,7 @@ SCA_CAPI int64_t sca_decode_splits(const ScaShape* shape, int64_t cu_count);
  * writes the split count and the sca_decode_params.slot_waves value (1 or 4; 0 with splits 1
  * when every length is 0) the paged backend uses when the cache's own page table is attended, made
  * for head_dim up to 128 and batches that fill the GPU: where one wave per slot would leave half the
- * CUs idle the backend takes four (and shorter splits), and from head_dim 160 on always four.
+ * CUs idle the backend takes four (and shorter splits), and from head_dim 160 on it has rules of its own.
  * Returns 0, or SCA_E_SHAPE_MISMATCH. */
 SCA_CAPI int sca_paged_decode_plan(const int64_t* lengths, int64_t batch, int64_t num_heads,
                                    int64_t num_kv_heads, int64_t cu_count, int64_t* splits,

@@ -1047,11 +1047,13 @@ int LaunchForDim(const sca_decode_params& p, hipStream_t s) {
     // kernel: with so little reuse it is as fast, and for D >= 160 four of its workgroups share a CU
     // where the MFMA kernel's rings allow one (bf16: D 96, 16 x 32/32 x 2000 68.5 us against 69.5;
     // D 256, 16 x 16/16 x 4096 176 against 180, 4 x 16/8 x 8192 54 against 60 at the same 16 splits).
-    // Larger groups and paged KV gain from 1% to 5.6x (64 x 64/8 x 4096, D 192: 536 -> 271 us;
-    // 128 x 28/4 x 2000, D 32: 127 -> 23; 64 x 512..16384 paged, D 256: 1,377 -> 689).
-    // Paged D 256 with one head per KV head too (4 x 4000..9000, 16 heads: 76 us against 81 at its best).
-    const bool valu_group = kPaged ? D == 256 && group == 1
-                                   : D != 64 && D != 128 && (group == 1 || (group == 2 && D >= 160));
+    // Larger groups gain from 1% to 5.6x (64 x 64/8 x 4096, D 192: 536 -> 271 us; 128 x 28/4 x 2000, D 32:
+    // 127 -> 23; 64 x 512..16384 paged, D 256: 1,377 -> 689). Paged KV too (bf16, VALU / MFMA at its best, us:
+    // 16/16 heads, 153 x 108 keys D 96 24.1 / 31.9, D 160 34.3 / 57.3, 64 x 1000 D 96 71.9 / 72.9, D 192 141 /
+    // 135; 16/8, 153 x 108 D 160 24.9 / 38.2, D 256 27.9 / 51.2, 64 x 512..8192 D 160 280 / 248), except
+    // D 32 with one head per KV head, where neither is ahead (64 x 1000 31 / 30).
+    const bool valu_group = D != 64 && D != 128 &&
+                            ((group == 1 && !(kPaged && D == 32)) || (group == 2 && D >= 160));
     const bool mfma_ok = !std::is_same_v<E, DecF32> && !valu_group &&
                          (!kPaged || (int64_t{1} << block_shift) == p.block_size);
     if constexpr (!std::is_same_v<E, DecF32>) {

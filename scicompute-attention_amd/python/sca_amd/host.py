@@ -453,7 +453,7 @@ def decode_splits(shape: AttentionShape, cu_count: int) -> int:
 def paged_decode_plan(lengths, num_heads: int, num_kv_heads: int, cu_count: int):
     """(splits, slot_waves) of the paged MFMA decode kernel for a batch of host-side lengths:
     the plan the paged backend applies when it attends the cache's own page table, up to head_dim
-    128 and with enough sequences to fill the GPU (else it takes four waves per slot)."""
+    128 and with enough sequences to fill the GPU."""
     lens = np.ascontiguousarray(lengths, dtype=np.int64)
     splits, waves = c_i64(0), c_i32(0)
     _raise(host_lib().sca_paged_decode_plan(_ptr(lens) if lens.size else None, lens.size,

@@ -337,19 +337,22 @@ sci::Result<AttentionResult> RunPaged(const sci::Tensor& q, const PagedKVCache& 
     // params.seq_lens (device memory) do not feed the plan: the kernel reads them, so results
     // follow them exactly, while the plan is fitted to the cache's host lengths (which a decode
     // loop passing its own lengths, with this step's token, tracks to within a token).
-    // (One query head per KV head at head_dim 256 runs the VALU kernel, with its own split rule.)
-    const bool mfma_shape = kv_cfg.dtype != sci::DType::kFloat32 &&
-                            !(head_dim == 256 && num_heads == kv_cfg.num_kv_heads) &&
-                            (block_size & (block_size - 1)) == 0;
-    if (cfg.num_splits <= 0 && params.page_table == nullptr && mfma_shape) {
+    // (Small groups at some head dims run the VALU kernel, with a split rule of its own.)
+    const bool pow2_pages = kv_cfg.dtype != sci::DType::kFloat32 && (block_size & (block_size - 1)) == 0;
+    if (cfg.num_splits <= 0 && params.page_table == nullptr && pow2_pages) {
+        const int cus = DeviceCapability::ForDevice(0).sm_count;
         std::vector<int64_t> lengths(static_cast<size_t>(num_seqs));
         for (int64_t b = 0; b < num_seqs; ++b) lengths[static_cast<size_t>(b)] = kv.SeqLength(b);
-        const auto plan = detail::PagedDecodePlanFor(head_dim, lengths.data(), num_seqs, num_heads,
-                                                     kv_cfg.num_kv_heads,
-                                                     DeviceCapability::ForDevice(0).sm_count);
-        if (plan.slot_waves != 0) {
-            splits = plan.splits;
-            slot_waves = plan.slot_waves;
+        if (detail::PagedValuGroup(head_dim, num_heads / kv_cfg.num_kv_heads)) {
+            splits = detail::PagedValuSplits(head_dim, lengths.data(), num_seqs, num_heads,
+                                             kv_cfg.num_kv_heads, cus);
+        } else {
+            const auto plan = detail::PagedDecodePlanFor(head_dim, lengths.data(), num_seqs, num_heads,
+                                                         kv_cfg.num_kv_heads, cus);
+            if (plan.slot_waves != 0) {
+                splits = plan.splits;
+                slot_waves = plan.slot_waves;
+            }
         }
     }
 

@@ -120,6 +120,47 @@ inline int64_t ContiguousDecodeSplits(int64_t batch, int64_t num_heads, int64_t 
     return FillSplits(splits, batch * slots, seq_kv, cu_count, 2 * head_dim * (half ? 2 : 4));
 }
 
+struct LengthSummary {
+    int64_t longest;
+    bool uniform;  // longest <= 11/10 of the mean
+};
+inline LengthSummary SummarizeLengths(const int64_t* lengths, int64_t batch) {
+    int64_t longest = 0;
+    int64_t total = 0;
+    for (int64_t b = 0; b < batch; ++b) {
+        const int64_t len = lengths[b] > 0 ? lengths[b] : 0;
+        longest = len > longest ? len : longest;
+        total += len;
+    }
+    return {longest, 10 * longest * batch <= 11 * total};
+}
+
+// Paged 16-bit calls whose group is too small for the MFMA kernel (the launcher's rule) run the VALU
+// kernel, a workgroup per (sequence, KV head, split), four to a CU.
+inline bool PagedValuGroup(int64_t head_dim, int64_t group) {
+    return head_dim != 64 && head_dim != 128 &&
+           ((group == 1 && head_dim != 32) || (group == 2 && head_dim >= 160));
+}
+// Its splits for known lengths: unsplit from two workgroups per CU on (four, below head_dim 192 from 512
+// keys on), else until every CU holds four; and eight where the batch is ragged (the launch ends with its
+// longest sequences) or, with one head per KV head, below head_dim 192 from 512 keys on; 128 keys each at
+// least (bf16, unsplit / 8, us: 16/16 heads, D 96: 64 x 1000 85 / 72, 128 x
+// 128..4000 405 / 274; D 256: 64 x 1000 180 / 186, 128 x 128..4000 765 / 712; 16/8, D 160: 128 x 600 77 / 98,
+// 32 x 2000 119 / 64, 64 x 512..8192 524 / 280; unsplit / 2: D 96 40 x 300 20 / 22, D 192 16/8 64 x 1000 78 / 80,
+// D 160 75 / 68).
+inline int64_t PagedValuSplits(int64_t head_dim, const int64_t* lengths, int64_t batch, int64_t num_heads,
+                               int64_t num_kv_heads, int64_t cu_count) {
+    const LengthSummary len = SummarizeLengths(lengths, batch);
+    const int64_t cus = cu_count > 0 ? cu_count : 256;
+    const int64_t jobs = batch * num_kv_heads;
+    const bool split_pays = head_dim < 192 && len.longest >= 512;
+    int64_t splits = jobs >= (split_pays ? 4 : 2) * cus ? 1 : (4 * cus + jobs - 1) / jobs;
+    if ((!len.uniform || (split_pays && num_heads == num_kv_heads)) && splits < 8) splits = 8;
+    if (splits > len.longest / 128) splits = len.longest / 128;
+    if (splits > kDispatchThresholds.max_splits) splits = kDispatchThresholds.max_splits;
+    return splits < 1 ? 1 : splits;
+}
+
 // Work split of the paged MFMA decode kernel for a batch whose host-side lengths are known.
 // slot_waves = 1: one wave per head slot, a workgroup serves four slots; 4: four waves share one
 // slot's key tiles. Measured on MI355X over 48-step decode loops (bf16, H_q 32, H_kv 8, D 128):
@@ -143,19 +184,14 @@ inline PagedDecodePlanResult PagedDecodePlan(const int64_t* lengths, int64_t bat
     if (lengths == nullptr || batch < 1 || num_kv_heads < 1 || num_heads < num_kv_heads) {
         return {1, 0};
     }
-    int64_t longest = 0;
-    int64_t total = 0;
-    for (int64_t b = 0; b < batch; ++b) {
-        const int64_t len = lengths[b] > 0 ? lengths[b] : 0;
-        longest = len > longest ? len : longest;
-        total += len;
-    }
+    const LengthSummary len = SummarizeLengths(lengths, batch);
+    const int64_t longest = len.longest;
     if (longest < 1) return {1, 0};
     const int64_t group = num_heads / num_kv_heads;
     const int64_t slots = num_kv_heads * ((group + 15) / 16);
     const int64_t quads = (slots + 3) / 4;
     const int64_t cus = cu_count > 0 ? cu_count : 256;
-    const bool uniform = 10 * longest * batch <= 11 * total;
+    const bool uniform = len.uniform;
     int64_t splits;
     int32_t slot_waves;
     if (uniform && batch * quads <= cus) {
@@ -179,11 +215,13 @@ inline PagedDecodePlanResult PagedDecodePlan(const int64_t* lengths, int64_t bat
 //    their minimum length) becomes four waves per slot at the same splits: four times the
 //    workgroups, each with a quarter of the tiles per wave, and shorter splits where that still
 //    leaves CUs idle (FillSplits);
-//  - head_dim >= 160, where the kernel's rings leave room for one workgroup per CU: four waves per
-//    slot, unsplit from two slots per CU on, two workgroups per CU down to half a slot per CU and one
-//    below (bf16, H_kv 8: D 256, 16 x 512..16384 4 splits 5.52 TB/s against 5.00 at 12; D 160, 128 x
-//    128..4000 1 split 5.01 against 2.95 at 6; D 256, 4 x 4000..9000 x 16 heads 4 splits 4.73 against
-//    3.95 at 12).
+//  - head_dim >= 160, where the kernel's rings leave room for one workgroup per CU. Near-uniform or short
+//    (up to 512 keys) batches that reach a quarter of the CUs with one wave per slot: that, split until
+//    every CU has a workgroup, 128 keys each at least (us, one wave / four: bf16 32/8, D 160: 153 x 108
+//    keys 38 / 62, 40 x 300 23 / 31, 128 x 600 73 / 107, 64 x 1000 62 / 72, 150 x 16..200 30 / 64). Others
+//    four waves per slot, unsplit from two slots per CU on, two workgroups per CU down to half a slot per
+//    CU and one below (bf16, H_kv 8: D 256, 16 x 512..16384 4 splits 5.52 TB/s against 5.00 at 12; D 256,
+//    4 x 4000..9000 x 16 heads 4 splits 4.73 against 3.95 at 12).
 inline PagedDecodePlanResult PagedDecodePlanFor(int64_t head_dim, const int64_t* lengths,
                                                 int64_t batch, int64_t num_heads,
                                                 int64_t num_kv_heads, int64_t cu_count) {
@@ -192,10 +230,16 @@ inline PagedDecodePlanResult PagedDecodePlanFor(int64_t head_dim, const int64_t*
     const int64_t slots = num_kv_heads * ((num_heads / num_kv_heads + 15) / 16);
     const int64_t jobs = batch * slots;
     const int64_t cus = cu_count > 0 ? cu_count : 256;
-    int64_t longest = 0;
-    for (int64_t b = 0; b < batch; ++b) longest = lengths[b] > longest ? lengths[b] : longest;
+    const LengthSummary len = SummarizeLengths(lengths, batch);
+    const int64_t longest = len.longest;
     if (head_dim >= 160) {
         const auto& th = kDispatchThresholds;
+        const int64_t wgs = batch * ((slots + 3) / 4);  // of one wave per slot
+        if ((len.uniform || longest <= 512) && 4 * wgs >= cus) {
+            int64_t splits = cus / wgs;
+            splits = splits < longest / 128 ? splits : longest / 128;
+            return {splits < 1 ? 1 : splits, 1};
+        }
         const int64_t by_length = (longest + th.min_tokens_per_split - 1) / th.min_tokens_per_split;
         int64_t splits = jobs >= 2 * cus ? 1 : 2 * jobs >= cus ? 2 * cus / jobs : cus / jobs;
         splits = splits < by_length ? splits : by_length;

@@ -65,12 +65,55 @@ int main() {
     CheckPlan("1 x 8000", 128, {8000}, 32, 8, 32, 4);
     CheckPlan("1 x 100", 96, {100}, 32, 8, 1, 4);
     CheckPlan("64 x 8448 keeps its plan", 128, std::vector<int64_t>(64, 8448), 32, 8, 2, 1);
-    CheckPlan("D 160, two slots per CU", 160, std::vector<int64_t>(64, 4000), 32, 8, 1, 4);
+    CheckPlan("D 160, 64 x 4000", 160, std::vector<int64_t>(64, 4000), 32, 8, 2, 1);
     CheckPlan("D 256, half a slot per CU", 256, std::vector<int64_t>(16, 16384), 32, 8, 4, 4);
+    CheckPlan("D 160, two slots per CU, ragged", 160, [] {
+        std::vector<int64_t> v(64, 1000);
+        v[5] = 4000;
+        return v;
+    }(), 32, 8, 1, 4);
     CheckPlan("D 256, below", 256, std::vector<int64_t>(4, 9000), 64, 16, 4, 4);
     CheckPlan("3 x 511", 128, std::vector<int64_t>(3, 511), 16, 16, 1, 4);
     CheckPlan("D 192, 300 keys", 192, {300, 5}, 32, 8, 1, 4);
     CheckPlan("D 192, 400 keys", 192, {400, 5}, 32, 8, 4, 4);
+    CheckPlan("D 160, 153 x 108: one wave", 160, std::vector<int64_t>(153, 108), 32, 8, 1, 1);
+    CheckPlan("D 160, 40 x 300", 160, std::vector<int64_t>(40, 300), 32, 8, 2, 1);
+    CheckPlan("D 192, 150 short ragged", 192, [] {
+        std::vector<int64_t> v(150, 60);
+        v[3] = 512;
+        return v;
+    }(), 32, 8, 1, 1);
+    CheckPlan("D 192, one past", 192, [] {
+        std::vector<int64_t> v(150, 60);
+        v[3] = 513;
+        return v;
+    }(), 32, 8, 1, 4);
+    CheckPlan("D 160, 31 x 300: too few", 160, std::vector<int64_t>(31, 300), 32, 8, 1, 4);
+
+    // Small groups over paged KV: the VALU kernel's own splits.
+    const auto valu = [](int64_t d, int64_t n, int64_t len, int64_t heads, int64_t kv, int64_t first) {
+        std::vector<int64_t> v(static_cast<size_t>(n), len);
+        v[0] = first;
+        return PagedValuSplits(d, v.data(), n, heads, kv, 256);
+    };
+    Check("group 1, D 96", PagedValuGroup(96, 1), 1);
+    Check("group 1, D 32", PagedValuGroup(32, 1), 0);
+    Check("group 1, D 128", PagedValuGroup(128, 1), 0);
+    Check("group 2, D 96", PagedValuGroup(96, 2), 0);
+    Check("group 2, D 160", PagedValuGroup(160, 2), 1);
+    Check("group 3, D 256", PagedValuGroup(256, 3), 0);
+    Check("153 x 108", valu(96, 153, 108, 16, 16, 108), 1);
+    Check("64 x 1000, D 96", valu(96, 64, 1000, 16, 16, 1000), 7);
+    Check("64 x 1000, D 192", valu(192, 64, 1000, 16, 16, 1000), 1);
+    Check("64 x 511", valu(96, 64, 511, 16, 16, 511), 1);
+    Check("40 x 300", valu(96, 40, 300, 16, 16, 300), 1);
+    Check("two heads, 64 x 1000, D 160", valu(160, 64, 1000, 16, 8, 1000), 2);
+    Check("two heads, 64 x 1000, D 192", valu(192, 64, 1000, 16, 8, 1000), 1);
+    Check("two heads, 63 x 1000, D 192", valu(192, 63, 1000, 16, 8, 1000), 3);
+    Check("ragged", valu(256, 64, 500, 16, 16, 4000), 8);
+    Check("four workgroups per CU", valu(160, 32, 2000, 16, 8, 2000), 4);
+    Check("one short sequence", valu(256, 1, 100, 8, 8, 100), 1);
+    Check("no keys", valu(256, 4, 0, 8, 8, 0), 1);
     if (failures == 0) std::printf("decode rules: ok\n");
     return failures == 0 ? 0 : 1;
 }

@@ -287,3 +287,13 @@ def test_other_head_dims_keep_fp32_weights(hip, D, dtype):
         limit = 1.01 * u * np.abs(ref) + (4 * u * u + 4e-6) * float(np.max(np.abs(vd)))
         worst = float(np.max(np.abs(got - ref) / limit))
         assert worst <= 1.0, f"{worst:.2f} times the bound"
+
+
+@pytest.mark.parametrize("D", [96, 160, 192, 256])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_small_groups_at_other_head_dims(hip, D, dtype):
+    """One and two query heads per KV head, either side of the rule that picks the kernel: short, ragged
+    and page-crossing lengths, unsplit and split."""
+    for Hq, Hkv in ((3, 3), (6, 3), (9, 3)):
+        for splits, bs in ((1, 16), (3, 32)):
+            _case([1, 31, 33, 300], bs, Hq, Hkv, D, dtype, 88000 + D + Hq, splits=splits)
